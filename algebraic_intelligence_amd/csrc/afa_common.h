@@ -83,6 +83,78 @@ struct Elem<AFA_F32> {
   static __device__ __forceinline__ void store(void* p, int64_t i, float x) { ((float*)p)[i] = x; }
 };
 
+// ------------------------------------------------------------------ rows in 16-byte chunks
+// A row of n elements at any element-aligned address, seen as the 16-byte aligned chunks that
+// cover it: chunk c holds elements c * EPC - lead .. + EPC - 1, lead the elements between the
+// aligned address at or below the row's start and the start.  Whole chunks move as one 16-byte
+// access; the first and the last chunk of a row that starts or ends inside one move element by
+// element, so nothing outside the row is read or written (entries outside it load as zeros).
+template <int DT>
+struct RowChunk {
+  static constexpr int ESZ = DT == AFA_F32 ? 4 : 2;
+  static constexpr int EPC = 16 / ESZ;
+  static __device__ __forceinline__ int lead(const void* row) { return (int)((uintptr_t)row & 15u) / ESZ; }
+  static __host__ __device__ __forceinline__ int count(int n, int lead) {
+    return (int)(((int64_t)n + lead + EPC - 1) / EPC);
+  }
+  // chunks of the worst start
+  static __host__ __device__ __forceinline__ int count_max(int n) { return count(n, EPC - 1); }
+  static __device__ __forceinline__ u32x4_t load(const void* row, int e0, int n) {
+    if (e0 >= 0 && n - e0 >= EPC) return *(const u32x4_t*)((const char*)row + (int64_t)e0 * ESZ);
+    u32x4_t w = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < EPC; ++i) {
+      if (e0 + i >= 0 && (int64_t)e0 + i < n) {
+        if constexpr (DT == AFA_F32) {
+          w[i] = ((const unsigned*)row)[e0 + i];
+        } else {
+          const unsigned u = ((const unsigned short*)row)[e0 + i];
+          w[i >> 1] |= u << (16 * (i & 1));
+        }
+      }
+    }
+    return w;
+  }
+  static __device__ __forceinline__ void unpack(u32x4_t w, float (&v)[EPC]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned u = w[i];  // a bit_cast of a subscripted vector element reads element 0
+      if constexpr (DT == AFA_F32) {
+        v[i] = __builtin_bit_cast(float, u);
+      } else {
+        v[2 * i] = Elem<DT>::lo(u);
+        v[2 * i + 1] = Elem<DT>::hi(u);
+      }
+    }
+  }
+  static __device__ __forceinline__ u32x4_t pack(const float (&v)[EPC]) {
+    u32x4_t w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (DT == AFA_F32) {
+        const float f = v[i];
+        w[i] = __builtin_bit_cast(unsigned, f);
+      } else {
+        w[i] = Elem<DT>::pack(v[2 * i], v[2 * i + 1]);
+      }
+    }
+    return w;
+  }
+  static __device__ __forceinline__ void store(void* row, int e0, int n, u32x4_t w) {
+    if (e0 >= 0 && n - e0 >= EPC) {
+      *(u32x4_t*)((char*)row + (int64_t)e0 * ESZ) = w;
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < EPC; ++i) {
+      if (e0 + i >= 0 && (int64_t)e0 + i < n) {
+        if constexpr (DT == AFA_F32) ((unsigned*)row)[e0 + i] = w[i];
+        else ((unsigned short*)row)[e0 + i] = (unsigned short)(w[i >> 1] >> (16 * (i & 1)));
+      }
+    }
+  }
+};
+
 // ------------------------------------------------------------------ key-shard sums
 // One element of a key shard's unnormalised sums: stored (mode 1, ACC_STORE) or added (mode 2,
 // ACC_ADD) to what the caller's array holds.

@@ -202,7 +202,7 @@ size_t oace_generic_chunk_rows(int dtype, int64_t N, int64_t V);
 size_t oace_generic_workspace(int dtype, int64_t N, int64_t d, int64_t V, bool backward);
 hipError_t oace_linear_fwd_generic(int dtype, const OaceArgs& a, void* rows, void* ws, hipStream_t st);
 hipError_t oace_linear_bwd_generic(int dtype, const OaceArgs& a, const void* rows, void* ws, hipStream_t st);
-hipError_t oace_mean_launch(int dtype, const void* rows, int64_t N, void* loss, hipStream_t st);
+hipError_t oace_mean_launch(int dtype, void* rows, int64_t N, void* loss, hipStream_t st);
 hipError_t oace_softmax_fwd_launch(int dtype, const OaceArgs& a, void* rows, hipStream_t st);
 hipError_t oace_softmax_bwd_launch(int dtype, const OaceArgs& a, const void* rows, void* dz, hipStream_t st);
 hipError_t oace_transpose16(const void* x, int64_t rows, int64_t cols, int64_t ldx, void* y, int64_t ldy,

@@ -99,14 +99,201 @@ __global__ __launch_bounds__(256) void oace_rows_fwd_kernel(const ZT* z, int64_t
   }
 }
 
-// loss = mean of the per-row losses, in a fixed order (one workgroup).
+// loss = mean of the per-row losses, in a fixed order.  One workgroup for up to MEAN_ROWS rows; more
+// rows are first summed MEAN_ROWS at a time into the last (unused) field of each group's first
+// record (one workgroup reads its records at the rate of one compute unit: the forward
+// call on (134000, 1000) bf16 took 257 us with one, 114 us with groups).
+constexpr int MEAN_ROWS = 4096;
 template <typename A>
-__global__ __launch_bounds__(256) void oace_mean_kernel(const A* rows, int64_t N, A* loss) {
+__global__ __launch_bounds__(256) void oace_mean_kernel(A* rows, int64_t N, int64_t stride, int field, A scale,
+                                                        A* loss) {
   __shared__ A sh[4];
   A s[1] = {A(0)};
-  for (int64_t i = threadIdx.x; i < N; i += 256) s[0] += rows[i * OACE_ROW + OACE_LOSS];
+  const int64_t i0 = (int64_t)blockIdx.x * MEAN_ROWS, i1 = loss == nullptr && i0 + MEAN_ROWS < N ? i0 + MEAN_ROWS : N;
+#pragma unroll 4
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) s[0] += rows[i * stride + field];
   block_sum<A, 1>(s, sh);
-  if (threadIdx.x == 0) *loss = s[0] / (A)N;
+  if (threadIdx.x == 0) {
+    if (loss != nullptr) *loss = s[0] / scale;
+    else rows[i0 * OACE_ROW + OACE_ROW - 1] = s[0];
+  }
+}
+
+// The row records of 16- and 32-bit logits: T threads per row, the row read once into registers as
+// 16-byte chunks (NCH per thread; NCH = 0 streams a longer row twice).  Bound by the octic terms' VALU issue (about
+// 20 instructions and two quarter-rate ones per 16-bit entry) just above its one HBM read:
+// (2048, 50257) bf16, forward call with the mean 176 -> 76 us (2.7 TB/s; the two passes of 2-byte
+// loads by one 256-thread workgroup per row took 171 of the 176), fp32 97 us (4.3 TB/s).
+template <int DT, int T, int NCH>
+__global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel(const void* z, int64_t ldz, int64_t N,
+                                                                             int V, const int64_t* targets, float eps,
+                                                                             float gamma, float inv_v, float* rows) {
+  using R = RowChunk<DT>;
+  constexpr int RPB = T < 256 ? 256 / T : 1;  // rows per workgroup
+  constexpr int NW = T / 64;                  // waves per row
+  __shared__ float sh[NW > 1 ? 5 * NW : 1];
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / T;
+  if (row >= N) return;  // whole waves, and only where no barrier follows (one wave per row)
+  const int tid = threadIdx.x % T, lane = threadIdx.x & 63, wave = tid >> 6;
+  const char* zr = (const char*)z + row * ldz * R::ESZ;
+  const int lead = R::lead(zr), nch = R::count(V, lead);
+  constexpr int NR = NCH > 0 ? NCH : 1;
+  u32x4_t raw[NR];
+  float ss = 0.f;
+  auto sq = [&](u32x4_t w) {
+    float v[R::EPC];
+    R::unpack(w, v);
+#pragma unroll
+    for (int i = 0; i < R::EPC; ++i) ss = __builtin_fmaf(v[i], v[i], ss);
+  };
+  if constexpr (NCH > 0) {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const int c = tid + T * j;
+      raw[j] = u32x4_t{0u, 0u, 0u, 0u};
+      if (c < nch) raw[j] = R::load(zr, c * R::EPC - lead, V);
+    }
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      sq(raw[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    for (int c = tid; c < nch; c += T) sq(R::load(zr, c * R::EPC - lead, V));
+  }
+  ss = wave_sum(ss);
+  if constexpr (NW > 1) {
+    if (lane == 0) sh[4 * NW + wave] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) ss += sh[4 * NW + w];
+  }
+  const float tau = o_rsq<float>(ss * inv_v + eps);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  // entries of a covering chunk outside the row are zeros, whose terms are exact (rho = 1): they
+  // add 1 each to the first two sums, taken off again below
+  auto eval = [&](u32x4_t w) {
+    float v[R::EPC];
+    R::unpack(w, v);
+#pragma unroll
+    for (int i = 0; i < R::EPC; ++i) {
+      const float x = v[i] * tau;
+      float rho, rho7, r;
+      octic7(x, rho, rho7, r);
+      s[0] = __builtin_fmaf(rho7, rho, s[0]);
+      s[1] += rho7;
+      const float m = (r * x) * rho7;
+      s[2] = __builtin_fmaf(m, rho, s[2]);
+      s[3] += m;
+    }
+  };
+  if constexpr (NCH > 0) {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      asm("" : "+v"(raw[j]));  // unpack again here: the first pass's floats would take twice the registers
+      if (tid + T * j < nch) eval(raw[j]);
+      __builtin_amdgcn_sched_barrier(0);  // one chunk's terms live at a time
+    }
+  } else {
+    for (int c = tid; c < nch; c += T) eval(R::load(zr, c * R::EPC - lead, V));
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) s[q] = wave_sum(s[q]);
+  if constexpr (NW > 1) {
+    if (lane == 0)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sh[q * NW + wave] = s[q];
+    __syncthreads();
+    if (tid != 0) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      s[q] = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s[q] += sh[q * NW + w];
+    }
+  }
+  if (tid == 0) {
+    const float pad = (float)(nch * R::EPC - V);
+    const int64_t t = targets[row];
+    float rho_t = 0.f, rn_t = 0.f;  // a target outside [0, V) leaves rho_t = 0 (loss = inf), as the reference
+    if (t >= 0 && t < V) {
+      const float x = Elem<DT>::load(zr, t) * tau;
+      const Oct<float> o = octic(x);
+      rho_t = o.rho;
+      rn_t = o.r * x;
+    }
+    oace_finalize_row<float>(rows + row * OACE_ROW, tau, s[0] - pad, s[1] - pad, s[2], s[3], rho_t, rn_t, inv_v,
+                             gamma);
+  }
+}
+
+// dz of 16- and 32-bit logits: one wave per U * 64 chunks of a row, U 16-byte loads in flight per
+// lane.  The terms of every entry are formed without the target (the tau, c and sum factors folded
+// into three row scalars); the one chunk that holds it is formed again with it.  HBM
+// bound: (2048, 50257) bf16 157 -> 84 us for the call (4.9 TB/s read and written; the device copies
+// at the same rate), against 2-byte loads and stores before.
+template <int DT, int U>
+__global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, int64_t ldz, int64_t N, int V,
+                                                                const int64_t* targets, const float* rows,
+                                                                const float* g_loss, float c0, void* dz,
+                                                                int64_t lddz) {
+  using R = RowChunk<DT>;
+  const int lane = threadIdx.x & 63;
+  const int spans = (R::count_max(V) + 64 * U - 1) / (64 * U);
+  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = w / spans;
+  if (row >= N) return;
+  const char* zr = (const char*)z + row * ldz * R::ESZ;
+  char* dr = (char*)dz + row * lddz * R::ESZ;
+  const int lead = R::lead(zr), nch = R::count(V, lead);
+  const int cb = (int)(w % spans) * (64 * U) + lane;
+  u32x4_t raw[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = cb + 64 * u;
+    raw[u] = u32x4_t{0u, 0u, 0u, 0u};
+    if (c < nch) raw[u] = R::load(zr, c * R::EPC - lead, V);
+  }
+  const float* rec = rows + row * OACE_ROW;
+  const float tau = rec[OACE_TAU], inv_S = rec[OACE_INV_S], pc = rec[OACE_PC_INV8];
+  const float tc = tau * (c0 * (g_loss ? *g_loss : 1.f));
+  const float scale = rec[OACE_S8] * inv_S;
+  const float cs = tc * scale, cd = tc * (inv_S * (rec[OACE_SUM_P78] - pc)), cr = tc * rec[OACE_RADIAL];
+  const int64_t t = targets[row];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = cb + 64 * u;
+    if (c < nch) {
+      const int e0 = c * R::EPC - lead;
+      float v[R::EPC], o[R::EPC];
+      R::unpack(raw[u], v);
+      // the entry of this chunk that is the target (outside [0, EPC): none)
+      const int64_t et = t >= 0 && t < V ? t - e0 : -1;
+      const bool hit = et >= 0 && et < R::EPC;
+#pragma unroll
+      for (int i = 0; i < R::EPC; ++i) {
+        const float x = v[i] * tau;
+        float rho, rho7, r;
+        octic7(x, rho, rho7, r);
+        const float b = rho7 * __builtin_fmaf(-cd, rho, cs);
+        o[i] = __builtin_fmaf(r, b, -cr * x);
+      }
+      if (hit) {
+#pragma unroll
+        for (int i = 0; i < R::EPC; ++i) {
+          if (i == (int)et) {
+            const float x = v[i] * tau;
+            float rho, rho7, r;
+            octic7(x, rho, rho7, r);
+            const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - tc * pc;
+            o[i] = __builtin_fmaf(r, b, -cr * x);
+          }
+        }
+      }
+      R::store(dr, e0, V, R::pack(o));
+    }
+  }
 }
 
 // dz = tau c (r bracket - radial x) for every element of rows (grid.y = row), c = c0 * g.
@@ -267,17 +454,63 @@ void w_strides(const OaceArgs& a, int64_t& sk, int64_t& sv) {
   }
 }
 
+// Threads per row and 16-byte chunks per thread by the row's length: the fewest threads that hold
+// the row in at most 4 chunks each, then 512 threads with up to 26 (104 registers of a 128-register
+// wave, so two workgroups still share a compute unit and one loads while the other evaluates);
+// longer rows are streamed.
+template <int DT>
+void rows_fwd_vec(const OaceArgs& a, const void* z, int64_t ldz, void* rows, hipStream_t st) {
+  const int nch = RowChunk<DT>::count_max((int)a.V);
+  const float inv_v = (float)(1.0 / (double)a.V);
+#define OACE_ROWS_VEC(T, NCH)                                                                                       \
+  hipLaunchKernelGGL((oace_rows_fwd_vec_kernel<DT, T, NCH>), dim3((unsigned)((a.N * T + (T < 256 ? 255 : T - 1)) /  \
+                     (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, z, ldz, a.N, (int)a.V, a.targets,       \
+                     (float)a.eps, (float)a.gamma, inv_v, (float*)rows)
+  if (nch <= 64) OACE_ROWS_VEC(64, 1);
+  else if (nch <= 128) OACE_ROWS_VEC(64, 2);
+  else if (nch <= 256) OACE_ROWS_VEC(64, 4);
+  else if (nch <= 512) OACE_ROWS_VEC(256, 2);
+  else if (nch <= 1024) OACE_ROWS_VEC(256, 4);
+  else if (nch <= 2048) OACE_ROWS_VEC(512, 4);
+  else if (nch <= 256 * 13) OACE_ROWS_VEC(256, 13);
+  else if (nch <= 512 * 13) OACE_ROWS_VEC(512, 13);
+  else if (nch <= 512 * 25) OACE_ROWS_VEC(512, 25);
+  else OACE_ROWS_VEC(512, 0);
+#undef OACE_ROWS_VEC
+}
+
+// z and dz rows must start at the same offset from a 16-byte boundary (the chunks of the one are
+// then the chunks of the other); false: the caller takes the element-wise kernel.
+template <int DT>
+bool rows_bwd_vec(const OaceArgs& a, const void* rows, void* dz, float c0, hipStream_t st) {
+  using R = RowChunk<DT>;
+  if ((((uintptr_t)a.h ^ (uintptr_t)dz) & 15u) != 0) return false;
+  const int nch = R::count_max((int)a.V);
+  // four chunks per lane when that still leaves four waves per SIMD, else one
+  const bool wide = a.N * ((nch + 255) / 256) >= 4096;
+  const int64_t waves = a.N * (int64_t)((nch + (wide ? 255 : 63)) / (wide ? 256 : 64));
+  const dim3 grid((unsigned)((waves + 3) / 4));
+  if (wide)
+    hipLaunchKernelGGL((oace_rows_bwd_vec_kernel<DT, 4>), grid, dim3(256), 0, st, a.h, a.ldh, a.N, (int)a.V, a.targets,
+                       (const float*)rows, (const float*)a.g_loss, c0, dz, a.ldh);
+  else
+    hipLaunchKernelGGL((oace_rows_bwd_vec_kernel<DT, 1>), grid, dim3(256), 0, st, a.h, a.ldh, a.N, (int)a.V, a.targets,
+                       (const float*)rows, (const float*)a.g_loss, c0, dz, a.ldh);
+  return true;
+}
+
 template <int DT>
 hipError_t rows_fwd_dt(const OaceArgs& a, const void* z, int64_t ldz, bool z_is_acc, void* rows, hipStream_t st) {
   typedef typename OTypes<DT>::E E;
   typedef typename OTypes<DT>::A A;
-  const A inv_v = (A)(1.0 / (double)a.V);
-  if (z_is_acc)
-    hipLaunchKernelGGL((oace_rows_fwd_kernel<A, A>), dim3((unsigned)a.N), dim3(256), 0, st, (const A*)z, ldz, a.V,
-                       a.targets, (A)a.eps, (A)a.gamma, inv_v, (A*)rows);
-  else
+  if constexpr (DT == AFA_F64) {
     hipLaunchKernelGGL((oace_rows_fwd_kernel<E, A>), dim3((unsigned)a.N), dim3(256), 0, st, (const E*)z, ldz, a.V,
-                       a.targets, (A)a.eps, (A)a.gamma, inv_v, (A*)rows);
+                       a.targets, a.eps, a.gamma, 1.0 / (double)a.V, (A*)rows);
+  } else if (z_is_acc) {
+    rows_fwd_vec<AFA_F32>(a, z, ldz, rows, st);
+  } else {
+    rows_fwd_vec<DT>(a, z, ldz, rows, st);
+  }
   return hipGetLastError();
 }
 
@@ -375,12 +608,24 @@ hipError_t oace_linear_bwd_generic(int dtype, const OaceArgs& a, const void* row
   }
 }
 
-hipError_t oace_mean_launch(int dtype, const void* rows, int64_t N, void* loss, hipStream_t st) {
-  if (dtype == AFA_F64)
-    hipLaunchKernelGGL((oace_mean_kernel<double>), dim3(1), dim3(256), 0, st, (const double*)rows, N, (double*)loss);
-  else
-    hipLaunchKernelGGL((oace_mean_kernel<float>), dim3(1), dim3(256), 0, st, (const float*)rows, N, (float*)loss);
+template <typename A>
+static hipError_t mean_launch(A* rows, int64_t N, A* loss, hipStream_t st) {
+  if (N <= MEAN_ROWS) {
+    hipLaunchKernelGGL((oace_mean_kernel<A>), dim3(1), dim3(256), 0, st, rows, N, (int64_t)OACE_ROW, (int)OACE_LOSS,
+                       (A)N, loss);
+    return hipGetLastError();
+  }
+  const int64_t groups = (N + MEAN_ROWS - 1) / MEAN_ROWS;
+  hipLaunchKernelGGL((oace_mean_kernel<A>), dim3((unsigned)groups), dim3(256), 0, st, rows, N, (int64_t)OACE_ROW,
+                     (int)OACE_LOSS, A(1), (A*)nullptr);
+  hipLaunchKernelGGL((oace_mean_kernel<A>), dim3(1), dim3(256), 0, st, rows, groups, (int64_t)OACE_ROW * MEAN_ROWS,
+                     (int)OACE_ROW - 1, (A)N, loss);
   return hipGetLastError();
+}
+
+hipError_t oace_mean_launch(int dtype, void* rows, int64_t N, void* loss, hipStream_t st) {
+  if (dtype == AFA_F64) return mean_launch((double*)rows, N, (double*)loss, st);
+  return mean_launch((float*)rows, N, (float*)loss, st);
 }
 
 hipError_t oace_softmax_fwd_launch(int dtype, const OaceArgs& a, void* rows, hipStream_t st) {
@@ -400,6 +645,8 @@ static hipError_t softmax_bwd_dt(const OaceArgs& a, const void* rows, void* dz, 
   typedef typename OTypes<DT>::E E;
   typedef typename OTypes<DT>::A A;
   const A c0 = (A)(8.0 * a.gamma / (double)a.N);
+  if constexpr (DT != AFA_F64)
+    if (rows_bwd_vec<DT>(a, rows, dz, c0, st)) return hipGetLastError();
   hipLaunchKernelGGL((oace_rows_bwd_kernel<E, E, A>), dim3(bwd_grid_x(a.V), (unsigned)a.N), dim3(256), 0, st,
                      (const E*)a.h, a.ldh, a.V, a.targets, (const A*)rows, (const A*)a.g_loss, c0, (E*)dz, a.ldh);
   return hipGetLastError();

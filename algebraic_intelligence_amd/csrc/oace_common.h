@@ -42,6 +42,21 @@ __device__ __forceinline__ Oct<A> octic(A x) {
   return o;
 }
 
+// rho, rho^7 and r of the two-branch form in fp32 for the row kernels: rho(|x|) = |x| + (1+x^2) r
+// has no cancellation and rho(-x) = 1 / rho(x), so one reciprocal and one select serve the
+// negative branch; rho^8 is left to the caller as rho^7 rho.
+__device__ __forceinline__ void octic7(float x, float& rho, float& rho7, float& r) {
+  const float t = __builtin_fmaf(x, x, 1.0f);
+  r = __builtin_amdgcn_rsqf(t);
+  const float pos = __builtin_fmaf(t, r, __builtin_fabsf(x));
+  const float neg = __builtin_amdgcn_rcpf(pos);
+  // selected by the sign bit: one v_bfi instead of a compare and a v_cndmask, which waits for VCC
+  const unsigned m = (unsigned)(__builtin_bit_cast(int, x) >> 31);
+  rho = __builtin_bit_cast(float, (__builtin_bit_cast(unsigned, neg) & m) | (__builtin_bit_cast(unsigned, pos) & ~m));
+  const float k2 = rho * rho;
+  rho7 = (k2 * rho) * (k2 * k2);
+}
+
 // Branch-free fp32 octic parts: rho = fma(1 + x^2, rsqrt(1 + x^2), x) for both signs.  For x < 0
 // this cancels, but the absolute error of rho^7, rho^8 stays below ~1e-7 there (rho < 1), far
 // below the resolution of sums over a vocabulary of such terms, which is where it is used; the

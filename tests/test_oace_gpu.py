@@ -106,6 +106,34 @@ def test_softmax_loss_vs_oracle(shape, dtype):
     assert normwise(to_f64(z.grad), rz) <= (tol if dtype != torch.bfloat16 else 1e-2)
 
 
+@pytest.mark.parametrize("dtype,epc", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 8)])
+@pytest.mark.parametrize("chunks", [0, 1, 64, 128, 256, 512, 1024, 2048, 3328, 6656, 12800])
+def test_softmax_loss_row_kernels(dtype, epc, chunks):
+    """Rows at each limit of the register-resident row kernels (16-byte chunks per row), whose odd
+    lengths start every row at another offset from a 16-byte boundary, from an aligned base and from
+    one an element past it (its dz, allocated aligned, then takes the element-wise kernel); and the
+    mean over more rows than one workgroup sums.  Tolerances as test_softmax_loss_vs_oracle; fp16
+    dz (2^-11 rounding, entries of 1e-4 and up at 2^10 times the loss) 2e-3."""
+    for V in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1}):
+        N = 4099 if V <= 9 else 3
+        rng = np.random.default_rng(V)
+        for off in (0, 1):
+            buf = torch.empty(N * V + off, dtype=dtype, device=DEV)
+            buf[off:] = _t(rng.standard_normal(N * V) * 10.0, dtype)
+            z = buf[off:].view(N, V).requires_grad_(True)
+            t = torch.from_numpy(rng.integers(0, V, size=N)).to(DEV)
+            loss = A.fused_oace_softmax_loss(z, t)
+            g = 1024.0
+            (dz,) = torch.autograd.grad(loss * g, z)
+            ref, cache = O.oace_softmax_loss(to_f64(z), t.cpu().numpy())
+            # at V = 1 the loss is 0, the difference of terms of 2 * 64/7 = 18.3 whose S^(1/8) and
+            # reciprocals are within about 8 roundings of 2^-24: 8.7e-6
+            assert abs(float(loss) - ref) <= 2e-5 * abs(ref) + 8.7e-6, (V, off)
+            tol = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
+            if V > 1:
+                assert normwise(to_f64(dz), O.oace_softmax_loss_vjp(cache, g)) <= tol, (V, off)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("shape", [(16, 32, 256), (10, 20, 203), (7, 48, 1031)])
 @pytest.mark.parametrize("tied", [False, True])
