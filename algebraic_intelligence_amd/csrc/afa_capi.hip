@@ -607,9 +607,17 @@ size_t oace_rows_bytes(int dtype, int64_t rows) {
 }
 
 size_t oace_path_bytes(int dtype, const afa::OaceArgs& a, bool use_mfma) {
-  if (use_mfma) return afa::oace_mfma_workspace(dtype, a);
+  if (use_mfma) return dtype == AFA_F32 ? afa::oace_f32_workspace(a) : afa::oace_mfma_workspace(dtype, a);
   return std::max(afa::oace_generic_workspace(dtype, a.N, a.d, a.V, false),
                   afa::oace_generic_workspace(dtype, a.N, a.d, a.V, true));
+}
+
+// Matrix-core path of a call: bf16/fp16 operands that fit its loads, or fp32 split into bf16 planes.
+enum { OACE_GENERIC = 0, OACE_MFMA16 = 1, OACE_F32 = 2 };
+int oace_path(int dtype, const afa::OaceArgs& a, unsigned flags) {
+  if (flags & AFA_FLAG_GENERIC) return OACE_GENERIC;
+  if (dtype == AFA_F32) return afa::oace_f32_supported(a) ? OACE_F32 : OACE_GENERIC;
+  return afa::oace_mfma_supported(dtype, a) ? OACE_MFMA16 : OACE_GENERIC;
 }
 
 // Workspace: [row records | path scratch]; the first part is unused when the caller passes
@@ -653,9 +661,10 @@ int oace_linear_fwd(int dtype, int64_t rows, int64_t d_model, int64_t vocab, con
   }
   void* recs = row_cache ? row_cache : ws;
   void* scratch = (char*)ws + oace_rows_bytes(dtype, rows);
-  const bool mfma = !(flags & AFA_FLAG_GENERIC) && afa::oace_mfma_supported(dtype, a);
-  hipError_t e = mfma ? afa::oace_linear_fwd_mfma(dtype, a, recs, scratch, s)
-                      : afa::oace_linear_fwd_generic(dtype, a, recs, scratch, s);
+  const int path = oace_path(dtype, a, flags);
+  hipError_t e = path == OACE_MFMA16 ? afa::oace_linear_fwd_mfma(dtype, a, recs, scratch, s)
+                 : path == OACE_F32  ? afa::oace_linear_fwd_f32(a, recs, scratch, s)
+                                     : afa::oace_linear_fwd_generic(dtype, a, recs, scratch, s);
   if (owned) {
     hipError_t e2 = hipFreeAsync(ws, s);
     if (e == hipSuccess) e = e2;
@@ -687,9 +696,10 @@ int oace_linear_bwd(int dtype, int64_t rows, int64_t d_model, int64_t vocab, con
     return AFA_ERR_WORKSPACE;
   }
   void* scratch = (char*)ws + oace_rows_bytes(dtype, rows);
-  const bool mfma = !(flags & AFA_FLAG_GENERIC) && afa::oace_mfma_supported(dtype, a);
-  hipError_t e = mfma ? afa::oace_linear_bwd_mfma(dtype, a, row_cache, scratch, s)
-                      : afa::oace_linear_bwd_generic(dtype, a, row_cache, scratch, s);
+  const int path = oace_path(dtype, a, flags);
+  hipError_t e = path == OACE_MFMA16 ? afa::oace_linear_bwd_mfma(dtype, a, row_cache, scratch, s)
+                 : path == OACE_F32  ? afa::oace_linear_bwd_f32(a, row_cache, scratch, s)
+                                     : afa::oace_linear_bwd_generic(dtype, a, row_cache, scratch, s);
   if (owned) {
     hipError_t e2 = hipFreeAsync(ws, s);
     if (e == hipSuccess) e = e2;

@@ -214,6 +214,14 @@ size_t oace_mfma_workspace(int dtype, const OaceArgs& a);
 hipError_t oace_linear_fwd_mfma(int dtype, const OaceArgs& a, void* rows, void* ws, hipStream_t st);
 hipError_t oace_linear_bwd_mfma(int dtype, const OaceArgs& a, const void* rows, void* ws, hipStream_t st);
 
+// fp32 path on the bf16 matrix cores (oace_f32.hip): any d_model, strides and alignment.
+bool oace_f32_supported(const OaceArgs& a);
+size_t oace_f32_workspace(const OaceArgs& a);
+hipError_t oace_linear_fwd_f32(const OaceArgs& a, void* rows, void* ws, hipStream_t st);
+hipError_t oace_linear_bwd_f32(const OaceArgs& a, const void* rows, void* ws, hipStream_t st);
+// Row records of fp32 logits z (a.N rows of a.V, row stride ldz) (oace.hip).
+hipError_t oace_rows_z(const OaceArgs& a, const float* z, int64_t ldz, void* rows, hipStream_t st);
+
 // MFMA GEMM of the OACE backward (oace_bwd_gemm.hip): D[n][m] = sum_k A[m][k] B[n][k] in the
 // element type at out[n * ldo + m], fp32 accumulation.  An operand is row-contiguous (mc:
 // element (r, k) at p[k * ld + r]) or contraction-contiguous (element (r, k) at p[r * ld + k]).

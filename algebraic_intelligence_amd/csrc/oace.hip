@@ -628,6 +628,11 @@ hipError_t oace_mean_launch(int dtype, void* rows, int64_t N, void* loss, hipStr
   return mean_launch((float*)rows, N, (float*)loss, st);
 }
 
+hipError_t oace_rows_z(const OaceArgs& a, const float* z, int64_t ldz, void* rows, hipStream_t st) {
+  rows_fwd_vec<AFA_F32>(a, z, ldz, rows, st);
+  return hipGetLastError();
+}
+
 hipError_t oace_softmax_fwd_launch(int dtype, const OaceArgs& a, void* rows, hipStream_t st) {
   hipError_t e;
   switch (dtype) {

@@ -211,19 +211,21 @@ int ago_rotate(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int64_t
  * OACE_W_VD, (vocab, d_model) with row stride ldw (a tied token embedding, W = E^T).
  * Backward outputs: dh (rows, d_model) contiguous, in h's dtype; dw in w's layout, dtype and
  * ldw.  The vocabulary chunk size of the reference does not change the result and is not an
- * argument.  workspace: oace_workspace_size() bytes of device memory, or NULL to let the call
+ * argument.  fp32 products run as six bf16 matrix-core products of operands split exactly into
+ * three bf16 planes, accumulated in fp32; the planes take 6 bytes per element of h and w in the
+ * workspace.  workspace: oace_workspace_size() bytes of device memory, or NULL to let the call
  * allocate and free it on `stream`.  AFA_FLAG_GENERIC forces the generic (non-MFMA) kernels.
  */
 #define OACE_W_DV 0
 #define OACE_W_VD 1
 #define OACE_ROW_FIELDS 8
 /* oace_linear_bwd: the workspace is the one an oace_linear_fwd call with the same arguments used,
-   and the weights have not changed since; the transposed copy of an OACE_W_DV weight that call
-   left in it is reused. */
+   and the weights have not changed since; the transposed copy of an OACE_W_DV weight (fp32: the
+   bf16 planes of the weight) that call left in it is reused. */
 #define OACE_FLAG_WT_READY 0x10u
 /* oace_linear_bwd: as OACE_FLAG_WT_READY, and h has not changed either; the fp32 logits that the
-   forward keeps in the workspace (bf16/fp16 when rows x vocab x 4 bytes fit 256 MB) are reused,
-   so dz is formed elementwise instead of by a second GEMM.  No counterpart in the reference. */
+   forward keeps in the workspace (when rows x vocab x 4 bytes fit 256 MB) are reused, so dz is
+   formed elementwise instead of by a second GEMM.  No counterpart in the reference. */
 #define OACE_FLAG_Z_READY 0x20u
 /* oace_workspace_size / oace_linear_fwd / oace_linear_bwd (the same on all three): never keep
    the logits; the backward recomputes them (a workspace of O(rows x d_model + vocab x d_model)).

@@ -154,6 +154,51 @@ def test_linear_generic_vs_oracle(shape, dtype, tied):
     assert normwise(to_f64(dw), rw) <= (tol if dtype == torch.float64 else 1e-4)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (31, 33, 63), (128, 64, 256), (129, 65, 257), (255, 127, 513),
+                                   (257, 288, 130), (300, 40, 270000)])
+@pytest.mark.parametrize("tied", [False, True])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_linear_fp32_split_planes(shape, tied, pad):
+    """fp32 through the three-plane bf16 products at the edges of tiles, steps and splits, with odd
+    row strides (pad), and in row chunks (270000 entries: 256 rows at a time), against the fp64
+    path.  Tolerance: sums of up to 270000 terms, 16 to a rounding of 2^-24, add up to about
+    sqrt(270000 / 16) 2^-24 = 8e-6 of the largest result."""
+    N, d, V = shape
+    h, w, t = _case(N, d, V, torch.float32, seed=N + V)
+    hs = torch.zeros((N, d + pad), device=DEV)
+    hs[:, :d] = h
+    rows_n, cols = (V, d) if tied else (d, V)
+    ws = torch.zeros((rows_n, cols + pad), device=DEV)
+    ws[:, :cols] = w.t() if tied else w
+    wv = ws[:, :cols].t() if tied else ws[:, :cols]
+    loss, cache = _fwd(hs[:, :d], wv, t)
+    dh, dw = _grads(cache, 1.3)
+    ref, rcache = _fwd(h.double(), w.double(), t)
+    rh, rw = _grads(rcache, 1.3)
+    assert abs(float(loss) - float(ref)) <= 2e-5 * abs(float(ref)) + 8.7e-6  # as test_softmax_loss_row_kernels
+    if V > 1:
+        # in place of a new forward: weights changed since, or hidden rows changed since
+        assert normwise(to_f64(dh), to_f64(rh)) <= 1e-5 and normwise(to_f64(dw), to_f64(rw)) <= 1e-5
+        loss2, cache2 = _fwd(hs[:, :d], wv, t)
+        hs.add_(0.0)  # a new version: the backward forms h's planes and the logits again
+        dh2, dw2 = _grads(cache2, 1.3)
+        assert torch.equal(dh, dh2) and torch.equal(dw, dw2) and torch.equal(loss, loss2)
+
+
+def test_linear_fp32_keeps_infinities_and_nan():
+    """An infinite or NaN hidden row, and values past the largest bf16, as in the fp32 sums: only
+    the rows that hold them lose their finite results."""
+    h, w, t = _case(5, 40, 300, torch.float32, seed=4)
+    h[1, 3], h[2, 0], h[4] = float("inf"), float("nan"), 0.0
+    h[4, 0], w[0] = 3.4e38, 1e-38
+    loss, cache = _fwd(h, w, t)
+    ref, rcache = _fwd(h.double(), w.double(), t)
+    rows, rrows = cache[3][:, 6], rcache[3][:, 6]
+    assert torch.equal(torch.isfinite(rows), torch.tensor([True, False, False, True, True], device=DEV))
+    ok = torch.isfinite(rows)
+    assert normwise(to_f64(rows[ok]), to_f64(rrows[ok])) <= 2e-5
+
+
 @pytest.mark.parametrize("dtype", LOW)
 @pytest.mark.parametrize("shape", [(8, 64, 300), (130, 96, 1000), (512, 768, 50257), (3, 32, 7)])
 @pytest.mark.parametrize("tied", [False, True])
