@@ -1,23 +1,23 @@
-// fp32 ("HIGHEST") analytical AFA backward on the fp32 matrix cores (v_mfma_f32_32x32x2_f32),
-// head_dim 32, 64 and 128.  Contract of tiled_afa_backward (src/kernels/pallas_afa.py:437-522)
-// with fp32 operands, as the generic fp32 kernel computes it:
+// fp32 ("HIGHEST") analytical AFA backward on the bf16 matrix cores, head_dim 32, 48, 64, 96 and 128.
+// Contract of tiled_afa_backward (src/kernels/pallas_afa.py:437-522) with fp32 operands, as the
+// generic fp32 kernel computes it:
 //   E_i = sum_d g_id out_id;  s = (q_i . k_j) * scale;  r = rsqrt(1 + s^2);  w = rho(s)^8 / d_i;
 //   ds = 8 scale r w (g_i . v_j - E_i);  dq_i += ds_ij k_j;  dk_j += ds_ij q_i;  dv_j += w_ij g_i,
-// with rho^8 by the two-branch form; only the order of the fp32 additions differs.
+// with rho^8 by the two-branch form; only the order of the fp32 additions differs.  Every product
+// is six bf16 plane products of exactly split operands (afa_f32_split.h), as in the forward.
 //
 // Three launches, no atomics:
 //   * afa_bwd_f32_prep_kernel: E_i and 1/d_i per row into the workspace;
 //   * afa_bwd_f32_dq_kernel: one lane per query (32 per wave, 128 per workgroup), the layout of
-//     the fp32 forward: q and g stay in registers, lane group g holding head_dim entries
-//     [g D/2, (g+1) D/2); S^T = K Q^T and dP^T = V g^T contract K / V rows read as 16-byte LDS
-//     fragments; dQ^T += K^T dS^T takes the dS^T accumulator element j as its B operand as it is
-//     (element j of lane (query, g) is key 8 (j >> 2) + 4 g + (j & 3));
-//   * afa_bwd_f32_dkdv_kernel: one lane per key, the mirror image: k and v in registers, S = Q K^T
-//     and dP = g V^T from Q / g rows in LDS, then dV^T += g^T W and dK^T += Q^T dS.
-// Tiles of 32 rows are staged through registers into padded, double-buffered LDS (one barrier per
-// tile); with Cayley tables q and k are rotated in fp32 as they are staged, and dq, dk are rotated
-// back through R^T before they are stored.
+//     the fp32 forward: the planes of q and g stay in registers; S^T = K Q^T and dP^T = V g^T read
+//     K / V rows from LDS; dQ^T += K^T dS^T reads K's columns (ds_read_tr16_b64) and takes the
+//     dS^T accumulator, split in registers, as its B operand;
+//   * afa_bwd_f32_dkdv_kernel: one lane per key, the mirror image: k and v planes in registers,
+//     S = Q K^T and dP = g V^T from Q / g rows in LDS, then dV^T += g^T W and dK^T += Q^T dS.
+// Tiles of 32 rows are staged through registers, rotated and split there, into double-buffered LDS
+// (one barrier per tile); dq and dk are rotated back through R^T before they are stored.
 #include "afa_common.h"
+#include "afa_f32_split.h"
 #include "afa_launch.h"
 
 namespace afa {
@@ -25,19 +25,6 @@ namespace afa {
 namespace {
 
 constexpr int FKT = 32;  // rows per tile
-
-__device__ __forceinline__ f32x16_t fmma(float a, float b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float frot_first(float c, float s, float x0, float x1) {
-#pragma clang fp contract(off)
-  return c * x0 - s * x1;
-}
-__device__ __forceinline__ float frot_second(float c, float s, float x0, float x1) {
-#pragma clang fp contract(off)
-  return s * x0 + c * x1;
-}
 
 // rho(s)^8 (two-branch: rho(|s|)^8, reciprocal for s < 0) and r = rsqrt(1 + s^2)
 __device__ __forceinline__ float frho8r(float s, float& r) {
@@ -94,17 +81,107 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_prep_kernel(const GenArgs a) 
 }
 
 // ------------------------------------------------------------------------------ dQ
+// Bound by the sum of matrix and vector issue, as the forward.  dQ + dK/dV with prep, against
+// v_mfma_f32_32x32x2_f32: B=32 H=4 L=1024 D=64 causal rotary 798 -> 472 us, B=1 H=8 L=4096 D=64 1271 ->
+// 746 us, B=2 H=8 L=2048 D=128 causal rotary 1323 -> 813 us, B=16 H=6 L=512 D=48 205 -> 130 us; error
+// of dq, dk and dv against 64 bits 0.75 to 0.85 of what it was at every size.
+// Waves per SIMD by the register planes and accumulators of each kernel (dK/dV at head_dim 64 holds 96
+// registers of planes and 64 of accumulators: one wave with 318 of 512).
+constexpr int f32_dq_waves(int d) { return d <= 64 ? 2 : 1; }
+constexpr int f32_dkdv_waves(int d) { return d <= 32 ? 2 : 1; }
+
+// A 32-row tile of two matrices (x rotated when ROT) in flight from memory to their LDS planes.
 template <int D, bool ROT>
-__global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
-  constexpr int DV = (D + 31) / 32 * 32;  // features in 32-feature output blocks (48 -> 64)
-  constexpr int LDR = DV + 4;  // padded LDS row (shifts 16 bytes per row); features [D, DV) zero
-  constexpr int KH = D / 2;
-  constexpr int NDB = DV / 32;
-  constexpr int KJOBS = FKT * (D / 2) / 256;  // K rotation pairs per thread per tile
-  constexpr int VJOBS = (FKT * (D / 4) + 255) / 256;  // float4 of V per thread per tile
-  static_assert(FKT * (D / 2) % 256 == 0 && KJOBS >= 1, "head_dim does not fit the tile loader");
-  __shared__ __attribute__((aligned(16))) float ks[2][FKT * LDR];
-  __shared__ __attribute__((aligned(16))) float vs[2][FKT * LDR];
+struct F32Stage {
+  using X = F32Tile<D>;
+  static constexpr int JOBS = (FKT * (D / 4) + 255) / 256;  // float4 of each matrix per thread
+  static constexpr bool RAGGED = FKT * (D / 4) % 256 != 0;  // head_dim 48: the last job is half a workgroup's
+  f32x4_t x[JOBS], y[JOBS];
+  float c[JOBS][2], s[JOBS][2];
+
+  static __device__ __forceinline__ int row(int i) { return (int)(threadIdx.x + 256 * i) / (D / 4); }
+  static __device__ __forceinline__ int col(int i) { return 4 * ((int)(threadIdx.x + 256 * i) % (D / 4)); }
+
+  // rows from `r0` of two contiguous (L, D) matrices; rows past L load the last one (finite data of
+  // masked scores)
+  __device__ __forceinline__ void load(const float* xp, const float* yp, const float* rc, const float* rs, int r0,
+                                       int L) {
+    const int last = L - 1 - r0;
+    const char* xt = (const char*)(xp + (int64_t)r0 * D);
+    const char* yt = (const char*)(yp + (int64_t)r0 * D);
+    const char* ct = (const char*)(rc + (int64_t)r0 * (D / 2));
+    const char* st = (const char*)(rs + (int64_t)r0 * (D / 2));
+#pragma unroll
+    for (int i = 0; i < JOBS; ++i) {
+      const uint32_t off = (uint32_t)(min(row(i), last) * D + col(i)) * 4u;
+      x[i] = *(const f32x4_t*)(xt + off);
+      y[i] = *(const f32x4_t*)(yt + off);
+      if constexpr (ROT) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          c[i][p] = ((const float*)(ct + off / 2))[p];
+          s[i][p] = ((const float*)(st + off / 2))[p];
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void store(unsigned short* xl, unsigned short* yl) const {
+#pragma unroll
+    for (int i = 0; i < JOBS; ++i) {
+      if (RAGGED && row(i) >= FKT) continue;
+      const int at = X::at(row(i), col(i));
+      unsigned w[3][2];
+      const f32x4_t xr = ROT ? f32_rotate4(x[i], c[i], s[i]) : x[i];
+      split3_rne(xr[0], xr[1], w[0][0], w[1][0], w[2][0]);
+      split3_rne(xr[2], xr[3], w[0][1], w[1][1], w[2][1]);
+      X::put(xl, at, w);
+      split3_rne(y[i][0], y[i][1], w[0][0], w[1][0], w[2][0]);
+      split3_rne(y[i][2], y[i][3], w[0][1], w[1][1], w[2][1]);
+      X::put(yl, at, w);
+    }
+  }
+  // zero the padding features of both buffers of both matrices, once (read as operand rows)
+  static __device__ __forceinline__ void pad(unsigned short (*xl)[3 * X::PLANE], unsigned short (*yl)[3 * X::PLANE]) {
+    if constexpr (D % 32 != 0) {
+      for (int e = threadIdx.x; e < 2 * 3 * FKT * 4; e += 256) {
+        const int r = (e >> 2) % FKT, pl = (e / (4 * FKT)) % 3, buf = e / (12 * FKT);
+        const int at = pl * X::PLANE + X::at(r, D + 4 * (e & 3));
+        *(u32x2_t*)&xl[buf][at] = u32x2_t{0u, 0u};
+        *(u32x2_t*)&yl[buf][at] = u32x2_t{0u, 0u};
+      }
+    }
+  }
+};
+
+// Planes of one row's features 16 kk + 8 g .. + 7 (rotated when ROT), zeros for rows past L.
+template <int D, bool ROT>
+__device__ __forceinline__ void f32_row_planes(const float* rows, const float* rc, const float* rs, int row, int L,
+                                               int g, u32x4_t (&f)[3][D / 16]) {
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk) {
+    const int d0 = 16 * kk + 8 * g;
+    f32x4_t x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if (row < L) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        x[hh] = *(const f32x4_t*)(rows + (int64_t)row * D + d0 + 4 * hh);
+        if constexpr (ROT) {
+          const int64_t t = (int64_t)row * (D / 2) + d0 / 2 + 2 * hh;
+          x[hh] = f32_rotate4(x[hh], rc + t, rs + t);
+        }
+      }
+    }
+    split8(x[0], x[1], f[0][kk], f[1][kk], f[2][kk]);
+  }
+}
+
+template <int D, bool ROT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_dq_waves(D), f32_dq_waves(D))))
+void afa_bwd_f32_dq_kernel(const GenArgs a) {
+  using X = F32Tile<D>;
+  constexpr int NK = D / 16, NDB = (D + 31) / 32;
+  __shared__ __attribute__((aligned(16))) unsigned short ks[2][3 * X::PLANE];
+  __shared__ __attribute__((aligned(16))) unsigned short vs[2][3 * X::PLANE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -119,93 +196,21 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
   const int kend_w = a.causal ? min(vlen, q0_w + 32) : vlen;
   const int ntiles = (kend_wg + FKT - 1) / FKT;
   const int64_t base = (int64_t)bh * L * D;
-  const float* qp = (const float*)a.q + base;
   const float* kp = (const float*)a.k + base;
   const float* vp = (const float*)a.v + base;
-  const float* gp = (const float*)a.g + base;
   const float* rc = (const float*)a.rc;
   const float* rs = (const float*)a.rs;
   const float scale = (float)a.scale;
   const float c8 = 8.0f * scale;
 
-  float qf[KH], gf[KH];
-#pragma unroll
-  for (int j = 0; j < KH; j += 2) {
-    const int d0 = g * KH + j;
-    float x0 = 0.f, x1 = 0.f, y0 = 0.f, y1 = 0.f;
-    if (qi < L) {
-      x0 = qp[(int64_t)qi * D + d0];
-      x1 = qp[(int64_t)qi * D + d0 + 1];
-      y0 = gp[(int64_t)qi * D + d0];
-      y1 = gp[(int64_t)qi * D + d0 + 1];
-      if constexpr (ROT) {
-        const float c = rc[(int64_t)qi * (D / 2) + d0 / 2], s = rs[(int64_t)qi * (D / 2) + d0 / 2];
-        const float r0 = frot_first(c, s, x0, x1), r1 = frot_second(c, s, x0, x1);
-        x0 = r0;
-        x1 = r1;
-      }
-    }
-    qf[j] = x0;
-    qf[j + 1] = x1;
-    gf[j] = y0;
-    gf[j + 1] = y1;
-  }
+  F32Stage<D, ROT> stage;
+  if (ntiles > 0) stage.load(kp, vp, rc, rs, 0, L);
+  u32x4_t qf[3][NK], gf[3][NK];
+  f32_row_planes<D, ROT>((const float*)a.q + base, rc, rs, qi, L, g, qf);
+  f32_row_planes<D, false>((const float*)a.g + base, nullptr, nullptr, qi, L, g, gf);
   const int64_t rows = (int64_t)BH * L;
   const float ei = qi < L ? ((const float*)a.e_ws)[(int64_t)bh * L + qi] : 0.f;
   const float invd = qi < L ? ((const float*)a.e_ws)[rows + (int64_t)bh * L + qi] : 0.f;
-
-  float kx[KJOBS][2], kc[KJOBS], ksn[KJOBS];
-  f32x4_t vx[VJOBS];
-  auto load = [&](int t) {
-#pragma unroll
-    for (int i = 0; i < KJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-      const int key = t * FKT + r;
-      kx[i][0] = kx[i][1] = 0.f;
-      kc[i] = 1.f;
-      ksn[i] = 0.f;
-      if (key < L) {
-        kx[i][0] = kp[(int64_t)key * D + 2 * p];
-        kx[i][1] = kp[(int64_t)key * D + 2 * p + 1];
-        if constexpr (ROT) {
-          kc[i] = rc[(int64_t)key * (D / 2) + p];
-          ksn[i] = rs[(int64_t)key * (D / 2) + p];
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-      const int key = t * FKT + r;
-      f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-      vx[i] = key < L && e < FKT * (D / 4) ? *(const f32x4_t*)(vp + (int64_t)key * D + 4 * c4) : z;
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < KJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-      float y0 = kx[i][0], y1 = kx[i][1];
-      if constexpr (ROT) {
-        y0 = frot_first(kc[i], ksn[i], kx[i][0], kx[i][1]);
-        y1 = frot_second(kc[i], ksn[i], kx[i][0], kx[i][1]);
-      }
-      ks[buf][r * LDR + 2 * p] = y0;
-      ks[buf][r * LDR + 2 * p + 1] = y1;
-    }
-#pragma unroll
-    for (int i = 0; i < VJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-      if (e < FKT * (D / 4)) *(f32x4_t*)&vs[buf][r * LDR + 4 * c4] = vx[i];
-    }
-  };
-  if constexpr (DV > D) {  // the padding features of every K and V row, once
-    for (int e = tid; e < 2 * FKT * (DV - D); e += 256) {
-      const int buf = e / (FKT * (DV - D)), r = (e / (DV - D)) % FKT, f = D + e % (DV - D);
-      ks[buf][r * LDR + f] = 0.f;
-      vs[buf][r * LDR + f] = 0.f;
-    }
-  }
 
   f32x16_t dq[NDB];
 #pragma unroll
@@ -213,17 +218,15 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) dq[db][e] = 0.f;
 
-  if (ntiles > 0) {
-    load(0);
-    store(0);
-  }
+  F32Stage<D, ROT>::pad(ks, vs);
+  if (ntiles > 0) stage.store(ks[0], vs[0]);
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
-    if (t + 1 < ntiles) load(t + 1);
+    if (t + 1 < ntiles) stage.load(kp, vp, rc, rs, (t + 1) * FKT, L);
     const int key0 = t * FKT;
     if (key0 < kend_w && q0_w < L) {
-      const float* kt = ks[t & 1];
-      const float* vt = vs[t & 1];
+      const unsigned short* kt = ks[t & 1];
+      const unsigned short* vt = vs[t & 1];
       f32x16_t st, pt;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -231,14 +234,15 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
         pt[e] = 0.f;
       }
 #pragma unroll
-      for (int j4 = 0; j4 < KH / 4; ++j4) {
-        const f32x4_t kv = *(const f32x4_t*)(kt + l32 * LDR + g * KH + 4 * j4);
-        const f32x4_t vv = *(const f32x4_t*)(vt + l32 * LDR + g * KH + 4 * j4);
+      for (int kk = 0; kk < NK; ++kk) {
+        u32x4_t kf[3], vf[3];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          st = fmma(kv[u], qf[4 * j4 + u], st);
-          pt = fmma(vv[u], gf[4 * j4 + u], pt);
+        for (int p = 0; p < 3; ++p) {
+          kf[p] = X::row_frag(kt + p * X::PLANE, kk, lane);
+          vf[p] = X::row_frag(vt + p * X::PLANE, kk, lane);
         }
+        st = mma_planes(kf, qf[0][kk], qf[1][kk], qf[2][kk], st);
+        pt = mma_planes(vf, gf[0][kk], gf[1][kk], gf[2][kk], pt);
       }
       const bool need_mask = (a.causal && key0 + 31 > q0_w) || key0 + 31 >= vlen || q0_w + 31 >= L;
       float ds[16];
@@ -246,24 +250,31 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
       for (int e = 0; e < 16; ++e) {
         float rr;
         const float w = frho8r(st[e] * scale, rr) * invd;
-        float d = c8 * rr * w * (pt[e] - ei);
-        if (need_mask) {
+        ds[e] = c8 * rr * w * (pt[e] - ei);
+      }
+      if (need_mask) {
+        asm volatile("" ::: "memory");  // kept a branch on the wave-uniform test
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
           const int key = key0 + 8 * (e >> 2) + 4 * g + (e & 3);
           const bool keep = key < vlen && qi < L && (!a.causal || key <= qi);
-          d = keep ? d : 0.f;
+          ds[e] = keep ? ds[e] : 0.f;
         }
-        ds[e] = d;
       }
+      u32x4_t pk[3][2];
+      split_acc(ds, pk);
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int kr = 8 * (j >> 2) + 4 * g + (j & 3);
-          dq[db] = fmma(kt[kr * LDR + db * 32 + l32], ds[j], dq[db]);
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4_t kf[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) kf[p] = X::col_frag(kt + p * X::PLANE, db, kk, lane);
+          dq[db] = mma_planes(kf, pk[0][kk], pk[1][kk], pk[2][kk], dq[db]);
         }
     }
     // the buffer of tile t+1 was last read in tile t-1, before the previous barrier
-    if (t + 1 < ntiles) store((t + 1) & 1);
+    if (t + 1 < ntiles) stage.store(ks[(t + 1) & 1], vs[(t + 1) & 1]);
     __syncthreads();
   }
 
@@ -274,7 +285,7 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
         const int m = db * 32 + 8 * e4 + 4 * g;  // features m .. m+3 (two rotation pairs)
-        if (DV == D || m < D) {
+        if (D % 32 == 0 || m < D) {
           if constexpr (ROT) f_unrotate4<D>(dq[db], 4 * e4, rc, rs, qi, m);
           f32x4_t w;
 #pragma unroll
@@ -287,17 +298,13 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dq_kernel(const GenArgs a) {
 
 // ------------------------------------------------------------------------------ dK, dV
 template <int D, bool ROT>
-__global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) {
-  constexpr int DV = (D + 31) / 32 * 32;  // features in 32-feature output blocks (48 -> 64)
-  constexpr int LDR = DV + 4;  // features [D, DV) of the q and g rows stay zero
-  constexpr int KH = D / 2;
-  constexpr int NDB = DV / 32;
-  constexpr int QJOBS = FKT * (D / 2) / 256;  // Q rotation pairs per thread per tile
-  constexpr int GJOBS = (FKT * (D / 4) + 255) / 256;  // float4 of g per thread per tile
-  static_assert(FKT * (D / 2) % 256 == 0 && QJOBS >= 1, "head_dim does not fit the tile loader");
-  __shared__ __attribute__((aligned(16))) float qs[2][FKT * LDR];
-  __shared__ __attribute__((aligned(16))) float gs[2][FKT * LDR];
-  __shared__ float es[2][2 * FKT];  // E, then 1/d of the tile's rows
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_dkdv_waves(D), f32_dkdv_waves(D))))
+void afa_bwd_f32_dkdv_kernel(const GenArgs a) {
+  using X = F32Tile<D>;
+  constexpr int NK = D / 16, NDB = (D + 31) / 32;
+  __shared__ __attribute__((aligned(16))) unsigned short qs[2][3 * X::PLANE];
+  __shared__ __attribute__((aligned(16))) unsigned short gs[2][3 * X::PLANE];
+  __shared__ __attribute__((aligned(16))) float es[2][2 * FKT];  // E, then 1/d of the tile's rows
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -314,8 +321,6 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) 
   const int ntiles = (L + FKT - 1) / FKT;
   const int64_t base = (int64_t)bh * L * D;
   const float* qp = (const float*)a.q + base;
-  const float* kp = (const float*)a.k + base;
-  const float* vp = (const float*)a.v + base;
   const float* gp = (const float*)a.g + base;
   const float* rc = (const float*)a.rc;
   const float* rs = (const float*)a.rs;
@@ -324,87 +329,23 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) 
   const float scale = (float)a.scale;
   const float c8 = 8.0f * scale;
 
-  float kf[KH], vf[KH];
-#pragma unroll
-  for (int j = 0; j < KH; j += 2) {
-    const int d0 = g * KH + j;
-    float x0 = 0.f, x1 = 0.f, y0 = 0.f, y1 = 0.f;
-    if (kj < L) {
-      x0 = kp[(int64_t)kj * D + d0];
-      x1 = kp[(int64_t)kj * D + d0 + 1];
-      y0 = vp[(int64_t)kj * D + d0];
-      y1 = vp[(int64_t)kj * D + d0 + 1];
-      if constexpr (ROT) {
-        const float c = rc[(int64_t)kj * (D / 2) + d0 / 2], s = rs[(int64_t)kj * (D / 2) + d0 / 2];
-        const float r0 = frot_first(c, s, x0, x1), r1 = frot_second(c, s, x0, x1);
-        x0 = r0;
-        x1 = r1;
-      }
-    }
-    kf[j] = x0;
-    kf[j + 1] = x1;
-    vf[j] = y0;
-    vf[j + 1] = y1;
-  }
-
-  float qx[QJOBS][2], qc[QJOBS], qsn[QJOBS];
-  f32x4_t gx[GJOBS];
+  F32Stage<D, ROT> stage;
   float ex = 0.f;
   auto load = [&](int t) {
-#pragma unroll
-    for (int i = 0; i < QJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-      const int row = t * FKT + r;
-      qx[i][0] = qx[i][1] = 0.f;
-      qc[i] = 1.f;
-      qsn[i] = 0.f;
-      if (row < L) {
-        qx[i][0] = qp[(int64_t)row * D + 2 * p];
-        qx[i][1] = qp[(int64_t)row * D + 2 * p + 1];
-        if constexpr (ROT) {
-          qc[i] = rc[(int64_t)row * (D / 2) + p];
-          qsn[i] = rs[(int64_t)row * (D / 2) + p];
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < GJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-      const int row = t * FKT + r;
-      f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-      gx[i] = row < L && e < FKT * (D / 4) ? *(const f32x4_t*)(gp + (int64_t)row * D + 4 * c4) : z;
-    }
+    stage.load(qp, gp, rc, rs, t * FKT, L);
     if (tid < 2 * FKT) {
       const int row = t * FKT + (tid & (FKT - 1));
       ex = row < L ? (tid < FKT ? ep : ip)[row] : 0.f;
     }
   };
   auto store = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < QJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-      float y0 = qx[i][0], y1 = qx[i][1];
-      if constexpr (ROT) {
-        y0 = frot_first(qc[i], qsn[i], qx[i][0], qx[i][1]);
-        y1 = frot_second(qc[i], qsn[i], qx[i][0], qx[i][1]);
-      }
-      qs[buf][r * LDR + 2 * p] = y0;
-      qs[buf][r * LDR + 2 * p + 1] = y1;
-    }
-#pragma unroll
-    for (int i = 0; i < GJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-      if (e < FKT * (D / 4)) *(f32x4_t*)&gs[buf][r * LDR + 4 * c4] = gx[i];
-    }
+    stage.store(qs[buf], gs[buf]);
     if (tid < 2 * FKT) es[buf][tid] = ex;
   };
-  if constexpr (DV > D) {  // the padding features of every q and g row, once
-    for (int e = tid; e < 2 * FKT * (DV - D); e += 256) {
-      const int buf = e / (FKT * (DV - D)), r = (e / (DV - D)) % FKT, f = D + e % (DV - D);
-      qs[buf][r * LDR + f] = 0.f;
-      gs[buf][r * LDR + f] = 0.f;
-    }
-  }
+  if (t0 < ntiles) load(t0);
+  u32x4_t kf[3][NK], vf[3][NK];
+  f32_row_planes<D, ROT>((const float*)a.k + base, rc, rs, kj, L, g, kf);
+  f32_row_planes<D, false>((const float*)a.v + base, nullptr, nullptr, kj, L, g, vf);
 
   f32x16_t dk[NDB], dv[NDB];
 #pragma unroll
@@ -415,18 +356,16 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) 
       dv[db][e] = 0.f;
     }
 
-  if (t0 < ntiles) {
-    load(t0);
-    store(t0 & 1);
-  }
+  F32Stage<D, ROT>::pad(qs, gs);
+  if (t0 < ntiles) store(t0 & 1);
   __syncthreads();
   for (int t = t0; t < ntiles; ++t) {
     if (t + 1 < ntiles) load(t + 1);
     const int i0 = t * FKT;  // first query of the tile
     const bool live = wave_live && i0 < L && (!a.causal || i0 + 31 >= k0_w);
     if (live) {
-      const float* qt = qs[t & 1];
-      const float* gt = gs[t & 1];
+      const unsigned short* qt = qs[t & 1];
+      const unsigned short* gt = gs[t & 1];
       const float* et = es[t & 1];
       f32x16_t st, pt;
 #pragma unroll
@@ -435,42 +374,61 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) 
         pt[e] = 0.f;
       }
 #pragma unroll
-      for (int j4 = 0; j4 < KH / 4; ++j4) {
-        const f32x4_t qv = *(const f32x4_t*)(qt + l32 * LDR + g * KH + 4 * j4);
-        const f32x4_t gv = *(const f32x4_t*)(gt + l32 * LDR + g * KH + 4 * j4);
+      for (int kk = 0; kk < NK; ++kk) {
+        u32x4_t qa[3], ga[3];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          st = fmma(qv[u], kf[4 * j4 + u], st);
-          pt = fmma(gv[u], vf[4 * j4 + u], pt);
+        for (int p = 0; p < 3; ++p) {
+          qa[p] = X::row_frag(qt + p * X::PLANE, kk, lane);
+          ga[p] = X::row_frag(gt + p * X::PLANE, kk, lane);
         }
+        st = mma_planes(qa, kf[0][kk], kf[1][kk], kf[2][kk], st);
+        pt = mma_planes(ga, vf[0][kk], vf[1][kk], vf[2][kk], pt);
       }
       const bool need_mask = (a.causal && i0 < k0_w + 31) || k0_w + 31 >= vlen || i0 + 31 >= L;
       float w[16], ds[16];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int qr = 8 * (e >> 2) + 4 * g + (e & 3);  // query of element e within the tile
-        float rr;
-        float we = frho8r(st[e] * scale, rr) * et[FKT + qr];
-        float d = c8 * rr * we * (pt[e] - et[qr]);
-        if (need_mask) {
-          const int i = i0 + qr;
+      for (int e4 = 0; e4 < 4; ++e4) {
+        // queries 8 e4 + 4 g .. + 3 of the tile: their E and 1/d
+        const f32x4_t ei = *(const f32x4_t*)(et + 8 * e4 + 4 * g), iv = *(const f32x4_t*)(et + FKT + 8 * e4 + 4 * g);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int e = 4 * e4 + u;
+          float rr;
+          w[e] = frho8r(st[e] * scale, rr) * iv[u];
+          ds[e] = c8 * rr * w[e] * (pt[e] - ei[u]);
+        }
+      }
+      if (need_mask) {
+        asm volatile("" ::: "memory");  // kept a branch on the wave-uniform test
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int i = i0 + 8 * (e >> 2) + 4 * g + (e & 3);
           const bool keep = kj < vlen && i < L && (!a.causal || kj <= i);
-          we = keep ? we : 0.f;
-          d = keep ? d : 0.f;
+          w[e] = keep ? w[e] : 0.f;
+          ds[e] = keep ? ds[e] : 0.f;
         }
-        w[e] = we;
-        ds[e] = d;
       }
+      u32x4_t pk[3][2];
+      split_acc(w, pk);
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) {
+      for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int qr = 8 * (j >> 2) + 4 * g + (j & 3);
-          dv[db] = fmma(gt[qr * LDR + db * 32 + l32], w[j], dv[db]);
-          dk[db] = fmma(qt[qr * LDR + db * 32 + l32], ds[j], dk[db]);
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4_t f[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) f[p] = X::col_frag(gt + p * X::PLANE, db, kk, lane);
+          dv[db] = mma_planes(f, pk[0][kk], pk[1][kk], pk[2][kk], dv[db]);
         }
-        __builtin_amdgcn_sched_barrier(0);  // keep each feature block's LDS reads with its MFMAs
-      }
+      split_acc(ds, pk);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4_t f[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) f[p] = X::col_frag(qt + p * X::PLANE, db, kk, lane);
+          dk[db] = mma_planes(f, pk[0][kk], pk[1][kk], pk[2][kk], dk[db]);
+        }
     }
     if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
@@ -484,7 +442,7 @@ __global__ __launch_bounds__(256) void afa_bwd_f32_dkdv_kernel(const GenArgs a) 
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
         const int m = db * 32 + 8 * e4 + 4 * g;
-        if (DV == D || m < D) {
+        if (D % 32 == 0 || m < D) {
           if constexpr (ROT) f_unrotate4<D>(dk[db], 4 * e4, rc, rs, kj, m);
           f32x4_t wk, wv;
 #pragma unroll

@@ -208,7 +208,7 @@ FwdPlan fwd_plan(int dtype, int64_t B, int64_t H, int64_t L, int64_t D, int64_t 
     p.kind = FWD_F32;
     // fewer 128-query workgroups than CUs: split every query block's key tiles over up to
     // 2 * CUs workgroups in all (partials in the workspace, then a combine kernel).  Fewer than
-    // the kernel's resident slots (4, 2 and 1 per CU at head_dim 32, 48-64 and 96-128) with rows
+    // about the kernel's resident slots (4, 2 and 1 per CU at head_dim 32, 48-64 and 96-128) with rows
     // of at least 1024 keys: split up to the slots.  Shorter rows do not repay the partials'
     // traffic and the combine (a 16-shard ring hop of 256 keys: 31 against 39 us per hop).
     const int64_t nwg = B * H * ((L + 127) / 128);
@@ -306,6 +306,9 @@ int afa_fwd(int dtype, int64_t batch, int64_t heads, int64_t seq_len, int64_t he
   bool f32_layout = aligned16(v) && aligned16(out);
   for (int i : {6, 7, 8, 9, 10, 11})
     if (st.v[i] % 4 != 0) f32_layout = false;
+  // 32-bit byte offsets within a tile of 32 keys
+  for (int i : {5, 8})
+    if (st.v[i] < 0 || st.v[i] >= (int64_t(1) << 23)) f32_layout = false;
   auto in_head_32 = [&](int64_t row_stride) {
     return row_stride >= 0 && (seq_len - 1) * row_stride + head_dim < (int64_t(1) << 31);
   };
@@ -380,7 +383,6 @@ int afa_fwd(int dtype, int64_t batch, int64_t heads, int64_t seq_len, int64_t he
       }
     }
   } else if (plan.kind == FWD_F32) {
-    a.q_scale = (float)(1.0 / std::sqrt((double)head_dim));
     a.part = plan.nsplit > 1 ? (float*)(ws + plan.part) : nullptr;
     e = afa::f32_fwd_launch((int)head_dim, a, plan.nsplit, s);
   } else {

@@ -1,0 +1,174 @@
+// fp32 products on the bf16 matrix cores: exact three-plane splits and the LDS tiles of planes.
+//
+// x = hi + mid + lo with three bf16 values holds an fp32 value exactly (3 x 8 significant bits), and
+//   x y = hi hi' + (hi mid' + mid hi') + (mid mid' + hi lo' + lo hi') + terms below 2^-23 |x y|,
+// six products of the bf16 matrix cores, accumulated in fp32.  They run at 16 times the fp32 rate:
+// 2.7 times after six passes, and one fp32 rounding serves 16 of the contraction where the fp32
+// MFMA's serves two.
+#pragma once
+
+#include "afa_common.h"
+
+namespace afa {
+
+// Planes of a pair, packed.  Rounded to nearest: the dropped terms are at most 2^-24 |x y|.  An
+// infinity, or a value that rounds past the largest bf16, gives a NaN in the lower planes: for
+// operands whose infinite products already end as NaN (scores: rho of an infinite score is NaN).
+__device__ __forceinline__ void split3_rne(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
+  hi = pack_bf16(x0, x1);
+  const float r0 = x0 - bf16_lo(hi), r1 = x1 - bf16_hi(hi);
+  mid = pack_bf16(r0, r1);
+  lo = pack_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));
+}
+
+// Planes of four values whose infinities must come out of the product as infinities (v, and the
+// cotangent): hi is rounded towards zero, so it cannot overflow, and an infinity, which the planes
+// of the other operand (zeros and both signs) would turn into NaN, leaves zeros and returns true:
+// its terms are added by inf_terms.
+__device__ __forceinline__ bool split3_trunc(f32x4_t x, unsigned (&w)[3][2]) {
+  const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])),
+                                  __builtin_fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])));
+  const bool inf = m == __builtin_inff();
+  if (inf) {
+    asm volatile("" ::: "memory");  // keeps the rare case a branch
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = __builtin_isinf(x[i]) ? 0.f : x[i];
+  }
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const float x0 = x[2 * p], x1 = x[2 * p + 1];
+    const unsigned u0 = __builtin_bit_cast(unsigned, x0), u1 = __builtin_bit_cast(unsigned, x1);
+    w[0][p] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+    const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xffff0000u);
+    const float r1 = x1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
+    w[1][p] = pack_bf16(r0, r1);
+    w[2][p] = pack_bf16(r0 - bf16_lo(w[1][p]), r1 - bf16_hi(w[1][p]));
+  }
+  return inf;
+}
+
+// The terms of infinite elements of one 32-row tile x (row stride ld, `rows` rows of it exist):
+// acc[db][e] += p[row] x[row][feature] over
+// the infinite x, p in accumulator order (element e of lane group g is row 8 (e >> 2) + 4 g +
+// (e & 3)) and acc as the transposed product leaves it.  Reached only by tiles that hold an infinity.
+template <int D, int NDB>
+__device__ __forceinline__ void inf_terms(const float* x, int64_t ld, int rows, const float (&p)[16],
+                                          f32x16_t (&acc)[NDB]) {
+  const int g = (threadIdx.x >> 5) & 1;
+#pragma unroll 1
+  for (int r = 0; r < min(32, rows); ++r) {
+    float mine = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mine = e == 4 * (r >> 3) + (r & 3) ? p[e] : mine;
+    const float other = __shfl_xor(mine, 32);
+    const float pr = ((r >> 2) & 1) == g ? mine : other;
+    const float* row = x + (int64_t)r * ld;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int f = db * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
+        const float v = f < D ? row[f] : 0.f;
+        if (__builtin_isinf(v)) acc[db][e] += pr * v;
+      }
+  }
+}
+
+// acc += A B over 16 of the contraction, both operands as planes; smallest terms first.
+__device__ __forceinline__ f32x16_t mma_planes(const u32x4_t (&a)[3], u32x4_t b0, u32x4_t b1, u32x4_t b2,
+                                               f32x16_t acc) {
+  const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, a[0]), a1 = __builtin_bit_cast(bf16x8_t, a[1]);
+  const bf16x8_t a2 = __builtin_bit_cast(bf16x8_t, a[2]);
+  const bf16x8_t c0 = __builtin_bit_cast(bf16x8_t, b0), c1 = __builtin_bit_cast(bf16x8_t, b1);
+  const bf16x8_t c2 = __builtin_bit_cast(bf16x8_t, b2);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, c0, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, c2, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, c1, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, c0, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, c1, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, c0, acc, 0, 0, 0);
+}
+
+typedef __attribute__((ext_vector_type(4))) short f32s_s16x4_t;
+typedef __attribute__((address_space(3))) f32s_s16x4_t f32s_lds_s16x4_t;
+
+// LDS tile of 32 rows x D features of one plane: rows of RP = 64 or 128 elements whose 16-byte chunks
+// are permuted by a key of the row that is conflict-free for reads along the rows (16-byte fragments
+// of 32 rows: the 16 rows of a pass take all 16 chunk slots of a bank period) and down the columns
+// (ds_read_tr16_b64: the 8 rows of a pass go to different 4-chunk groups).
+template <int D>
+struct F32Tile {
+  static constexpr int RP = D <= 64 ? 64 : 128;
+  static constexpr int PLANE = 32 * RP;
+  static __device__ __forceinline__ int key(int r) {
+    return RP == 128 ? (r & 15) ^ ((r & 3) << 2) : ((r & 2) << 1) | ((r >> 2) & 3);
+  }
+  // element offset in the plane of features c .. c + 3 (c a multiple of 4) of row r
+  static __device__ __forceinline__ int at(int r, int c) { return r * RP + (((c >> 3) ^ key(r)) << 3) + (c & 4); }
+  static __device__ __forceinline__ void put(unsigned short* tile, int at, const unsigned (&w)[3][2]) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *(u32x2_t*)(tile + p * PLANE + at) = u32x2_t{w[p][0], w[p][1]};
+  }
+  // operand rows l32, contraction over the features 16 kk + 8 g .. + 7
+  static __device__ __forceinline__ u32x4_t row_frag(const unsigned short* plane, int kk, int lane) {
+    const int r = lane & 31, g = lane >> 5;
+    return *(const u32x4_t*)(plane + r * RP + (((2 * kk + g) ^ key(r)) << 3));
+  }
+  // operand rows = features 32 db + l32, contraction over the tile rows
+  // 16 kk + 8 (i >> 2) + 4 g + (i & 3), i = 0 .. 7: the row order of an accumulator's elements
+  static __device__ __forceinline__ u32x4_t col_frag(const unsigned short* plane, int db, int kk, int lane) {
+    const int l16 = lane & 15, m16 = (lane >> 4) & 1, g = lane >> 5;
+    u32x4_t f;
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const int row = 16 * kk + 8 * hh + 4 * g + (l16 >> 2);
+      const int col = db * 32 + m16 * 16 + 4 * (l16 & 3);
+      const f32s_s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((f32s_lds_s16x4_t*)(plane + at(row, col)));
+      const u32x2_t w = __builtin_bit_cast(u32x2_t, v);
+      f[2 * hh] = w[0];
+      f[2 * hh + 1] = w[1];
+    }
+    return f;
+  }
+};
+
+// The 16 elements of an accumulator as B-operand planes of a product that contracts its rows.
+__device__ __forceinline__ void split_acc(const float (&x)[16], u32x4_t (&pk)[3][2]) {
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      unsigned hi, mid, lo;
+      split3_rne(x[8 * kk + 2 * u], x[8 * kk + 2 * u + 1], hi, mid, lo);
+      pk[0][kk][u] = hi;
+      pk[1][kk][u] = mid;
+      pk[2][kk][u] = lo;
+    }
+}
+
+// Planes of 8 consecutive features (two float4), as one 16-feature step's operand.
+__device__ __forceinline__ void split8(f32x4_t a, f32x4_t b, u32x4_t& p0, u32x4_t& p1, u32x4_t& p2) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    unsigned hi, mid, lo;
+    const f32x4_t x = u < 2 ? a : b;
+    split3_rne(x[2 * (u & 1)], x[2 * (u & 1) + 1], hi, mid, lo);
+    p0[u] = hi;
+    p1[u] = mid;
+    p2[u] = lo;
+  }
+}
+
+// (x0, x1) -> (c x0 - s x1, s x0 + c x1) of two pairs, every operation rounded.
+__device__ __forceinline__ f32x4_t f32_rotate4(f32x4_t x, const float* c, const float* s) {
+#pragma clang fp contract(off)
+  f32x4_t y;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    y[2 * p] = c[p] * x[2 * p] - s[p] * x[2 * p + 1];
+    y[2 * p + 1] = s[p] * x[2 * p] + c[p] * x[2 * p + 1];
+  }
+  return y;
+}
+
+}  // namespace afa

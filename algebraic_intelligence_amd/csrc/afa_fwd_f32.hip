@@ -1,25 +1,29 @@
-// fp32 ("HIGHEST") fused AFA forward on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), for
-// head_dim 32, 64 and 128.  Same contract as the generic fp32 path (src/kernels/pallas_afa.py:
-// 52-151 with fp32 operands): s = (q . k) scale in fp32, w = rho(s)^8 by the cancellation-safe
-// two-branch form, out = sum_j w v_j / (sum_j w + Omega), d = sum_j w + Omega; only the order of
-// the fp32 additions differs.
+// fp32 ("HIGHEST") fused AFA forward on the bf16 matrix cores, for head_dim 32, 48, 64, 96 and 128.
+// Same contract as the generic fp32 path (src/kernels/pallas_afa.py:52-151 with fp32 operands): s =
+// (q . k) scale in fp32, w = rho(s)^8 by the cancellation-safe two-branch form, out = sum_j w v_j /
+// (sum_j w + Omega), d = sum_j w + Omega; only the order of the fp32 additions differs.
+//
+// Every fp32 operand of the two products is split exactly into three bf16 planes (F32Planes in
+// afa_f32_split.h) and a product is the six plane products of at least 2^-16 relative weight,
+// accumulated in fp32: 2.7 times the rate of v_mfma_f32_32x32x2_f32 for both products.
 //
 // A wave owns 32 queries; a unit is 32 keys x 32 queries.
-//   S^T = K Q^T: 32x32x2 steps over head_dim.  The two k-slots of a step are split by lane group
-//   g: group g contracts head_dim entries [g D/2, (g+1) D/2), so a lane reads its K row as
-//   contiguous 16-byte LDS fragments and keeps its query's half of q in registers.
+//   S^T = K Q^T: 32x32x16 steps over head_dim, the query planes in registers, K planes read as
+//   16-byte LDS fragments.
 //   O^T += V^T P^T: the S^T accumulator of lane (query c, group g) holds keys 8 (e >> 2) + 4 g +
-//   (e & 3); contracting key (j, g) at step j makes element j of that accumulator the B operand as
-//   it is, and the A operand one V element per lane (consecutive lanes, consecutive features).
-// K/V tiles of 32 keys are staged through registers into double-buffered, padded LDS rows (the
-// Cayley rotation of k is applied in that pass, as the generic kernel does), one barrier per tile.
-// Query blocks are dispatched heaviest first (block_item).
+//   (e & 3); its weights are split in registers and are the B operand as they are, in the key order
+//   in which ds_read_tr16_b64 returns the V planes' columns.
+// K/V tiles of 32 keys are staged through registers (loads of tile t + 1 in flight during tile t),
+// rotated and split there -- a pre-pass that left planes in memory would write and read 6 bytes
+// per element where a tile is read by only L / 256 query blocks on average -- into double-buffered
+// LDS, one barrier per tile.  Query blocks are dispatched heaviest first (block_item).
 // Small grids (fewer workgroups than CUs) split every query block's key tiles over blockIdx.y:
 // the numerator and denominator are sums over keys, so each split writes its partial O and row
 // sum, and afa_fwd_f32_combine_kernel adds them, adds the sink and divides.
-#include <climits>
+#include <cmath>
 
 #include "afa_common.h"
+#include "afa_f32_split.h"
 #include "afa_launch.h"
 
 namespace afa {
@@ -28,33 +32,30 @@ namespace {
 
 constexpr int KT = 32;  // keys per tile
 
-__device__ __forceinline__ f32x16_t mma_f32(float a, float b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float rot_first(float c, float s, float x0, float x1) {
-#pragma clang fp contract(off)
-  return c * x0 - s * x1;
-}
-__device__ __forceinline__ float rot_second(float c, float s, float x0, float x1) {
-#pragma clang fp contract(off)
-  return s * x0 + c * x1;
-}
-
 }  // namespace
 
+// Waves per SIMD: the query planes alone take 24, 48 and 96 registers at head_dim 32, 64 and 128 (at
+// head_dim 64 three waves spill 7 to 21 registers and measured 10% slower; at 32 they measured 293 -> 272
+// us on B=8 H=16 L=2048).
+constexpr int f32_waves(int d) { return d <= 32 ? 3 : d <= 64 ? 2 : 1; }
+
+// Bound by the sum of its matrix and vector issue: at B=1 H=8 L=4096 D=64, 1536 matrix cycles per
+// unit and 430 vector instructions of four cycles (rho^8 with its reciprocal 128, the split of the
+// weights 88, staging 140) account for 98% of the SIMD cycles, at the 2.0 GHz the device holds.  332
+// -> 216 us there, 233 -> 147 us at B=32 H=4 L=1024 D=64 (causal, rotary), 384 -> 267 us at B=2 H=8
+// L=2048 D=128, against v_mfma_f32_32x32x2_f32; error against 64 bits 6.3e-7 -> 4.9e-7, 8.3e-7 ->
+// 6.5e-7, 9.3e-7 -> 7.6e-7.
 template <int D, bool ROT, bool SPLIT>
-__global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
-  constexpr int LDR = D + 4;   // padded LDS row: consecutive rows shift by 16 bytes (no conflicts)
-  constexpr int DV = (D + 31) / 32 * 32;  // V features in 32-feature output blocks (48 -> 64)
-  constexpr int LDV = DV + 4;  // V rows; features [D, DV) stay zero
-  constexpr int KH = D / 2;    // head_dim entries per lane group
-  constexpr int NDB = DV / 32; // 32-feature output blocks
-  constexpr int KJOBS = KT * (D / 2) / 256;  // rotation pairs per thread per tile
-  constexpr int VJOBS = (KT * (D / 4) + 255) / 256;  // float4 of V per thread per tile
-  static_assert(KT * (D / 2) % 256 == 0 && KJOBS >= 1, "head_dim does not fit the tile loader");
-  __shared__ __attribute__((aligned(16))) float ks[2][KT * LDR];
-  __shared__ __attribute__((aligned(16))) float vs[2][KT * LDV];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_waves(D), f32_waves(D))))
+void afa_fwd_f32_kernel(const FwdArgs a) {
+  using X = F32Tile<D>;
+  constexpr int NK = D / 16;               // 16-feature steps of S
+  constexpr int NDB = (D + 31) / 32;       // 32-feature output blocks
+  constexpr int JOBS = (KT * (D / 4) + 255) / 256;  // float4 of K, and of V, per thread per tile
+  constexpr bool RAGGED = KT * (D / 4) % 256 != 0;  // head_dim 48: the last job is half a workgroup's
+  __shared__ __attribute__((aligned(16))) unsigned short ks[2][3 * X::PLANE];
+  __shared__ __attribute__((aligned(16))) unsigned short vs[2][3 * X::PLANE];
+  __shared__ int vinf[2];  // the tile in each buffer if it holds an infinite v, else not
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -79,94 +80,93 @@ __global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
   const float* qp = (const float*)a.q + b * a.q_b + h * a.q_h;
   const float* kp = (const float*)a.k + b * a.k_b + h * a.k_h;
   const float* vp = (const float*)a.v + b * a.v_b + h * a.v_h;
-
-  // q: lane (query qi, group g) holds features [g KH, (g+1) KH), rotated in fp32 when ROT
-  float qf[KH];
+  // rows of q and k may start at any dword (a dwordx4 load needs no more); v and out rows are
+  // 16-byte aligned (checked by the caller)
+  typedef f32x4_t f32x4_dword_t __attribute__((aligned(4)));
+  auto load4 = [](const float* p) -> f32x4_t { return *(const f32x4_dword_t*)p; };
+  // the first tile's loads go out before q's
+  f32x4_t kx[JOBS], vx[JOBS];
+  float kc[JOBS][2], ksn[JOBS][2];
+  int jrow[JOBS], jcol[JOBS];
 #pragma unroll
-  for (int j = 0; j < KH; j += 2) {
-    const int d0 = g * KH + j;
-    float x0 = 0.f, x1 = 0.f;
-    if (qi < L) {
-      x0 = qp[(int64_t)qi * a.q_l + d0];
-      x1 = qp[(int64_t)qi * a.q_l + d0 + 1];
-      if constexpr (ROT) {
-        const float c = a.rc[(int64_t)qi * (D / 2) + d0 / 2], s = a.rs[(int64_t)qi * (D / 2) + d0 / 2];
-        const float y0 = rot_first(c, s, x0, x1), y1 = rot_second(c, s, x0, x1);
-        x0 = y0;
-        x1 = y1;
-      }
+  for (int i = 0; i < JOBS; ++i) {
+    const int e = tid + 256 * i;
+    jrow[i] = e / (D / 4);
+    jcol[i] = 4 * (e % (D / 4));
+  }
+  // Lane offsets within a tile are the same in every tile (32 bits, checked by the caller): a tile
+  // moves the uniform base pointers.  In the tile that reaches past the sequence, rows past it load
+  // its last row: finite data for masked keys.
+  uint32_t koff[JOBS], voff[JOBS], toff[JOBS];
+  auto offsets = [&](int last) {
+#pragma unroll
+    for (int i = 0; i < JOBS; ++i) {
+      const int r = min(jrow[i], last);
+      koff[i] = (uint32_t)(r * (int)a.k_l + jcol[i]) * 4u;
+      voff[i] = (uint32_t)(r * (int)a.v_l + jcol[i]) * 4u;
+      toff[i] = (uint32_t)(r * (D / 2) + jcol[i] / 2) * 4u;
     }
-    qf[j] = x0;
-    qf[j + 1] = x1;
-  }
-
-  // tile staging in registers: K as rotation pairs, V as float4.  Each thread's elements sit at
-  // the same offsets in every tile: those offsets are formed once, and a tile only moves the
-  // (wave-uniform) base pointers by KT rows.
-  float kx[KJOBS][2];
-  float kc[KJOBS], ksn[KJOBS];
-  f32x4_t vx[VJOBS];
-  int64_t koff[KJOBS], voff[VJOBS];
-  int krow[KJOBS], vrow[VJOBS], toff[KJOBS];
-#pragma unroll
-  for (int i = 0; i < KJOBS; ++i) {
-    const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-    krow[i] = r;
-    koff[i] = (int64_t)r * a.k_l + 2 * p;
-    toff[i] = r * (D / 2) + p;
-  }
-#pragma unroll
-  for (int i = 0; i < VJOBS; ++i) {
-    const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-    vrow[i] = e < KT * (D / 4) ? r : INT_MAX;  // past the tile (head_dim 48): never loaded
-    voff[i] = (int64_t)r * a.v_l + 4 * c4;
-  }
+  };
+  offsets(KT - 1);
   auto load = [&](int t) {
-    const int rows = L - t * KT;  // rows of tile t inside the sequence
-    const float* kt = kp + (int64_t)t * KT * a.k_l;
-    const float* vt = vp + (int64_t)t * KT * a.v_l;
+    if (L - t * KT < KT) offsets(L - 1 - t * KT);
+    const char* kt = (const char*)(kp + (int64_t)t * KT * a.k_l);
+    const char* vt = (const char*)(vp + (int64_t)t * KT * a.v_l);
+    const char* ct = (const char*)(a.rc + (int64_t)t * KT * (D / 2));
+    const char* st = (const char*)(a.rs + (int64_t)t * KT * (D / 2));
 #pragma unroll
-    for (int i = 0; i < KJOBS; ++i) {
-      kx[i][0] = kx[i][1] = 0.f;
-      kc[i] = 1.f;
-      ksn[i] = 0.f;
-      if (krow[i] < rows) {
-        kx[i][0] = kt[koff[i]];
-        kx[i][1] = kt[koff[i] + 1];
-        if constexpr (ROT) {
-          kc[i] = a.rc[(int64_t)t * KT * (D / 2) + toff[i]];
-          ksn[i] = a.rs[(int64_t)t * KT * (D / 2) + toff[i]];
+    for (int i = 0; i < JOBS; ++i) {
+      kx[i] = load4((const float*)(kt + koff[i]));
+      vx[i] = load4((const float*)(vt + voff[i]));
+      if constexpr (ROT) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          kc[i][p] = ((const float*)(ct + toff[i]))[p];
+          ksn[i][p] = ((const float*)(st + toff[i]))[p];
         }
       }
     }
+  };
+  auto store = [&](int t) {
+    const int buf = t & 1;
 #pragma unroll
-    for (int i = 0; i < VJOBS; ++i) {
-      f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-      vx[i] = vrow[i] < rows ? *(const f32x4_t*)(vt + voff[i]) : z;
+    for (int i = 0; i < JOBS; ++i) {
+      const int r = jrow[i], c = jcol[i];
+      if (RAGGED && r >= KT) continue;
+      const f32x4_t y = ROT ? f32_rotate4(kx[i], kc[i], ksn[i]) : kx[i];
+      unsigned w[3][2];
+      split3_rne(y[0], y[1], w[0][0], w[1][0], w[2][0]);
+      split3_rne(y[2], y[3], w[0][1], w[1][1], w[2][1]);
+      X::put(ks[buf], X::at(r, c), w);
+      if (split3_trunc(vx[i], w)) vinf[buf] = t;
+      X::put(vs[buf], X::at(r, c), w);
     }
   };
-  auto store = [&](int buf) {
+  if (t_beg < ntiles) load(t_beg);
+
+  // q planes (B operand of S^T): lane (query qi, group g) holds features 16 kc + 8 g .. + 7
+  u32x4_t qf[3][NK];
 #pragma unroll
-    for (int i = 0; i < KJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 2), p = e % (D / 2);
-      float y0 = kx[i][0], y1 = kx[i][1];
-      if constexpr (ROT) {
-        y0 = rot_first(kc[i], ksn[i], kx[i][0], kx[i][1]);
-        y1 = rot_second(kc[i], ksn[i], kx[i][0], kx[i][1]);
+  for (int kk = 0; kk < NK; ++kk) {
+    const int d0 = 16 * kk + 8 * g;
+    f32x4_t x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if (qi < L) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        x[hh] = load4(qp + (int64_t)qi * a.q_l + d0 + 4 * hh);
+        if constexpr (ROT) {
+          const float* c = a.rc + (int64_t)qi * (D / 2) + d0 / 2 + 2 * hh;
+          const float* s = a.rs + (int64_t)qi * (D / 2) + d0 / 2 + 2 * hh;
+          x[hh] = f32_rotate4(x[hh], c, s);
+        }
       }
-      ks[buf][r * LDR + 2 * p] = y0;
-      ks[buf][r * LDR + 2 * p + 1] = y1;
     }
-#pragma unroll
-    for (int i = 0; i < VJOBS; ++i) {
-      const int e = tid + 256 * i, r = e / (D / 4), c4 = e % (D / 4);
-      if (e < KT * (D / 4)) *(f32x4_t*)&vs[buf][r * LDV + 4 * c4] = vx[i];
-    }
-  };
-  if constexpr (DV > D) {  // the padding features of both V buffers, once
-    for (int e = tid; e < 2 * KT * (DV - D); e += 256) {
-      const int buf = e / (KT * (DV - D)), r = (e / (DV - D)) % KT, f = D + e % (DV - D);
-      vs[buf][r * LDV + f] = 0.f;
+    split8(x[0] * a.q_scale, x[1] * a.q_scale, qf[0][kk], qf[1][kk], qf[2][kk]);
+  }
+  if constexpr (D % 32 != 0) {  // the padding features of both V buffers, once
+    for (int e = tid; e < 2 * 3 * KT * 4; e += 256) {
+      const int r = (e >> 2) % KT, pl = (e / (4 * KT)) % 3, buf = e / (12 * KT);
+      *(u32x2_t*)&vs[buf][pl * X::PLANE + X::at(r, D + 4 * (e & 3))] = u32x2_t{0u, 0u};
     }
   }
 
@@ -176,31 +176,31 @@ __global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
   float dsum = 0.f;
-  const float scale = a.q_scale;
 
-  if (t_beg < ntiles) {
-    load(t_beg);
-    store(t_beg & 1);
-  }
+  if (tid < 2) vinf[tid] = -1;
+  __syncthreads();
+  if (t_beg < ntiles) store(t_beg);
   __syncthreads();
   for (int t = t_beg; t < ntiles; ++t) {
-    if (t + 1 < ntiles) load(t + 1);  // global loads in flight during this tile's MFMAs
+    if (t + 1 < ntiles) load(t + 1);  // global loads in flight during this tile's products
     const int key0 = t * KT;
     if (key0 < kend_w && q0_w < L) {
-      const float* kt = ks[t & 1];
-      const float* vt = vs[t & 1];
+      const unsigned short* kt = ks[t & 1];
+      const unsigned short* vt = vs[t & 1];
       f32x16_t st;
 #pragma unroll
       for (int e = 0; e < 16; ++e) st[e] = 0.f;
 #pragma unroll
-      for (int j4 = 0; j4 < KH / 4; ++j4) {
-        const f32x4_t kv = *(const f32x4_t*)(kt + l32 * LDR + g * KH + 4 * j4);
+      for (int kk = 0; kk < NK; ++kk) {
+        u32x4_t kf[3];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) st = mma_f32(kv[u], qf[4 * j4 + u], st);
+        for (int p = 0; p < 3; ++p) kf[p] = X::row_frag(kt + p * X::PLANE, kk, lane);
+        st = mma_planes(kf, qf[0][kk], qf[1][kk], qf[2][kk], st);
       }
       const bool need_mask = (a.causal && key0 + 31 > q0_w) || key0 + 31 >= vlen || q0_w + 31 >= L;
+      float w[16];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) st[e] = rho8_exact(st[e] * scale);
+      for (int e = 0; e < 16; ++e) w[e] = rho8_exact(D == 64 ? st[e] : st[e] * a.s_mult);
       if (need_mask) {
         // a side effect the compiler cannot move keeps this a branch on the wave-uniform test
         // instead of a compare and a select per score in every tile
@@ -209,33 +209,39 @@ __global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
         for (int e = 0; e < 16; ++e) {
           const int key = key0 + 8 * (e >> 2) + 4 * g + (e & 3);
           const bool keep = key < vlen && qi < L && (!a.causal || key <= qi);
-          st[e] = keep ? st[e] : 0.f;
+          w[e] = keep ? w[e] : 0.f;
         }
       }
       float ts = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) ts += st[e];
+      for (int e = 0; e < 16; ++e) ts += w[e];
       // two-level sums: the tile's own (row sum and PV from zero), then added to the running
       // ones, as the reference adds one block's dot(p, v) at a time
       // (src/kernels/pallas_afa.py:131-139); a single chain over L keys would carry a rounding
       // error growing with L (4.8e-6 normwise at L = 4096 against 1.3e-6 for 256-key chains)
       dsum += ts;
+      u32x4_t pk[3][2];
+      split_acc(w, pk);
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
         f32x16_t ot;
 #pragma unroll
         for (int e = 0; e < 16; ++e) ot[e] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int kr = 8 * (j >> 2) + 4 * g + (j & 3);
-          ot = mma_f32(vt[kr * LDV + db * 32 + l32], st[j], ot);
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4_t vf[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) vf[p] = X::col_frag(vt + p * X::PLANE, db, kk, lane);
+          ot = mma_planes(vf, pk[0][kk], pk[1][kk], pk[2][kk], ot);
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[db][e] += ot[e];
       }
+      if (__builtin_amdgcn_readfirstlane(vinf[t & 1]) == t)
+        inf_terms<D, NDB>(vp + (int64_t)t * KT * a.v_l, a.v_l, L - t * KT, w, o);
     }
     // the buffer of tile t+1 was last read in tile t-1, before the previous barrier
-    if (t + 1 < ntiles) store((t + 1) & 1);
+    if (t + 1 < ntiles) store(t + 1);
     __syncthreads();
   }
 
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int e4 = 0; e4 < 4; ++e4) {
-          if (DV == D || db * 32 + 8 * e4 + 4 * g < D) {
+          if (D % 32 == 0 || db * 32 + 8 * e4 + 4 * g < D) {
             f32x4_t w;
 #pragma unroll
             for (int u = 0; u < 4; ++u) w[u] = o[db][4 * e4 + u];
@@ -270,7 +276,7 @@ __global__ __launch_bounds__(256) void afa_fwd_f32_kernel(const FwdArgs a) {
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
-        if (DV == D || db * 32 + 8 * e4 + 4 * g < D) {
+        if (D % 32 == 0 || db * 32 + 8 * e4 + 4 * g < D) {
           f32x4_t* p = (f32x4_t*)(op + db * 32 + 8 * e4 + 4 * g);
           f32x4_t w;
           if (a.acc) {
@@ -362,6 +368,13 @@ static hipError_t f32_launch_d(const FwdArgs& a, int nsplit, hipStream_t st) {
 
 hipError_t f32_fwd_launch(int head_dim, FwdArgs a, int nsplit, hipStream_t st) {
   a.nqb = (a.L + 127) / 128;
+  // 1/sqrt(D): the power of two below it folded into q exactly, the rest an fp32 factor of the
+  // score (1 at D = 64)
+  const float scale = (float)(1.0 / std::sqrt((double)head_dim));
+  int ex = 0;
+  (void)std::frexp(scale, &ex);
+  a.q_scale = std::ldexp(1.0f, ex - 1);
+  a.s_mult = std::ldexp(scale, 1 - ex);
   if (head_dim == 32) return f32_launch_d<32>(a, nsplit, st);
   if (head_dim == 48) return f32_launch_d<48>(a, nsplit, st);
   if (head_dim == 64) return f32_launch_d<64>(a, nsplit, st);

@@ -127,8 +127,8 @@ PipeSplit pipe_split_plan(int head_dim, int64_t BH, int64_t L, bool causal, int 
 // a.ks_*: the split (ks_tiles = 0 for none; the counters cleared by a pre-pass of the same call).
 hipError_t pipe_fwd_launch(int dtype, int head_dim, FwdArgs a, bool exact, hipStream_t stream);
 
-// fp32 forward on the fp32 MFMA (afa_fwd_f32.hip): head_dim 32/64/128, V and out rows 16-byte
-// aligned; q_scale carries 1/sqrt(head_dim) (applied to the fp32 dot product).
+// fp32 forward on the bf16 MFMAs, operands split in three planes (afa_fwd_f32.hip): head_dim 32,
+// 48, 64, 96, 128, V and out rows 16-byte aligned.
 bool f32_fwd_supported(int head_dim);
 // nsplit > 1: the key range of every query block is split over nsplit workgroups whose partial
 // numerators and row sums go to a.part (f32_fwd_part_floats(a, head_dim, nsplit) floats), then

@@ -401,3 +401,30 @@ def test_pipelined_d128_edge_shapes(shape, causal, valid, rot, dt):
     tol = _ulp_tol(dt)
     assert e_s <= tol and e_c <= tol
     assert normwise(to_f64(da), c_den) <= 1e-5
+
+
+@pytest.mark.parametrize("D", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("L,causal,valid", [(1, True, None), (31, True, None), (33, False, 32), (160, True, 129),
+                                            (300, False, None)])
+@pytest.mark.parametrize("rot", [False, True])
+def test_f32_planes_strides_and_infinities(D, L, causal, valid, rot):
+    """The fp32 forward (operands split into bf16 planes) on rows of q and k that start at any
+    dword and are strided, against the fp64 kernel (4e-6 normwise: s to about 2^-24 |q||k|, eight times that
+    relative in rho^8), and an infinite v as an infinite output of its feature
+    only, in the rows that see it."""
+    shape = (1, 2, L, D)
+    q, k, v = make_qkv(shape, torch.float32, seed=L + D)
+    wide = torch.zeros((1, 2, L, D + 3), device="cuda")
+    flat = torch.empty(wide.numel() + 1, device="cuda")[1:].view(wide.shape)
+    wide[..., :D], flat[..., :D] = q, k
+    rotary = A.build_cayley_rotary_matrix(D, L) if rot else None
+    out, den = _fwd(wide[..., :D], flat[..., :D], v, causal=causal, valid=valid, rotary=rotary)
+    r64 = None if rotary is None else (rotary.c.double(), rotary.s.double())
+    ref, rden = _fwd(q.double(), k.double(), v.double(), causal=causal, valid=valid, rotary=r64)
+    assert normwise(to_f64(out), to_f64(ref)) <= 4e-6 and normwise(to_f64(den), to_f64(rden)) <= 4e-6
+    j = (L if valid is None else valid) // 2
+    v[0, 1, j, 5], v[0, 0, 0, 3] = float("-inf"), 1e30
+    out, _ = _fwd(q, k, v, causal=False, valid=valid, rotary=rotary)
+    gen, _ = _fwd(q, k, v, causal=False, valid=valid, rotary=rotary, flags=_lib.FLAG_GENERIC)
+    bad = ~torch.isfinite(gen)
+    assert bad[0, 1, :, 5].all() and torch.equal(bad, ~torch.isfinite(out)) and torch.equal(out[bad], gen[bad])
