@@ -77,8 +77,9 @@ __device__ __forceinline__ void inf_terms(const float* x, int64_t ld, int rows, 
 // acc += A B over 16 of the contraction, both operands as planes; smallest terms first.
 __device__ __forceinline__ f32x16_t mma_planes(const u32x4_t (&a)[3], u32x4_t b0, u32x4_t b1, u32x4_t b2,
                                                f32x16_t acc) {
-  const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, a[0]), a1 = __builtin_bit_cast(bf16x8_t, a[1]);
-  const bf16x8_t a2 = __builtin_bit_cast(bf16x8_t, a[2]);
+  const u32x4_t w0 = a[0], w1 = a[1], w2 = a[2];
+  const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, w0), a1 = __builtin_bit_cast(bf16x8_t, w1);
+  const bf16x8_t a2 = __builtin_bit_cast(bf16x8_t, w2);
   const bf16x8_t c0 = __builtin_bit_cast(bf16x8_t, b0), c1 = __builtin_bit_cast(bf16x8_t, b1);
   const bf16x8_t c2 = __builtin_bit_cast(bf16x8_t, b2);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, c0, acc, 0, 0, 0);
