@@ -46,6 +46,7 @@ SIGNATURES = {
     "octic_bwd": (_int, [_int, _i64, _vp, _vp, _vp, _vp]),
     "ago_build_tables": (_int, [_int, _i64, _i64, _vp, _dbl, _vp, _vp, _vp]),
     "ago_rotate": (_int, [_int, _i64, _i64, _i64, _i64, _vp, _vp, _int, _vp, _vp, _i64, _vp]),
+    "ago_rotate_qk": (_int, [_int, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp, _vp, _i64, _int, _vp]),
     "oace_workspace_size": (_sz, [_int, _i64, _i64, _i64, _int, _uint]),
     "oace_linear_fwd": (_int, [_int, _i64, _i64, _i64, _vp, _i64, _vp, _int, _i64, _vp, _dbl, _dbl, _vp, _vp,
                                _uint, _vp, _sz, _vp]),

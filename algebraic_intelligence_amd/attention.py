@@ -7,6 +7,7 @@ Every computation runs in the gfx950 kernels of libafa_hip.so (include/afa.h).
 """
 from __future__ import annotations
 
+import math
 from typing import NamedTuple
 
 import torch
@@ -216,24 +217,24 @@ def _infer_seq_axis(shape, param_len):
     return ndim - 2
 
 
-def _rotate_launch(x, c, s, seq_axis):
+def _rotate_launch(x, c, s, seq_axis, other=None, transpose=False):
+    """x, and other (of x's shape and dtype, or None) in the same launch, rotated by the table rows
+    of their sequence axis, or back when transpose."""
     dev = _lib.require_device(x, c, s)
     xc = x.contiguous()
-    seq = xc.shape[seq_axis]
-    outer = 1
-    for n in xc.shape[:seq_axis]:
-        outer *= n
-    inner = 1
-    for n in xc.shape[seq_axis + 1:-1]:
-        inner *= n
+    oc = None if other is None else other.contiguous()
+    shape = xc.shape
+    outer = math.prod(shape[:seq_axis])
+    inner = math.prod(shape[seq_axis + 1:-1])
     y = torch.empty_like(xc)
+    z = None if other is None else torch.empty_like(oc)
     cc, sc = c.contiguous(), s.contiguous()
     with torch.cuda.device(dev):
-        rc = _lib.lib().ago_rotate(_lib.dtype_code(x.dtype), outer, seq, inner, xc.shape[-1], _lib.ptr(xc),
-                                   _lib.ptr(y), _lib.dtype_code(cc.dtype), _lib.ptr(cc), _lib.ptr(sc),
-                                   cc.shape[0], _lib.stream_ptr(dev))
-    _lib.check(rc, "ago_rotate")
-    return y
+        rc = _lib.lib().ago_rotate_qk(_lib.dtype_code(x.dtype), outer, shape[seq_axis], inner, shape[-1], _lib.ptr(xc),
+                                      _lib.ptr(oc), _lib.ptr(y), _lib.ptr(z), _lib.dtype_code(cc.dtype), _lib.ptr(cc),
+                                      _lib.ptr(sc), cc.shape[0], int(transpose), _lib.stream_ptr(dev))
+    _lib.check(rc, "ago_rotate_qk")
+    return y if other is None else (y, z)
 
 
 class _Rotate(torch.autograd.Function):
@@ -247,19 +248,48 @@ class _Rotate(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         c, s, seq_axis = ctx.cfg
-        return _rotate_launch(g.contiguous(), c, -s, seq_axis), None, None, None
+        return _rotate_launch(g, c, s, seq_axis, transpose=True), None, None, None
+
+
+class _RotatePair(torch.autograd.Function):
+    """_Rotate of q and k of one shape and dtype, each direction in one launch."""
+
+    @staticmethod
+    def forward(ctx, q, k, c, s, seq_axis):
+        ctx.cfg = (c, s, seq_axis)
+        ctx.set_materialize_grads(False)
+        out = _rotate_launch(q, c, s, seq_axis, k)
+        fixed = [y for y, need in zip(out, ctx.needs_input_grad) if not need]
+        if fixed:
+            ctx.mark_non_differentiable(*fixed)
+        return out
+
+    @staticmethod
+    def backward(ctx, gq, gk):
+        c, s, seq_axis = ctx.cfg
+        if gq is not None and gk is not None and gq.dtype == gk.dtype:
+            gq, gk = _rotate_launch(gq, c, s, seq_axis, gk, transpose=True)
+        else:
+            gq, gk = (None if g is None else _rotate_launch(g, c, s, seq_axis, transpose=True) for g in (gq, gk))
+        return gq, gk, None, None, None
 
 
 def rotate_tensor(x: torch.Tensor, c: torch.Tensor, s: torch.Tensor, seq_axis: int) -> torch.Tensor:
     """Rotate (even, odd) feature pairs of x by the table rows of its sequence axis
     (src/attention.py:142-152); c and s are (>= L, D/2) tables."""
+    c, s = _tables_for(x, c, s, seq_axis)
+    return _Rotate.apply(_float_input(x), c, s, seq_axis % x.ndim)
+
+
+def _tables_for(x, c, s, seq_axis):
+    """(rows, D/2) views of tables that cover x's sequence axis."""
     if x.shape[-1] % 2 != 0:
         raise ValueError(f"Feature dimension must be even, got {x.shape[-1]}")
     c = _lib.table_2d(c, x.shape[-1])
     s = _lib.table_2d(s, x.shape[-1])
     if c.shape[0] < x.shape[seq_axis]:
         raise ValueError("rotary tables are shorter than the sequence")
-    return _Rotate.apply(_float_input(x), c, s, seq_axis % x.ndim)
+    return c, s
 
 
 def _align_param(param, q_shape, seq_axis=None):
@@ -329,4 +359,7 @@ def apply_ago_rotations(q, k, rotary_params=None, seq_axis=None):
     s_raw = torch.as_tensor(s_raw, device=q.device)
     if seq_axis is None:
         seq_axis = _infer_seq_axis(tuple(q.shape), c_raw.shape[0])
-    return rotate_tensor(q, c_raw, s_raw, seq_axis), rotate_tensor(k, c_raw, s_raw, seq_axis)
+    if q.dtype != k.dtype or q.device != k.device:
+        return rotate_tensor(q, c_raw, s_raw, seq_axis), rotate_tensor(k, c_raw, s_raw, seq_axis)
+    c, s = _tables_for(q, c_raw, s_raw, seq_axis)
+    return _RotatePair.apply(_float_input(q), _float_input(k), c, s, seq_axis % ndim)

@@ -562,12 +562,19 @@ int ago_build_tables(int table_dtype, int64_t dim, int64_t max_seq_len, const vo
 int ago_rotate(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int64_t dim,
                const void* x, void* y, int table_dtype, const void* rot_cos,
                const void* rot_sin, int64_t rot_len, void* stream) {
+  return ago_rotate_qk(dtype, outer, seq_len, inner, dim, x, nullptr, y, nullptr, table_dtype, rot_cos, rot_sin, rot_len,
+                       0, stream);
+}
+
+int ago_rotate_qk(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int64_t dim, const void* q,
+                  const void* k, void* q_out, void* k_out, int table_dtype, const void* rot_cos,
+                  const void* rot_sin, int64_t rot_len, int transpose, void* stream) {
   if (!valid_dtype(dtype) || !valid_dtype(table_dtype)) return AFA_ERR_DTYPE;
-  if (!x || !y || !rot_cos || !rot_sin) return AFA_ERR_NULL;
+  if (!q || !q_out || !rot_cos || !rot_sin || (k == nullptr) != (k_out == nullptr)) return AFA_ERR_NULL;
   if (outer <= 0 || seq_len <= 0 || inner <= 0 || dim <= 0) return AFA_ERR_SHAPE;
   if (dim % 2 != 0 || rot_len < seq_len) return AFA_ERR_ROTARY;
-  return hip_status(afa::ago_rotate_launch(dtype, table_dtype, outer, seq_len, inner, (int)dim, x, y,
-                                           rot_cos, rot_sin, (hipStream_t)stream));
+  return hip_status(afa::ago_rotate_launch(dtype, table_dtype, outer, seq_len, inner, (int)dim, q, k, q_out, k_out,
+                                           rot_cos, rot_sin, transpose != 0, (hipStream_t)stream));
 }
 
 // ------------------------------------------------------------------------------ OACE

@@ -152,9 +152,10 @@ hipError_t generic_bwd_launch(int dtype, const GenArgs& a, hipStream_t st);
 
 hipError_t ago_tables_launch(int table_dtype, int pairs, int len, const void* freqs, double base,
                              void* c_out, void* s_out, hipStream_t st);
-hipError_t ago_rotate_launch(int dtype, int table_dtype, int64_t outer, int64_t seq, int64_t inner,
-                             int dim, const void* x, void* y, const void* rc, const void* rs,
-                             hipStream_t st);
+// xb, yb: a second tensor of the same shape (nullptr: none).  transpose: the inverse rotation.
+hipError_t ago_rotate_launch(int dtype, int table_dtype, int64_t outer, int64_t seq, int64_t inner, int dim,
+                             const void* xa, const void* xb, void* ya, void* yb, const void* rc, const void* rs,
+                             bool transpose, hipStream_t st);
 
 hipError_t asoftmax_fwd_launch(int dtype, int64_t rows, int64_t n, const void* x, void* y,
                                double sink, double eps, hipStream_t st);

@@ -193,6 +193,12 @@ int ago_build_tables(int table_dtype, int64_t dim, int64_t max_seq_len, const vo
 int ago_rotate(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int64_t dim,
                const void* x, void* y, int table_dtype, const void* rot_cos,
                const void* rot_sin, int64_t rot_len, void* stream);
+/* The same for q and k in one launch (k and k_out both nullable); transpose != 0 rotates by the
+ * transposed blocks (the VJP).  Replaces the two rotations of apply_ago_rotations (:207-240). */
+int ago_rotate_qk(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int64_t dim,
+                  const void* q, const void* k, void* q_out, void* k_out, int table_dtype,
+                  const void* rot_cos, const void* rot_sin, int64_t rot_len, int transpose,
+                  void* stream);
 
 /*
  * OACE loss head.  Calc type A: fp32, fp64 for AFA_F64 inputs.  targets: int64 class indices

@@ -7,6 +7,8 @@ contract restatement (oracle/).  Tolerances are normwise, max|y - ref| / max|ref
 """
 import os
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -584,3 +586,47 @@ def test_backward_linearity_full_size(shape, rot):
         e = normwise(to_f64(a12), to_f64(a1) + to_f64(a2))
         print(f"{shape} rot={rot} {name}: d(g1+g2) vs d(g1)+d(g2) {e:.2e}")
         assert e <= 1e-2, name
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("table_dt", [torch.float32, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("shape,axis,off", [((1, 1, 1, 8), 2, 0), ((5, 3, 67, 64), 2, 0), ((5, 67, 3, 48), 1, 0),
+                                            ((9, 130, 4), 1, 0), ((3, 2, 33, 20), 2, 0), ((2, 2, 40, 32), 2, 1),
+                                            ((300, 96), 0, 0)])
+def test_rotation_of_q_and_k_in_one_launch(dt, table_dt, shape, axis, off):
+    """apply_ago_rotations (both tensors in one launch: 16-byte chunks of up to four slices per
+    thread, or element by element for rows of no whole chunks and unaligned tensors) is bitwise the
+    rotation in fp32 (fp64) of the tables cast to x's dtype, forward and backward, with one or both
+    gradients asked for."""
+    D, L = shape[-1], shape[axis]
+    acc = torch.float64 if dt == torch.float64 else torch.float32
+    gen = torch.Generator(device=DEV).manual_seed(D + L)
+    def draw():
+        flat = torch.empty(math.prod(shape) + off, dtype=dt, device=DEV)[off:]
+        flat.copy_(torch.randn(flat.numel(), generator=gen, device=DEV))
+        return flat.view(shape)
+    q, k, gq, gk = (draw() for _ in range(4))
+    rot = A.build_cayley_rotary_matrix(D, L + 3, device=DEV)
+    c, s = rot.c.to(table_dt), rot.s.to(table_dt)
+    bshape = [1] * len(shape)
+    bshape[axis], bshape[-1] = L, D // 2
+    cb, sb = (t[:L].to(table_dt).to(dt if dt != torch.float64 else torch.float64).to(acc).reshape(bshape)
+              for t in (c, s))
+    def want(x, sign):
+        a, b = x[..., 0::2].to(acc), x[..., 1::2].to(acc)
+        sg = sb * sign
+        return torch.stack((cb * a - sg * b, sg * a + cb * b), -1).reshape(shape).to(dt)
+    for need_q, need_k in ((True, True), (True, False), (False, True), (False, False)):
+        qi, ki = q.detach().requires_grad_(need_q), k.detach().requires_grad_(need_k)
+        qr, kr = A.apply_ago_rotations(qi, ki, (c, s), seq_axis=axis)
+        assert torch.equal(qr, want(q, 1)) and torch.equal(kr, want(k, 1))
+        assert qr.requires_grad == need_q and kr.requires_grad == need_k
+        outs = [(y, g) for y, g, n in ((qr, gq, need_q), (kr, gk, need_k)) if n]
+        if outs:
+            ins = [x for x, n in ((qi, need_q), (ki, need_k)) if n]
+            got = torch.autograd.grad([y for y, _ in outs], ins, [g for _, g in outs])
+            assert all(torch.equal(d, want(g, -1)) for d, (_, g) in zip(got, outs))
+    qi, ki = q.detach().requires_grad_(True), k.detach().requires_grad_(True)
+    qr, kr = A.apply_ago_rotations(qi, ki, (c, s), seq_axis=axis)
+    (only,) = torch.autograd.grad(kr, ki, gk)  # q's output unused
+    assert torch.equal(only, want(gk, -1))
