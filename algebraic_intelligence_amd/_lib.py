@@ -5,7 +5,9 @@ missing or stale build raises instead of falling back.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import os
 import threading
 
@@ -111,8 +113,35 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+# torch.cuda.current_stream() builds a Stream object (2 us of a 19 us forward call); the raw handle
+# of the same stream is a C call
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """A context in which `device` is the current one: torch.cuda.device(device), or nothing to do
+    where it already is."""
+    return _HERE if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+@functools.lru_cache(maxsize=4096)
+def _workspace(name: str, device_index, *sizes) -> int:
+    return getattr(lib(), name)(*sizes)
+
+
+def workspace_size(name: str, device: torch.device, *sizes) -> int:
+    """A workspace query, a function of the sizes and the device it runs on; called with that device
+    current.  Kept for the sizes a program repeats."""
+    return _workspace(name, device.index, *sizes)
 
 
 def ptr(t):

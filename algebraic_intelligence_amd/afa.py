@@ -47,6 +47,10 @@ def _rotary_tables(rotary_params, q: torch.Tensor):
         raise TypeError(f"Unsupported rotary parameters type: {type(rotary_params)}")
     tdt = torch.float64 if q.dtype == torch.float64 else torch.float32
     D = q.shape[-1]
+    if (isinstance(c, torch.Tensor) and isinstance(s, torch.Tensor) and c.dtype == tdt and s.dtype == tdt
+            and c.ndim == 2 and D % 2 == 0 and c.shape[1] == D // 2 and c.shape == s.shape and c.device == q.device
+            and s.device == q.device and c.is_contiguous() and s.is_contiguous()):
+        return c, s, c.shape[0]  # as the kernel takes them
     c = table_2d(torch.as_tensor(c, device=q.device), D)
     s = table_2d(torch.as_tensor(s, device=q.device), D)
     if c.shape != s.shape:
@@ -55,7 +59,10 @@ def _rotary_tables(rotary_params, q: torch.Tensor):
 
 
 def _strides(*ts):
-    """12 element strides (b, h, l per tensor); head_dim must be contiguous."""
+    """12 element strides (b, h, l per tensor), or None (NULL) where every tensor is contiguous;
+    head_dim must be contiguous."""
+    if all(t.is_contiguous() for t in ts):
+        return None
     out = []
     for t in ts:
         out.extend(t.stride()[:3])
@@ -77,9 +84,9 @@ def _launch_fwd(q, k, v, sink_omega, causal, valid_seq_len, rotary_params, flags
     B, H, L, D = q.shape
     out = torch.empty((B, H, L, D), dtype=q.dtype, device=dev)
     den = torch.empty((B, H, L, 1), dtype=_lib.accum_dtype(q.dtype), device=dev) if want_denominator else None
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         # the workspace comes from torch's caching allocator, so the library allocates nothing
-        ws_bytes = _lib.lib().afa_fwd_workspace_size(dt, B, H, L, D, int(c is not None))
+        ws_bytes = _lib.workspace_size("afa_fwd_workspace_size", dev, dt, B, H, L, D, int(c is not None))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         rc = _lib.lib().afa_fwd(
             dt, B, H, L, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _strides(q, k, v, out),
@@ -218,9 +225,9 @@ def tiled_afa_backward(
     d_total = d_total.to(_lib.accum_dtype(q.dtype)).contiguous()
     dq, dk, dv = (torch.empty_like(t) for t in (q, k, v))
     c, s, rot_len = _rotary_tables(rotary_params, q)
-    ws_bytes = _lib.lib().afa_bwd_workspace_size(dt, B, H, L, D, int(c is not None))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
+        ws_bytes = _lib.workspace_size("afa_bwd_workspace_size", dev, dt, B, H, L, D, int(c is not None))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         rc = _lib.lib().afa_bwd(
             dt, B, H, L, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(d_total),
             _lib.ptr(g_out), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(c), _lib.ptr(s),
@@ -317,7 +324,7 @@ def _ring_forward(q, k, v, sink_omega, causal, n, want_total):
     total = torch.empty((B, H, L, 1), dtype=acc.dtype, device=dev) if want_total else None
     accd = _device_major(acc, n)
     L_ = _lib.lib()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
         ws_bytes = max(L_.afa_fwd_workspace_size(dt, m, B * H, S, D, 0) for m in range(1, n + 1))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None

@@ -37,7 +37,7 @@ class _Octic(torch.autograd.Function):
         dev = _lib.require_device(x)
         xc = x.contiguous()
         y = torch.empty_like(xc)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().octic_fwd(_lib.dtype_code(x.dtype), xc.numel(), _lib.ptr(xc), _lib.ptr(y),
                                       _lib.stream_ptr(dev))
         _lib.check(rc, "octic_fwd")
@@ -50,7 +50,7 @@ class _Octic(torch.autograd.Function):
         dev = x.device
         gc = g.to(x.dtype).contiguous()
         dx = torch.empty_like(x)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().octic_bwd(_lib.dtype_code(x.dtype), x.numel(), _lib.ptr(x), _lib.ptr(gc),
                                       _lib.ptr(dx), _lib.stream_ptr(dev))
         _lib.check(rc, "octic_bwd")
@@ -85,7 +85,7 @@ def _kernel(z):
     acc = _lib.accum_dtype(z.dtype)
     k = torch.empty(zc.shape, dtype=acc, device=dev)
     r = torch.empty(zc.shape, dtype=acc, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().octic_fwd_r(_lib.dtype_code(z.dtype), zc.numel(), _lib.ptr(zc), _lib.ptr(k), _lib.ptr(r),
                                     _lib.stream_ptr(dev))
     _lib.check(rc, "octic_fwd_r")
@@ -101,7 +101,7 @@ class _ASoftmax(torch.autograd.Function):
         cols = xc.shape[-1]
         rows = xc.numel() // cols
         y = torch.empty_like(xc)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().asoftmax_fwd(_lib.dtype_code(x.dtype), rows, cols, _lib.ptr(xc), _lib.ptr(y),
                                          float(sink_omega), float(eps), _lib.stream_ptr(dev))
         _lib.check(rc, "asoftmax_fwd")
@@ -116,7 +116,7 @@ class _ASoftmax(torch.autograd.Function):
         gc = g.to(x.dtype).contiguous()
         dx = torch.empty_like(x)
         cols = x.shape[-1]
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             rc = _lib.lib().asoftmax_bwd(_lib.dtype_code(x.dtype), x.numel() // cols, cols, _lib.ptr(x),
                                          _lib.ptr(gc), _lib.ptr(dx), float(sink_omega), float(eps),
                                          _lib.stream_ptr(x.device))
@@ -181,7 +181,7 @@ def build_cayley_rotary_matrix(dim: int, max_seq_len: int, freqs=None, base: flo
     _lib.require_device(torch.empty(0, device=device))
     c = torch.empty((max_seq_len, pairs), dtype=calc, device=device)
     s = torch.empty_like(c)
-    with torch.cuda.device(device):
+    with _lib.on_device(device):
         rc = _lib.lib().ago_build_tables(_lib.dtype_code(calc), dim, max_seq_len, _lib.ptr(f), float(base),
                                          _lib.ptr(c), _lib.ptr(s), _lib.stream_ptr(device))
     _lib.check(rc, "ago_build_tables")
@@ -229,7 +229,7 @@ def _rotate_launch(x, c, s, seq_axis, other=None, transpose=False):
     y = torch.empty_like(xc)
     z = None if other is None else torch.empty_like(oc)
     cc, sc = c.contiguous(), s.contiguous()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().ago_rotate_qk(_lib.dtype_code(x.dtype), outer, shape[seq_axis], inner, shape[-1], _lib.ptr(xc),
                                       _lib.ptr(oc), _lib.ptr(y), _lib.ptr(z), _lib.dtype_code(cc.dtype), _lib.ptr(cc),
                                       _lib.ptr(sc), cc.shape[0], int(transpose), _lib.stream_ptr(dev))

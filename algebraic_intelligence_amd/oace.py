@@ -77,9 +77,9 @@ def fused_linear_oace_forward(h, w_vocab, targets, eps_vocab: float = 100.0, gam
     rows = torch.empty((N, ROW_FIELDS), dtype=acc, device=dev)
     code = _lib.dtype_code(h.dtype)
     # the backward reuses this workspace (and the transposed weights the forward leaves in it)
-    wsb = _lib.lib().oace_workspace_size(code, N, d, V, layout, flags)
-    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
+        wsb = _lib.workspace_size("oace_workspace_size", dev, code, N, d, V, layout, flags)
+        ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
         rc = _lib.lib().oace_linear_fwd(code, N, d, V, hf.data_ptr(), hf.stride(0), wop.data_ptr(), layout, ldw,
                                         t.data_ptr(), float(eps_vocab), float(gamma), loss.data_ptr(), rows.data_ptr(),
                                         flags, ws.data_ptr(), wsb, _lib.stream_ptr(dev))
@@ -109,7 +109,7 @@ def fused_linear_oace_backward(cache, g):
     # and its logits unless h or w_vocab was
     w_same = w_vocab._version == w_version
     bflags = flags | (FLAG_WT_READY if w_same else 0) | (FLAG_Z_READY if w_same and hf._version == h_version else 0)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().oace_linear_bwd(_lib.dtype_code(hf.dtype), hf.shape[0], d, V, hf.data_ptr(), hf.stride(0),
                                         wop.data_ptr(), layout, ldw, t.data_ptr(), float(gamma), rows.data_ptr(),
                                         gt.data_ptr(), dh.data_ptr(), dw_store.data_ptr(), bflags, ws.data_ptr(),
@@ -157,7 +157,7 @@ class _FusedOACESoftmaxLoss(torch.autograd.Function):
         acc = _lib.accum_dtype(z.dtype)
         loss = torch.empty((), dtype=acc, device=dev)
         rows = torch.empty((z2.shape[0], ROW_FIELDS), dtype=acc, device=dev)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().oace_softmax_loss_fwd(_lib.dtype_code(z.dtype), z2.shape[0], V, z2.data_ptr(), t.data_ptr(),
                                                   float(eps), float(gamma), loss.data_ptr(), rows.data_ptr(),
                                                   _lib.stream_ptr(dev))
@@ -173,7 +173,7 @@ class _FusedOACESoftmaxLoss(torch.autograd.Function):
         gt = torch.as_tensor(g, dtype=rows.dtype, device=dev).reshape(())
         dz = torch.empty_like(z)
         V = z.shape[-1]
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.lib().oace_softmax_loss_bwd(_lib.dtype_code(z.dtype), t.numel(), V, z.data_ptr(), t.data_ptr(),
                                                   ctx.gamma, rows.data_ptr(), gt.data_ptr(), dz.data_ptr(),
                                                   _lib.stream_ptr(dev))
