@@ -207,207 +207,189 @@ __device__ __forceinline__ float octic_hw(float z, float& r_out) {
 }
 
 // ---------------------------------------------------------------- register-resident row kernels
-// One wave per row, the whole row held in registers: 16-byte vector loads (lane l owns chunks
-// l, l + 64, ... of EPC elements), one HBM read of x (and g), one write; rho^8 and r are
-// evaluated once per element with the hardware rsqrt / reciprocal (octic_hw) and the row is
-// normalised with one division and products; the multi-pass kernels above keep IEEE 1/sqrt and
-// divisions throughout.  Used when the row fits
-// (cols <= 64 * EPC * NCH) and cols is a multiple of the chunk width on 16-byte-aligned rows.
-template <int DT>
-struct Chunk {
-  static constexpr int EPC = DT == AFA_F32 ? 4 : 8;
-  static __device__ __forceinline__ void load(const void* p, int64_t e0, float (&v)[8]) {
-    const u32x4_t w = *(const u32x4_t*)((const char*)p + e0 * (DT == AFA_F32 ? 4 : 2));
-    if constexpr (DT == AFA_F32) {
+// T threads per row (one wave, or 4 or 8 waves for longer rows), the whole row held in registers as the
+// aligned 16-byte chunks that cover it (RowChunk: any length and any start; thread l owns chunks
+// l, l + T, ...): one HBM read of x (and g), one write; rho^8 and r are evaluated once per element
+// with the hardware rsqrt / reciprocal (octic_hw) and the row is normalised with one division and
+// products; the multi-pass kernels above keep IEEE 1/sqrt and divisions throughout.  Entries of a
+// chunk outside the row are zeros: they add nothing to the sum of squares and 1 (rho(0)) each to the
+// octic sum, taken off again.
+// Forward of (18372, 1531) fp32 109 -> 41 us (5.5 TB/s) and its VJP 267 -> 80 us (4.2 TB/s) against the
+// multi-pass kernels, which served every row whose length was no multiple of a chunk or over 64 x 8
+// (VJP: 64 x 4) chunks.
+template <int T, int K>
+__device__ __forceinline__ void row_sum(float (&x)[K], float* sh) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // bind the element first: a bit_cast of a runtime-indexed vector element reads element 0
-        const unsigned u = w[i];
-        v[i] = __builtin_bit_cast(float, u);
-      }
-    } else {
+  for (int q = 0; q < K; ++q) x[q] = wave_sum(x[q]);
+  if constexpr (T > 64) {
+    constexpr int NW = T / 64;
+    const int wave = threadIdx.x >> 6;
+    __syncthreads();  // the previous sum's values have been read
+    if ((threadIdx.x & 63) == 0)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = Elem<DT>::lo(w[i]);
-        v[2 * i + 1] = Elem<DT>::hi(w[i]);
-      }
-    }
-  }
-  static __device__ __forceinline__ void store(void* p, int64_t e0, const float (&v)[8]) {
-    u32x4_t w;
-    if constexpr (DT == AFA_F32) {
+      for (int q = 0; q < K; ++q) sh[q * NW + wave] = x[q];
+    __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float f = v[i];
-        w[i] = __builtin_bit_cast(unsigned, f);
-      }
-    } else {
+    for (int q = 0; q < K; ++q) {
+      x[q] = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = Elem<DT>::pack(v[2 * i], v[2 * i + 1]);
-    }
-    *(u32x4_t*)((char*)p + e0 * (DT == AFA_F32 ? 4 : 2)) = w;
-  }
-};
-
-template <int DT, int NCH>
-__global__ __launch_bounds__(256) void asoftmax_fwd_reg_kernel(int64_t rows, int64_t n, const void* x,
-                                                               void* y, double sink, double eps) {
-#pragma clang fp contract(off)
-  constexpr int EPC = Chunk<DT>::EPC;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const int64_t base = row * n;
-  float v[NCH][8];
-  float ss = 0.f;
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int64_t e0 = (int64_t)(lane + 64 * j) * EPC;
-    if (e0 < n) {
-      Chunk<DT>::load(x, base + e0, v[j]);
-#pragma unroll
-      for (int i = 0; i < EPC; ++i) ss += v[j][i] * v[j][i];
-    }
-  }
-  ss = wave_sum(ss);
-  const float tau = inv_sqrt(ss * (1.f / (float)n) + (float)eps);
-  float ks = 0.f;
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    if ((int64_t)(lane + 64 * j) * EPC < n) {
-#pragma unroll
-      for (int i = 0; i < EPC; ++i) {
-        float r;
-        v[j][i] = octic_hw(v[j][i] * tau, r);
-        ks += v[j][i];
-      }
-    }
-  }
-  ks = wave_sum(ks);
-  const float inv = 1.0f / (ks + (float)sink);
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int64_t e0 = (int64_t)(lane + 64 * j) * EPC;
-    if (e0 < n) {
-#pragma unroll
-      for (int i = 0; i < EPC; ++i) v[j][i] = v[j][i] * inv;
-      Chunk<DT>::store(y, base + e0, v[j]);
+      for (int w = 0; w < NW; ++w) x[q] += sh[q * NW + w];
     }
   }
 }
 
-template <int DT, int NCH>
-__global__ __launch_bounds__(256) void asoftmax_bwd_reg_kernel(int64_t rows, int64_t n, const void* x,
-                                                               const void* g, void* dx, double sink,
-                                                               double eps) {
+template <int DT, int T, int NCH>
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int64_t rows, int n, const void* x,
+                                                                            void* y, float sink, float eps) {
+#pragma clang fp contract(off)
+  using R = RowChunk<DT>;
+  constexpr int RPB = T < 256 ? 256 / T : 1;  // rows per workgroup
+  __shared__ float sh[T > 64 ? T / 64 : 1];
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / T;
+  if (row >= rows) return;  // whole waves, and only where no barrier follows
+  const int tid = threadIdx.x % T;
+  const char* xr = (const char*)x + row * n * R::ESZ;
+  char* yr = (char*)y + row * n * R::ESZ;
+  const int lead = R::lead(xr), nch = R::count(n, lead);
+  u32x4_t raw[NCH];
+  float v[NCH][R::EPC];
+  float ss[1] = {0.f};
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    const int c = tid + T * j;
+    raw[j] = u32x4_t{0u, 0u, 0u, 0u};
+    if (c < nch) raw[j] = R::load(xr, c * R::EPC - lead, n);
+  }
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    R::unpack(raw[j], v[j]);
+#pragma unroll
+    for (int i = 0; i < R::EPC; ++i) ss[0] += v[j][i] * v[j][i];
+  }
+  row_sum<T, 1>(ss, sh);
+  const float tau = inv_sqrt(ss[0] * (1.f / (float)n) + eps);
+  float ks[1] = {0.f};
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    if (tid + T * j < nch) {
+#pragma unroll
+      for (int i = 0; i < R::EPC; ++i) {
+        float r;
+        v[j][i] = octic_hw(v[j][i] * tau, r);
+        ks[0] += v[j][i];
+      }
+    }
+  }
+  row_sum<T, 1>(ks, sh);
+  const float inv = 1.0f / (ks[0] - (float)(nch * R::EPC - n) + sink);
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    const int c = tid + T * j;
+    if (c < nch) {
+#pragma unroll
+      for (int i = 0; i < R::EPC; ++i) v[j][i] = v[j][i] * inv;
+      R::store(yr, c * R::EPC - lead, n, R::pack(v[j]));
+    }
+  }
+}
+
+template <int DT, int T, int NCH>
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int64_t rows, int n, const void* x,
+                                                                            const void* g, void* dx, float sink,
+                                                                            float eps) {
 #pragma clang fp contract(off)
   // The row's x and g stay in registers as their raw 16-byte chunks and are unpacked where used;
   // one float per element, w = 8 r rho^8, carries the octic between passes.  sum(p g) is taken
-  // as sum(rho^8 g) / (sum rho^8 + sink) in the pass that forms sum rho^8, so three wave
-  // reductions serve the row, and the kernel holds few enough registers for six or more waves
-  // per SIMD to keep loads in flight.
-  constexpr int EPC = Chunk<DT>::EPC;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
+  // as sum(rho^8 g) / (sum rho^8 + sink) in the pass that forms sum rho^8, so three row
+  // reductions serve the row, and the kernel holds few enough registers for several waves per SIMD
+  // to keep loads in flight.
+  using R = RowChunk<DT>;
+  constexpr int RPB = T < 256 ? 256 / T : 1;
+  __shared__ float sh[T > 64 ? 2 * (T / 64) : 1];
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / T;
   if (row >= rows) return;
-  const int64_t base = row * n;
+  const int tid = threadIdx.x % T;
+  const char* xr = (const char*)x + row * n * R::ESZ;
+  const char* gr = (const char*)g + row * n * R::ESZ;
+  char* dr = (char*)dx + row * n * R::ESZ;
+  const int lead = R::lead(xr), nch = R::count(n, lead);
   const float inv_n = 1.f / (float)n;
-  const int esz = DT == AFA_F32 ? 4 : 2;
-  u32x4_t xr[NCH], gr[NCH];
-  float w[NCH][8];
-  auto unpack = [&](const u32x4_t& c, float (&v)[8]) {
-    if constexpr (DT == AFA_F32) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const unsigned u = c[i];
-        v[i] = __builtin_bit_cast(float, u);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = Elem<DT>::lo(c[i]);
-        v[2 * i + 1] = Elem<DT>::hi(c[i]);
-      }
-    }
-  };
-  float ss = 0.f;
+  u32x4_t xw[NCH], gw[NCH];
+  float w[NCH][R::EPC];
+  float ss[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    const int64_t e0 = (int64_t)(lane + 64 * j) * EPC;
-    if (e0 < n) {
-      xr[j] = *(const u32x4_t*)((const char*)x + (base + e0) * esz);
-      gr[j] = *(const u32x4_t*)((const char*)g + (base + e0) * esz);
-      float z[8];
-      unpack(xr[j], z);
-#pragma unroll
-      for (int i = 0; i < EPC; ++i) ss += z[i] * z[i];
+    const int c = tid + T * j;
+    xw[j] = gw[j] = u32x4_t{0u, 0u, 0u, 0u};
+    if (c < nch) {
+      xw[j] = R::load(xr, c * R::EPC - lead, n);
+      gw[j] = R::load(gr, c * R::EPC - lead, n);
     }
   }
-  ss = wave_sum(ss);
-  const float tau = inv_sqrt(ss * inv_n + (float)eps);
-  float ks = 0.f, pg = 0.f;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if ((int64_t)(lane + 64 * j) * EPC < n) {
-      float z[8], gv[8];
-      unpack(xr[j], z);
-      unpack(gr[j], gv);
+    float z[R::EPC];
+    R::unpack(xw[j], z);
 #pragma unroll
-      for (int i = 0; i < EPC; ++i) {
+    for (int i = 0; i < R::EPC; ++i) ss[0] += z[i] * z[i];
+  }
+  row_sum<T, 1>(ss, sh);
+  const float tau = inv_sqrt(ss[0] * inv_n + eps);
+  float kp[2] = {0.f, 0.f};  // sum rho^8, sum rho^8 g
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    if (tid + T * j < nch) {
+      float z[R::EPC], gv[R::EPC];
+      R::unpack(xw[j], z);
+      R::unpack(gw[j], gv);
+#pragma unroll
+      for (int i = 0; i < R::EPC; ++i) {
         float r;
         const float p = octic_hw(z[i] * tau, r);
-        ks += p;
-        pg += p * gv[i];
+        kp[0] += p;
+        kp[1] += p * gv[i];
         w[j][i] = 8.f * r * p;
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // one chunk's unpacked values live at a time
   }
-  ks = wave_sum(ks);
-  pg = wave_sum(pg);
-  const float inv = 1.0f / (ks + (float)sink);
-  const float dot = pg * inv;
-  float rad = 0.f;
+  row_sum<T, 2>(kp, sh);
+  const float inv = 1.0f / (kp[0] - (float)(nch * R::EPC - n) + sink);
+  const float dot = kp[1] * inv;
+  float rad[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if ((int64_t)(lane + 64 * j) * EPC < n) {
-      float z[8], gv[8];
-      unpack(xr[j], z);
-      unpack(gr[j], gv);
+    if (tid + T * j < nch) {
+      float z[R::EPC], gv[R::EPC];
+      R::unpack(xw[j], z);
+      R::unpack(gw[j], gv);
 #pragma unroll
-      for (int i = 0; i < EPC; ++i) {
+      for (int i = 0; i < R::EPC; ++i) {
         w[j][i] = w[j][i] * inv * (gv[i] - dot);  // ng
-        rad += w[j][i] * (z[i] * tau);
+        rad[0] += w[j][i] * (z[i] * tau);  // z = 0 outside the row
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  rad = wave_sum(rad) * inv_n;
+  row_sum<T, 1>(rad, sh);
+  rad[0] *= inv_n;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    const int64_t e0 = (int64_t)(lane + 64 * j) * EPC;
-    if (e0 < n) {
-      float z[8];
-      unpack(xr[j], z);
+    const int c = tid + T * j;
+    if (c < nch) {
+      float z[R::EPC];
+      R::unpack(xw[j], z);
 #pragma unroll
-      for (int i = 0; i < EPC; ++i) w[j][i] = tau * (w[j][i] - rad * (z[i] * tau));
-      Chunk<DT>::store(dx, base + e0, w[j]);
+      for (int i = 0; i < R::EPC; ++i) w[j][i] = tau * (w[j][i] - rad[0] * (z[i] * tau));
+      R::store(dr, c * R::EPC - lead, n, R::pack(w[j]));
     }
   }
 }
 
-// Chunks per lane for the register kernels (0 = the row does not fit: use the multi-pass kernel).
-static int reg_chunks(int dtype, int64_t n, const void* a, const void* b, const void* c, int max_nch) {
-  if (dtype == AFA_F64) return 0;
-  const int epc = dtype == AFA_F32 ? 4 : 8;
-  const int esz = dtype == AFA_F32 ? 4 : 2;
-  if (n % epc != 0) return 0;
-  for (const void* p : {a, b, c})
-    if (p != nullptr && ((uintptr_t)p & 15u) != 0) return 0;
-  if (((n * esz) & 15) != 0) return 0;
-  for (int nch = 1; nch <= max_nch; nch *= 2)
-    if (n <= (int64_t)64 * epc * nch) return nch;
-  return 0;
+// The rows of all tensors start at the same offset from a 16-byte boundary (the chunks of one are the
+// chunks of the others).
+static bool same_lead(const void* a, const void* b, const void* c) {
+  return ((((uintptr_t)a ^ (uintptr_t)b) | (c != nullptr ? (uintptr_t)a ^ (uintptr_t)c : 0)) & 15u) == 0;
 }
 
 #define AFA_DISPATCH_DT(dtype, FN, ...)            \
@@ -439,56 +421,78 @@ static void oc_bwd(int64_t n, const void* x, const void* g, void* dx, hipStream_
   hipLaunchKernelGGL((octic_bwd_kernel<DT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, x, g, dx);
 }
 
-template <int DT, int NCH>
-static void sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
-  hipLaunchKernelGGL((asoftmax_fwd_reg_kernel<DT, NCH>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, rows, n, x, y, sink, eps);
+// Chunks that cover any row: rows of whole chunks all start where the first one does.
+template <int DT>
+static int row_chunks(int64_t n, const void* x) {
+  using R = RowChunk<DT>;
+  return n % R::EPC == 0 ? R::count((int)n, (int)((uintptr_t)x & 15u) / R::ESZ) : R::count_max((int)n);
 }
-template <int DT, int NCH>
-static void sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, void* dx, double sink, double eps,
+
+// Threads per row and chunks per thread by the row's chunk count: the fewest threads that hold the row
+// in at most four chunks each (the VJP's x, g and 8 r rho^8 take 12 or 16 registers a chunk: six
+// chunks a lane leave one wave per SIMD, and (18372, 1531) fp32 took 173 us instead of 80).  false: no
+// variant holds the row, or a launch would pass 2^32 threads (the multi-pass kernels take 64 per row).
+static bool sm_reg_fits(int64_t rows, int nch) { return nch <= 4096 && (nch <= 256 || rows < (1 << 22)); }
+#define AFA_SM_GO(KERNEL, T, NCH, ...)                                                                       \
+  hipLaunchKernelGGL((KERNEL<DT, T, NCH>), dim3((unsigned)((rows * T + (T < 256 ? 255 : T - 1)) /            \
+                     (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, rows, (int)n, __VA_ARGS__)
+template <int DT>
+static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
+  if (n > (1 << 20) || !same_lead(x, y, nullptr)) return false;
+  const int nch = row_chunks<DT>(n, x);
+  if (!sm_reg_fits(rows, nch)) return false;
+#define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_fwd_reg_kernel, T, NCH, x, y, (float)sink, (float)eps)
+  if (nch <= 64) AFA_SM(64, 1);
+  else if (nch <= 128) AFA_SM(64, 2);
+  else if (nch <= 192) AFA_SM(64, 3);
+  else if (nch <= 256) AFA_SM(64, 4);
+  else if (nch <= 512) AFA_SM(256, 2);
+  else if (nch <= 768) AFA_SM(256, 3);
+  else if (nch <= 1024) AFA_SM(256, 4);
+  else if (nch <= 1536) AFA_SM(512, 3);
+  else if (nch <= 2048) AFA_SM(512, 4);
+  else AFA_SM(1024, 4);
+#undef AFA_SM
+  return true;
+}
+template <int DT>
+static bool sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, void* dx, double sink, double eps,
                        hipStream_t st) {
-  hipLaunchKernelGGL((asoftmax_bwd_reg_kernel<DT, NCH>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, rows, n, x, g, dx, sink, eps);
+  if (n > (1 << 20) || !same_lead(x, g, dx)) return false;
+  const int nch = row_chunks<DT>(n, x);
+  if (!sm_reg_fits(rows, nch)) return false;
+#define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_bwd_reg_kernel, T, NCH, x, g, dx, (float)sink, (float)eps)
+  if (nch <= 64) AFA_SM(64, 1);
+  else if (nch <= 128) AFA_SM(64, 2);
+  else if (nch <= 192) AFA_SM(64, 3);
+  else if (nch <= 256) AFA_SM(64, 4);
+  else if (nch <= 512) AFA_SM(256, 2);
+  else if (nch <= 768) AFA_SM(256, 3);
+  else if (nch <= 1024) AFA_SM(256, 4);
+  else if (nch <= 1536) AFA_SM(512, 3);
+  else if (nch <= 2048) AFA_SM(512, 4);
+  else AFA_SM(1024, 4);
+#undef AFA_SM
+  return true;
 }
-template <int DT>
-static void sm_fwd_reg_dt(int nch, int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
-  switch (nch) {
-    case 1: sm_fwd_reg<DT, 1>(rows, n, x, y, sink, eps, st); break;
-    case 2: sm_fwd_reg<DT, 2>(rows, n, x, y, sink, eps, st); break;
-    case 4: sm_fwd_reg<DT, 4>(rows, n, x, y, sink, eps, st); break;
-    default: sm_fwd_reg<DT, 8>(rows, n, x, y, sink, eps, st); break;
-  }
-}
-template <int DT>
-static void sm_bwd_reg_dt(int nch, int64_t rows, int64_t n, const void* x, const void* g, void* dx, double sink,
-                          double eps, hipStream_t st) {
-  switch (nch) {
-    case 1: sm_bwd_reg<DT, 1>(rows, n, x, g, dx, sink, eps, st); break;
-    case 2: sm_bwd_reg<DT, 2>(rows, n, x, g, dx, sink, eps, st); break;
-    default: sm_bwd_reg<DT, 4>(rows, n, x, g, dx, sink, eps, st); break;
-  }
-}
+#undef AFA_SM_GO
 
 hipError_t asoftmax_fwd_launch(int dtype, int64_t rows, int64_t n, const void* x, void* y, double sink,
                                double eps, hipStream_t st) {
-  const int nch = reg_chunks(dtype, n, x, y, nullptr, 8);
-  if (nch > 0) {
-    if (dtype == AFA_F32) sm_fwd_reg_dt<AFA_F32>(nch, rows, n, x, y, sink, eps, st);
-    else if (dtype == AFA_BF16) sm_fwd_reg_dt<AFA_BF16>(nch, rows, n, x, y, sink, eps, st);
-    else sm_fwd_reg_dt<AFA_F16>(nch, rows, n, x, y, sink, eps, st);
-    return hipGetLastError();
-  }
-  AFA_DISPATCH_DT(dtype, sm_fwd, rows, n, x, y, sink, eps, st);
+  const bool done = dtype == AFA_F32    ? sm_fwd_reg<AFA_F32>(rows, n, x, y, sink, eps, st)
+                    : dtype == AFA_BF16 ? sm_fwd_reg<AFA_BF16>(rows, n, x, y, sink, eps, st)
+                    : dtype == AFA_F16  ? sm_fwd_reg<AFA_F16>(rows, n, x, y, sink, eps, st)
+                                        : false;
+  if (!done) AFA_DISPATCH_DT(dtype, sm_fwd, rows, n, x, y, sink, eps, st);
   return hipGetLastError();
 }
 hipError_t asoftmax_bwd_launch(int dtype, int64_t rows, int64_t n, const void* x, const void* g,
                                void* dx, double sink, double eps, hipStream_t st) {
-  const int nch = reg_chunks(dtype, n, x, g, dx, 4);
-  if (nch > 0) {
-    if (dtype == AFA_F32) sm_bwd_reg_dt<AFA_F32>(nch, rows, n, x, g, dx, sink, eps, st);
-    else if (dtype == AFA_BF16) sm_bwd_reg_dt<AFA_BF16>(nch, rows, n, x, g, dx, sink, eps, st);
-    else sm_bwd_reg_dt<AFA_F16>(nch, rows, n, x, g, dx, sink, eps, st);
-    return hipGetLastError();
-  }
-  AFA_DISPATCH_DT(dtype, sm_bwd, rows, n, x, g, dx, sink, eps, st);
+  const bool done = dtype == AFA_F32    ? sm_bwd_reg<AFA_F32>(rows, n, x, g, dx, sink, eps, st)
+                    : dtype == AFA_BF16 ? sm_bwd_reg<AFA_BF16>(rows, n, x, g, dx, sink, eps, st)
+                    : dtype == AFA_F16  ? sm_bwd_reg<AFA_F16>(rows, n, x, g, dx, sink, eps, st)
+                                        : false;
+  if (!done) AFA_DISPATCH_DT(dtype, sm_bwd, rows, n, x, g, dx, sink, eps, st);
   return hipGetLastError();
 }
 hipError_t octic_fwd_launch(int dtype, int64_t n, const void* x, void* y, hipStream_t st) {

@@ -630,3 +630,29 @@ def test_rotation_of_q_and_k_in_one_launch(dt, table_dt, shape, axis, off):
     qr, kr = A.apply_ago_rotations(qi, ki, (c, s), seq_axis=axis)
     (only,) = torch.autograd.grad(kr, ki, gk)  # q's output unused
     assert torch.equal(only, want(gk, -1))
+
+
+@pytest.mark.parametrize("dt,epc,tol", [(torch.float32, 4, 2e-5), (torch.bfloat16, 8, 1.6e-2), (torch.float16, 8, 4e-3)])
+@pytest.mark.parametrize("chunks", [0, 1, 64, 128, 192, 256, 512, 768, 1024, 1536, 2048, 4096])
+def test_algebraic_softmax_row_kernels(dt, epc, tol, chunks):
+    """Rows at each limit of the register-resident kernels, whose odd lengths start every row at
+    another offset from a 16-byte boundary, from an aligned base and from one an element past it (its
+    output, allocated aligned, then takes the multi-pass kernel), against the fp64 kernel;
+    tolerances as the tests of the same kernels above."""
+    for n in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1}):
+        gen = torch.Generator(device=DEV).manual_seed(n)
+        for off in (0, 1):
+            rows = 5
+            flat = torch.empty(rows * n + off, dtype=dt, device=DEV)[off:]
+            flat.copy_(torch.randn(rows * n, generator=gen, device=DEV) * 3)
+            x = flat.view(rows, n).requires_grad_(True)
+            g = torch.randn((rows, n), generator=gen, device=DEV).to(dt)
+            y = A.algebraic_softmax(x)
+            (dx,) = torch.autograd.grad(y, x, g)
+            xd = x.detach().double().requires_grad_(True)
+            yd = A.algebraic_softmax(xd)
+            (dd,) = torch.autograd.grad(yd, xd, g.double())
+            assert normwise(to_f64(y), to_f64(yd)) <= tol, (n, off)
+            # at n = 1 the gradient is 0 but for eps: the size of its terms, p g, stands in
+            scale = max(float(dd.abs().max()), 1e-3 * float((yd * g).abs().max()))
+            assert float((dx.double() - dd).abs().max()) <= tol * scale, (n, off)
