@@ -182,7 +182,7 @@ static hipError_t ago_rotate_go(const RotateArgs& a, hipStream_t st) {
     const int64_t slice = a.seq * a.inner * (a.dim / EPC), gx = (slice + 255) / 256;
     const int64_t blocks = gx * ((a.outer + ROT_OUTER - 1) / ROT_OUTER);
     const uintptr_t ptrs = (uintptr_t)a.xa | (uintptr_t)a.ya | (uintptr_t)a.xb | (uintptr_t)a.yb;
-    if (a.dim % EPC == 0 && (ptrs & 15u) == 0 && slice < (int64_t(1) << 31) && blocks < (int64_t(1) << 31)) {
+    if (a.dim % EPC == 0 && (ptrs & 15u) == 0 && slice < (int64_t(1) << 31) && blocks < (int64_t(1) << 24)) {
       hipLaunchKernelGGL((ago_rotate_vec_kernel<DT, TD>), dim3((unsigned)blocks, tensors), dim3(256), 0, st,
                          (uint32_t)slice, a.outer, (uint32_t)(a.inner * (a.dim / EPC)), (uint32_t)(a.dim / EPC),
                          (uint32_t)gx, a.xa, a.xb, a.ya, a.yb, a.rc, a.rs, a.sign);

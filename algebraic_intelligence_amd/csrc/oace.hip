@@ -466,7 +466,8 @@ void rows_fwd_vec(const OaceArgs& a, const void* z, int64_t ldz, void* rows, hip
   hipLaunchKernelGGL((oace_rows_fwd_vec_kernel<DT, T, NCH>), dim3((unsigned)((a.N * T + (T < 256 ? 255 : T - 1)) /  \
                      (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, z, ldz, a.N, (int)a.V, a.targets,       \
                      (float)a.eps, (float)a.gamma, inv_v, (float*)rows)
-  if (nch <= 64) OACE_ROWS_VEC(64, 1);
+  if (a.N >= (1 << 23)) OACE_ROWS_VEC(64, 0);  // 512 threads per row would pass 2^32 in one launch
+  else if (nch <= 64) OACE_ROWS_VEC(64, 1);
   else if (nch <= 128) OACE_ROWS_VEC(64, 2);
   else if (nch <= 256) OACE_ROWS_VEC(64, 4);
   else if (nch <= 512) OACE_ROWS_VEC(256, 2);
@@ -489,6 +490,7 @@ bool rows_bwd_vec(const OaceArgs& a, const void* rows, void* dz, float c0, hipSt
   // four chunks per lane when that still leaves four waves per SIMD, else one
   const bool wide = a.N * ((nch + 255) / 256) >= 4096;
   const int64_t waves = a.N * (int64_t)((nch + (wide ? 255 : 63)) / (wide ? 256 : 64));
+  if (waves >= (int64_t(1) << 26)) return false;  // 2^32 threads
   const dim3 grid((unsigned)((waves + 3) / 4));
   if (wide)
     hipLaunchKernelGGL((oace_rows_bwd_vec_kernel<DT, 4>), grid, dim3(256), 0, st, a.h, a.ldh, a.N, (int)a.V, a.targets,
