@@ -6,13 +6,12 @@
 //   ds = 8 scale r w (g_i . v_j - E_i);  dq_i += ds_ij k_j;  dk_j += ds_ij q_i;  dv_j += w_ij g_i,
 // with ds and w rounded to the input dtype as MFMA operands and fp32 accumulation.
 //
-// Three launches after the pre-passes of q and k (rotation with rotary tables, the fast-rho
-// guard's block bounds), no atomics:
-//   * rotary tables only: q and k rotated once into scratch by the forward's K rotation pass
-//     (afa_krot_kernel, which also writes the fast-rho guard's block bounds of the rotated rows),
-//     or by afa_bwd_mfma_rotate_kernel where no bounds are needed or at head_dim 256; dq and dk
-//     are rotated back through R^T in the dQ / dK store epilogues;
-//   * afa_bwd_mfma_prep_kernel: -E_i and 1/d_i per row into the workspace;
+// Three launches, no atomics:
+//   * afa_bwd_mfma_pre_kernel: with rotary tables q and k rotated once into scratch, the fast-rho
+//     guard's block bounds of the (rotated) rows, and -E_i and 1/d_i per row into the workspace;
+//     where no bounds are needed or at head_dim 256 these are afa_bwd_mfma_rotate_kernel,
+//     afa_rownorm_kernel and afa_bwd_mfma_prep_kernel.  dq and dk are rotated back through R^T in
+//     the dQ / dK store epilogues;
 //   * afa_bwd_mfma_dq_kernel (one lane per query, like the forward): S^T = K Q^T, dP^T = V g^T on
 //     MFMA, W and dS on the VALU, dQ^T += K^T dS^T with K^T read from the same LDS tile by
 //     ds_read_tr16_b64;
@@ -252,9 +251,9 @@ __host__ __device__ constexpr int ws_rows(int L) { return (L + 3) & ~3; }
 // padding rows hold zeros.  E is stored negated because the dK/dV kernel starts its dP
 // accumulators from it (dP - E out of the MFMA) and the dQ kernel adds it in an fma.
 template <int DT>
-__global__ __launch_bounds__(256) void afa_bwd_mfma_prep_kernel(const GenArgs a) {
+__device__ __forceinline__ void bwd_prep_rows(const GenArgs& a, int block) {
   const int LP = ws_rows(a.L);
-  const int64_t prow = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);  // workspace row
+  const int64_t prow = (int64_t)block * 32 + (threadIdx.x >> 3);  // workspace row
   const int64_t prows = (int64_t)a.B * a.H * LP;
   const int64_t bh = prow / LP;
   const int l = (int)(prow - bh * LP);
@@ -280,6 +279,80 @@ __global__ __launch_bounds__(256) void afa_bwd_mfma_prep_kernel(const GenArgs a)
     ((float*)a.e_ws)[prow] = live ? -part : 0.f;
     ((float*)a.e_ws)[prows + prow] = live ? 1.0f / ((const float*)a.dtot)[row] : 0.f;
   }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void afa_bwd_mfma_prep_kernel(const GenArgs a) {
+  bwd_prep_rows<DT>(a, (int)blockIdx.x);
+}
+
+// The backward's whole pre-pass in one launch: blocks [0, nrb) take q's 64-row blocks, [nrb, 2 nrb)
+// k's, the rest E and 1/d.  A wave reads one 64-row block (RowBlockLayout; four row iterations in
+// flight), rotates it into contiguous scratch when ROT (fp32, one rounding: afa_krot_kernel's
+// values), and writes the largest squared norm of its rows as the matrix kernels will read them: the
+// fast-rho guard's bounds.  HBM bound; three launches of a few microseconds each before, whose ramps
+// and gaps were most of their time on short sequences (B=16 H=6 L=512 D=48 rotary backward 62.9 -> 53.0 us, B=32 H=8 L=145 D=128 75.8 -> 62.6 us).
+template <int DT, int D, bool ROT>
+__global__ __launch_bounds__(256) void afa_bwd_mfma_pre_kernel(const GenArgs a, unsigned short* qr, unsigned short* kr,
+                                                               int nblk, int nwork, int nrb) {
+#pragma clang fp contract(off)
+  using RL = RowBlockLayout<D>;
+  int block = (int)blockIdx.x;
+  if (block >= 2 * nrb) {
+    bwd_prep_rows<DT>(a, block - 2 * nrb);
+    return;
+  }
+  const bool second = block >= nrb;
+  if (second) block -= nrb;
+  const int lane = threadIdx.x & 63;
+  const int w = block * 4 + (int)(threadIdx.x >> 6);  // wave-uniform work item
+  if (w >= nwork) return;
+  const int bh = w / nblk, blk = w - bh * nblk;
+  const unsigned short* x = (const unsigned short*)(second ? a.k : a.q) + (int64_t)bh * a.L * D;
+  unsigned short* y = (second ? kr : qr) + (int64_t)bh * a.L * D;
+  const float* rc = (const float*)a.rc;
+  const float* rs = (const float*)a.rs;
+  const int c = lane % RL::CHP, rsub = lane / RL::CHP;
+  constexpr int G = RL::CHP < 4 ? RL::CHP : 4;
+  float m = 0.0f;
+#pragma unroll
+  for (int g = 0; g < RL::CHP; g += G) {
+    u32x4_t wv[G];
+    f32x4_t cc[G], ss[G];
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int l = blk * 64 + (g + i) * RL::RPI + rsub;
+      wv[i] = u32x4_t{0u, 0u, 0u, 0u};
+      if (c < RL::CH && l < a.L) {
+        wv[i] = *(const u32x4_t*)(x + (int64_t)l * D + c * 8);
+        if constexpr (ROT) {
+          cc[i] = *(const f32x4_t*)(rc + (int64_t)l * (D / 2) + c * 4);
+          ss[i] = *(const f32x4_t*)(rs + (int64_t)l * (D / 2) + c * 4);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int l = blk * 64 + (g + i) * RL::RPI + rsub;
+      float n2 = 0.0f;
+      if (c < RL::CH && l < a.L) {
+        if constexpr (ROT) {
+          u32x4_t r;
+#pragma unroll
+          for (int p = 0; p < 4; ++p) {
+            const float x0 = Elem<DT>::lo(wv[i][p]), x1 = Elem<DT>::hi(wv[i][p]);
+            r[p] = Elem<DT>::pack(cc[i][p] * x0 - ss[i][p] * x1, ss[i][p] * x0 + cc[i][p] * x1);
+          }
+          *(u32x4_t*)(y + (int64_t)l * D + c * 8) = r;
+          wv[i] = r;
+        }
+        n2 = chunk_norm2<DT>(wv[i]);
+      }
+      m = __builtin_fmaxf(m, group_sum<RL::CHP>(n2));
+    }
+  }
+  m = wave_max(m);
+  if (lane == 0) ((float*)(second ? a.kbm : a.qbm))[(int64_t)bh * nblk + blk] = m;
 }
 
 // Cayley rotation of q (blockIdx.y = 0) and k (blockIdx.y = 1) into contiguous scratch: each
@@ -1122,59 +1195,49 @@ template <int DT, int D, bool EXACT>
 static hipError_t bwd_launch(GenArgs a, void* rot_scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a.B * a.H * a.L;
   const bool guard = !EXACT && a.qbm != nullptr && a.kbm != nullptr;
-  const int64_t sl = a.D, sh = (int64_t)a.L * a.D, sb = (int64_t)a.H * sh;  // q, k: contiguous
-  bool bounded = false;  // the guard's bounds already written by the rotation
-  if (a.rc != nullptr) {
-    if (rot_scratch == nullptr) return hipErrorInvalidValue;
-    unsigned short* qr = (unsigned short*)rot_scratch;
-    unsigned short* kr = qr + rows * D;
-    if (guard && D <= 128) {
-      // the forward's K rotation pass (afa_krot_kernel), once for q and once for k: the same fp32
-      // rotation and rounding as afa_bwd_mfma_rotate_kernel, and each 64-row block's largest
-      // squared norm from the rotated rows as they are written, in place of a second pass
-      FwdArgs f = {};
-      f.B = a.B;
-      f.H = a.H;
-      f.L = a.L;
-      f.rc = (const float*)a.rc;
-      f.rs = (const float*)a.rs;
-      f.k = a.q;
-      f.k_b = sb;
-      f.k_h = sh;
-      f.k_l = sl;
-      hipError_t e = krot_launch(DT, D, f, qr, (float*)a.qbm, st);
-      f.k = a.k;
-      f.k_b = sb;
-      f.k_h = sh;
-      f.k_l = sl;
-      if (e == hipSuccess) e = krot_launch(DT, D, f, kr, (float*)a.kbm, st);
-      if (e != hipSuccess) return e;
-      bounded = true;
-    } else {
-      const int64_t chunks = rows * (D / 8);
-      const unsigned gx = (unsigned)std::min<int64_t>((chunks + 255) / 256, 4096);
-      hipLaunchKernelGGL((afa_bwd_mfma_rotate_kernel<DT, D>), dim3(gx, 2), dim3(256), 0, st, a, qr, kr);
-    }
-    a.q = qr;
-    a.k = kr;
-  }
+  if (a.rc != nullptr && rot_scratch == nullptr) return hipErrorInvalidValue;
+  unsigned short* qr = (unsigned short*)rot_scratch;
+  unsigned short* kr = qr + (a.rc != nullptr ? rows * D : 0);
+  const int64_t prows = (int64_t)a.B * a.H * ws_rows(a.L);
+  const unsigned prep_blocks = (unsigned)((prows + 31) / 32);
   if (guard) {
-    // fast-rho guard bounds of the (rotated) q and k rows; without them every tile is exact
-    hipError_t e = hipSuccess;
-    if (!bounded) {
-      e = rownorm_launch(DT, a.q, sb, sh, sl, a.B, a.H, a.L, a.D, (float*)a.qbm, st);
-      if (e == hipSuccess) e = rownorm_launch(DT, a.k, sb, sh, sl, a.B, a.H, a.L, a.D, (float*)a.kbm, st);
-    }
-    if (e != hipSuccess) return e;
     a.nkb = (a.L + 63) / 64;
     // dQ forms s = S * score_factor with q / 8 and k as stored (dK/dV: q and k / 8); the half
     // form forms x = s / sqrt 2 from q / 16 (k / 16)
     a.nb_lim = fast_rho_lim(D == 64 ? 1.0 : half_form<DT, D>() ? 1.4142135623730951 : D == 128 ? 0.70710677 : 8.0 * a.scale);
-  } else {
-    a.qbm = a.kbm = nullptr;
   }
-  const int64_t prows = (int64_t)a.B * a.H * ws_rows(a.L);
-  hipLaunchKernelGGL((afa_bwd_mfma_prep_kernel<DT>), dim3((unsigned)((prows + 31) / 32)), dim3(256), 0, st, a);
+  bool prepped = false;
+  if constexpr (D <= 128) {
+    if (guard) {
+      const int nwork = a.B * a.H * a.nkb, nrb = (nwork + 3) / 4;
+      const dim3 grid(2u * (unsigned)nrb + prep_blocks);
+      if (a.rc != nullptr)
+        hipLaunchKernelGGL((afa_bwd_mfma_pre_kernel<DT, D, true>), grid, dim3(256), 0, st, a, qr, kr, a.nkb, nwork, nrb);
+      else
+        hipLaunchKernelGGL((afa_bwd_mfma_pre_kernel<DT, D, false>), grid, dim3(256), 0, st, a, qr, kr, a.nkb, nwork, nrb);
+      prepped = true;
+    }
+  }
+  if (!prepped && a.rc != nullptr) {
+    const int64_t chunks = rows * (D / 8);
+    const unsigned gx = (unsigned)std::min<int64_t>((chunks + 255) / 256, 4096);
+    hipLaunchKernelGGL((afa_bwd_mfma_rotate_kernel<DT, D>), dim3(gx, 2), dim3(256), 0, st, a, qr, kr);
+  }
+  if (a.rc != nullptr) {
+    a.q = qr;
+    a.k = kr;
+  }
+  if (!prepped) {
+    if (guard) {
+      // fast-rho guard bounds of the (rotated) q and k rows; without them every tile is exact
+      const int64_t sl = a.D, sh = (int64_t)a.L * a.D, sb = (int64_t)a.H * sh;  // contiguous
+      hipError_t e = rownorm_launch(DT, a.q, sb, sh, sl, a.B, a.H, a.L, a.D, (float*)a.qbm, st);
+      if (e == hipSuccess) e = rownorm_launch(DT, a.k, sb, sh, sl, a.B, a.H, a.L, a.D, (float*)a.kbm, st);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((afa_bwd_mfma_prep_kernel<DT>), dim3(prep_blocks), dim3(256), 0, st, a);
+  }
+  if (!guard) a.qbm = a.kbm = nullptr;
   const int nb = a.B * a.H * ((a.L + 127) / 128);
   hipLaunchKernelGGL((afa_bwd_mfma_dq_kernel<DT, D, EXACT>), dim3(nb), dim3(256), 0, st, a);
   hipLaunchKernelGGL((afa_bwd_mfma_dkdv_kernel<DT, D, EXACT>), dim3(nb), dim3(256), 0, st, a);
