@@ -241,7 +241,7 @@ struct OaceGemm {
 };
 bool oace_gemm_fits(const OaceGemm& g);
 // Contraction parts for about `wgs` workgroups (1: no split); parts > 1 need part_bytes of fp32
-// partials, added in part order by a second kernel (row-contiguous A, contiguous B only).
+// partials, added in part order by a second kernel (row-contiguous A only).
 int oace_gemm_parts(const OaceGemm& g, int wgs);
 size_t oace_gemm_part_bytes(const OaceGemm& g, int parts);
 hipError_t oace_gemm(int dtype, const OaceGemm& g, int parts, float* part, hipStream_t st);

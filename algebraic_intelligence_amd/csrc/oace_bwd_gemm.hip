@@ -1,7 +1,8 @@
 // Hand-written MFMA GEMMs of the fused Linear + OACE backward (src/kernels/pallas_oace.py:212-269):
 //   dh = dz W^T  (rows x d_model; the contraction runs over the whole vocabulary, so it is split
 //                 into parts whose fp32 partials a second kernel adds in part order)
-//   dW = h^T dz  (d_model x vocab in W's layout; the contraction runs over the rows)
+//   dW = h^T dz  (d_model x vocab in W's layout; the contraction runs over the rows, split likewise
+//                 when the tiles are few)
 // for bf16 / fp16 operands with fp32 accumulation, each result rounded once to the element type.
 //
 // One kernel template: D[n][m] = sum_k A[m][k] B[n][k] over 256 (m) x 128 WN (n) tiles, waves
@@ -466,6 +467,10 @@ __global__ __launch_bounds__(256) void oace_bwd_gemm_sum_kernel(const f32x4_t* p
   }
   for (; p < parts; ++p) s += part[p * per_part + i];
   unsigned short* o = out + (int64_t)n * ldo + m;
+  if (m + 4 <= M && ((uintptr_t)o & 7u) == 0) {
+    *(u32x2_t*)o = u32x2_t{Elem<DT>::pack(s[0], s[1]), Elem<DT>::pack(s[2], s[3])};
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < 4; ++u)
     if (m + u < M) Elem<DT>::store(o, u, s[u]);
@@ -499,8 +504,9 @@ hipError_t bg_launch(const BgArgs& g, hipStream_t st) {
 template <int DT, int WN>
 hipError_t bg_run(const OaceGemm& g, BgArgs& b, hipStream_t st) {
   if (b.parts > 1) {
-    if (!g.a_mc || g.b_mc) return hipErrorNotSupported;
-    hipError_t e = bg_launch<DT, true, false, OUT_PART, WN>(b, st);
+    if (!g.a_mc) return hipErrorNotSupported;
+    hipError_t e = g.b_mc ? bg_launch<DT, true, true, OUT_PART, WN>(b, st)
+                          : bg_launch<DT, true, false, OUT_PART, WN>(b, st);
     if (e != hipSuccess) return e;
     const int64_t threads = (int64_t)b.mt * b.nt * Cfg<WN>::NW * 32 * 64;
     hipLaunchKernelGGL((oace_bwd_gemm_sum_kernel<DT, WN>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
@@ -530,20 +536,20 @@ int oace_gemm_parts(const OaceGemm& g, int cus) {
   // rounds of workgroups over the CU slots, each as long as one tile over its share of the
   // contraction, plus writing and reading the parts' fp32 partials.  Rates: a workgroup of
   // 256 x 256 tiles (one per CU) at 6 TFLOP/s, 256 x 128 tiles (two per CU) at 3 TFLOP/s each;
-  // partials at 5 TB/s.  Parts hold at least 1024 of the contraction.  Part counts of 8 and
-  // more are multiples of 8: at N = 512 (6 tiles), 42 parts -- 32 workgroups on each XCD's 32
-  // CUs -- made dh 56.1 us against 51.4 us for 40 (30 per XCD), measured twice on one box.
+  // partials at 5 TB/s, 3 us for the second launch.  Parts hold at least 512 of the contraction.  Part
+  // counts of 8 and more are multiples of 8: at N = 512 (6 tiles), 42 parts -- 32 workgroups on each
+  // XCD's 32 CUs -- made dh 56.1 us against 51.4 us for 40 (30 per XCD), measured twice on one box.
   const int wn = wn_of(g);
   const int64_t tiles = (int64_t)tiles_m(g.m) * tiles_n(g.n, wn);
   const int64_t slots = (int64_t)cus * (wn == 1 ? Cfg<1>::CUS_SLOTS : Cfg<2>::CUS_SLOTS);
   const double t_tile = 2.0 * GM * 128.0 * wn * (double)g.k / (wn == 1 ? 3e12 : 6e12);
   const double t_part = 2.0 * (double)g.m * (double)g.n * 4.0 / 5e12;
-  const int pmax = (int)std::min<int64_t>(64, std::max<int64_t>(1, g.k / 1024));
+  const int pmax = (int)std::min<int64_t>(64, std::max<int64_t>(1, g.k / 512));
   int best = 1;
   double best_t = 0.0;
   for (int p = 1; p <= pmax; ++p) {
     const double rounds = (double)((tiles * p + slots - 1) / slots);
-    const double t = rounds * t_tile / p + (p > 1 ? p * t_part : 0.0);
+    const double t = rounds * t_tile / p + (p > 1 ? p * t_part + 3e-6 : 0.0);
     if (p >= 8 && p % 8 != 0) continue;
     if (p == 1 || t < best_t) {
       best = p;

@@ -552,13 +552,22 @@ bool z_cached(const OaceArgs& a) {
 // model features, B = dz contraction-contiguous.  Its vocabulary contraction is split for this
 // many workgroups: a constant, so that the summation order, and the result, do not depend on
 // the device.
-constexpr int DH_WGS = 256;
+constexpr int SPLIT_WGS = 256;
 OaceGemm dh_gemm(const OaceArgs& a, const unsigned short* wt, int64_t ldwt, const unsigned short* dz) {
   return OaceGemm{wt, ldwt, true, a.d, dz, ldz_of(a.V), false, a.N, a.V, a.dh, a.d};
 }
 
+// dW = h^T dz in W's layout, split over the rows when its tiles are fewer than the workgroup slots
+// (backward of 6403 x 128 x 2752, 11 tiles: 206 -> 77 us; 8000 x 992 x 1100, 20 tiles: 231 -> 81 us).
+OaceGemm dw_gemm(const OaceArgs& a, const unsigned short* dz) {
+  if (a.w_layout == OACE_W_DV)  // dW (d, V): D[k][v] = sum_n dz[n][v] h[n][k]
+    return OaceGemm{dz, ldz_of(a.V), true, a.V, a.h, a.ldh, true, a.d, a.N, a.dw, a.ldw};
+  // dW^T (V, d): D[v][k] = sum_n h[n][k] dz[n][v]
+  return OaceGemm{a.h, a.ldh, true, a.d, dz, ldz_of(a.V), true, a.V, a.N, a.dw, a.ldw};
+}
+
 struct Layout {
-  size_t wt, zc, part, dz, dhp, total;
+  size_t wt, zc, part, dz, gp, total;
 };
 Layout layout_of(const OaceArgs& a) {
   Layout l;
@@ -566,9 +575,11 @@ Layout layout_of(const OaceArgs& a) {
   l.zc = z_cached(a) ? al((size_t)a.N * ldz_of(a.V) * sizeof(float)) : 0;
   l.part = al((size_t)nvt_of(a.V) * a.N * 4 * sizeof(float));
   l.dz = al((size_t)a.N * ldz_of(a.V) * 2);
-  const OaceGemm gh = dh_gemm(a, nullptr, a.d, nullptr);
-  l.dhp = al(oace_gemm_part_bytes(gh, oace_gemm_parts(gh, DH_WGS)));  // split-K partials of dh
-  l.total = l.wt + l.zc + std::max(l.part, l.dz + l.dhp);
+  // split partials of dh, then (its sum done) of dW
+  const OaceGemm gh = dh_gemm(a, nullptr, a.d, nullptr), gw = dw_gemm(a, nullptr);
+  l.gp = al(std::max(oace_gemm_part_bytes(gh, oace_gemm_parts(gh, SPLIT_WGS)),
+                     oace_gemm_part_bytes(gw, oace_gemm_parts(gw, SPLIT_WGS))));
+  l.total = l.wt + l.zc + std::max(l.part, l.dz + l.gp);
   return l;
 }
 
@@ -701,14 +712,11 @@ hipError_t oace_linear_bwd_mfma(int dtype, const OaceArgs& a, const void* rows, 
     e = launch_gemm_dt<MODE_DZ>(dtype, g, st);
   }
   if (e != hipSuccess) return e;
+  float* parts = (float*)(sbase + l.dz);
   const OaceGemm gh = dh_gemm(a, wt, ldwt, dz);
-  if ((e = oace_gemm(dtype, gh, oace_gemm_parts(gh, DH_WGS), (float*)(sbase + l.dz), st)) != hipSuccess) return e;
-  const OaceGemm gw = a.w_layout == OACE_W_DV
-                          // dW (d, V): D[k][v] = sum_n dz[n][v] h[n][k]
-                          ? OaceGemm{dz, g.ldz, true, a.V, a.h, a.ldh, true, a.d, a.N, a.dw, a.ldw}
-                          // dW^T (V, d): D[v][k] = sum_n h[n][k] dz[n][v]
-                          : OaceGemm{a.h, a.ldh, true, a.d, dz, g.ldz, true, a.V, a.N, a.dw, a.ldw};
-  return oace_gemm(dtype, gw, 1, nullptr, st);
+  if ((e = oace_gemm(dtype, gh, oace_gemm_parts(gh, SPLIT_WGS), parts, st)) != hipSuccess) return e;
+  const OaceGemm gw = dw_gemm(a, dz);
+  return oace_gemm(dtype, gw, oace_gemm_parts(gw, SPLIT_WGS), parts, st);
 }
 
 }  // namespace afa

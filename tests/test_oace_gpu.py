@@ -356,3 +356,23 @@ def test_dw_rows_of_any_stride_and_start(tied, V, pad, off):
     assert normwise(to_f64(dh), to_f64(dh_ref)) <= 1e-6
     assert bool((mat[:, cols:] == sentinel).all()), "padding columns changed"
     assert bool((store[:off] == sentinel).all()) and bool((store[off + rows_n * ldw:] == sentinel).all())
+
+
+@pytest.mark.parametrize("dtype", LOW)
+@pytest.mark.parametrize("shape", [(2049, 32, 9), (1500, 96, 1003), (1024, 64, 257), (4100, 288, 520)])
+@pytest.mark.parametrize("tied", [False, True])
+def test_dw_split_over_the_rows(shape, dtype, tied):
+    """dW from parts of its contraction over the rows (few tiles, many rows), with ragged last parts
+    and tiles in both dimensions, against the fp64 path: the element type's rounding of dz and of
+    dW, 2e-2 normwise as the other gradients; and repeated calls bitwise equal."""
+    N, d, V = shape
+    h, w, t = _case(N, d, V, dtype, seed=N + V, scale=1.0 if dtype == torch.bfloat16 else 0.5)
+    wv = _tied(w) if tied else w
+    g = 1.0 if dtype == torch.bfloat16 else 4096.0  # fp16: dz of a mean over this many rows is small
+    _, cache = _fwd(h, wv, t)
+    dh, dw = _grads(cache, g)
+    dh2, dw2 = _grads(cache, g)
+    assert torch.equal(dh, dh2) and torch.equal(dw, dw2)
+    _, rcache = _fwd(h.double(), wv.double(), t)
+    rh, rw = _grads(rcache, g)
+    assert normwise(to_f64(dh), to_f64(rh)) <= 2e-2 and normwise(to_f64(dw), to_f64(rw)) <= 2e-2
