@@ -544,6 +544,11 @@ bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // holds -- and then evaluates the octic sums, and the backward dz, from them instead of a
 // second GEMM sweep.  Larger problems recompute z, which keeps the workspace O(rows x d_model).
 constexpr size_t ZC_MAX_BYTES = (size_t)256 << 20;
+// Rows of kept logits up to this long take the row kernels of given logits (oace_rows_z), which fit
+// their threads to the row; the 512-thread streaming kernel below, whose groups of 8192 entries mostly
+// idle on them, takes longer ones (forward of 6403 x 128 x 2752 69 -> 55 us and 4000 x 992 x 1408 58 ->
+// 47; the other way round at 8000 entries: 50 against 52 us for 2000 x 512).
+constexpr int64_t ROWS_VEC_MAX_V = 4096;
 bool z_cached(const OaceArgs& a) {
   return !(a.flags & OACE_FLAG_RECOMPUTE_Z) && (size_t)a.N * ldz_of(a.V) * sizeof(float) <= ZC_MAX_BYTES;
 }
@@ -663,6 +668,10 @@ hipError_t oace_linear_fwd_mfma(int dtype, const OaceArgs& a, void* rows, void* 
     e = launch_gemm_dt<MODE_SQ>(dtype, g, st);
   }
   if (e != hipSuccess) return e;
+  if (zc && a.V <= ROWS_VEC_MAX_V) {
+    if ((e = oace_rows_z(a, g.zc, g.ldz, rows, st)) != hipSuccess) return e;
+    return oace_mean_launch(dtype, rows, a.N, a.loss, st);
+  }
   if (zc) {
     hipLaunchKernelGGL(oace_mfma_row_cached_kernel, dim3((unsigned)a.N), dim3(RC_THREADS), 0, st, (const float*)part,
                        g.nvt, (const float*)g.zc, g.ldz, g.N, g.V, inv_v, (float)a.eps, (float)a.gamma, a.targets,

@@ -376,3 +376,16 @@ def test_dw_split_over_the_rows(shape, dtype, tied):
     _, rcache = _fwd(h.double(), wv.double(), t)
     rh, rw = _grads(rcache, g)
     assert normwise(to_f64(dh), to_f64(rh)) <= 2e-2 and normwise(to_f64(dw), to_f64(rw)) <= 2e-2
+
+
+@pytest.mark.parametrize("V", [4095, 4096, 4097])
+@pytest.mark.parametrize("N", [3, 130])
+def test_forward_rows_at_the_kernel_change(N, V):
+    """Kept logits on both sides of the row length at which the forward changes its row kernel
+    (4096), against the fp64 path: fp32 sums of exact inputs, 2e-5 as test_linear_matches_golden."""
+    h, w, t = _case(N, 64, V, torch.bfloat16, seed=N + V, scale=0.5)
+    loss, cache = _fwd(h, w, t)
+    ref, rcache = _fwd(h.double(), w.double(), t)
+    assert abs(float(loss) - float(ref)) <= 2e-5 * abs(float(ref))
+    for f in range(7):
+        assert normwise(to_f64(cache[3][:, f]), to_f64(rcache[3][:, f])) <= (1e-4 if f == 5 else 2e-5), f
