@@ -206,8 +206,10 @@ hipError_t oace_linear_bwd_generic(int dtype, const OaceArgs& a, const void* row
 hipError_t oace_mean_launch(int dtype, void* rows, int64_t N, void* loss, hipStream_t st);
 hipError_t oace_softmax_fwd_launch(int dtype, const OaceArgs& a, void* rows, hipStream_t st);
 hipError_t oace_softmax_bwd_launch(int dtype, const OaceArgs& a, const void* rows, void* dz, hipStream_t st);
-hipError_t oace_transpose16(const void* x, int64_t rows, int64_t cols, int64_t ldx, void* y, int64_t ldy,
-                            hipStream_t st);
+// y (rows x ldy, ldy a multiple of 8, 16-byte aligned) = the rows x cols 2-byte elements of x (row
+// stride ldx, rows of any alignment), zeros in [cols, ldy) (oace.hip).
+hipError_t oace_align_rows16(const void* x, int64_t rows, int64_t cols, int64_t ldx, void* y, int64_t ldy,
+                             hipStream_t st);
 // MFMA path (oace_mfma.hip): bf16/fp16, d_model a multiple of 32, 16-byte aligned rows of h (and
 // of W^T for OACE_W_VD).
 bool oace_mfma_supported(int dtype, const OaceArgs& a);
@@ -241,7 +243,7 @@ struct OaceGemm {
 };
 bool oace_gemm_fits(const OaceGemm& g);
 // Contraction parts for about `wgs` workgroups (1: no split); parts > 1 need part_bytes of fp32
-// partials, added in part order by a second kernel (row-contiguous A only).
+// partials, added in part order by a second kernel.
 int oace_gemm_parts(const OaceGemm& g, int wgs);
 size_t oace_gemm_part_bytes(const OaceGemm& g, int parts);
 hipError_t oace_gemm(int dtype, const OaceGemm& g, int parts, float* part, hipStream_t st);

@@ -21,7 +21,8 @@
 // taken first.  Rows and columns past the operand extents read the last valid row / 8-column chunk
 // (data whose results are never stored).
 //
-//   dh: A = W^T (V x d, d contiguous) as MC over (m = d_model, k = vocab), B = dz (N x ldz) as KC;
+//   dh: A = a (V, d) embedding as MC over (m = d_model, k = vocab), or the (d, V) head as KC, B = dz
+//       (N x ldz) as KC;
 //   dW, (d, V) layout: A = dz as MC over (m = vocab, k = rows), B = h as MC over (n = d_model);
 //   dW, (V, d) layout: A = h as MC, B = dz as MC (D[v][k], d contiguous).
 #include <algorithm>
@@ -504,15 +505,17 @@ hipError_t bg_launch(const BgArgs& g, hipStream_t st) {
 template <int DT, int WN>
 hipError_t bg_run(const OaceGemm& g, BgArgs& b, hipStream_t st) {
   if (b.parts > 1) {
-    if (!g.a_mc) return hipErrorNotSupported;
-    hipError_t e = g.b_mc ? bg_launch<DT, true, true, OUT_PART, WN>(b, st)
-                          : bg_launch<DT, true, false, OUT_PART, WN>(b, st);
+    if (!g.a_mc && g.b_mc) return hipErrorNotSupported;
+    hipError_t e = g.b_mc   ? bg_launch<DT, true, true, OUT_PART, WN>(b, st)
+                   : g.a_mc ? bg_launch<DT, true, false, OUT_PART, WN>(b, st)
+                            : bg_launch<DT, false, false, OUT_PART, WN>(b, st);
     if (e != hipSuccess) return e;
     const int64_t threads = (int64_t)b.mt * b.nt * Cfg<WN>::NW * 32 * 64;
     hipLaunchKernelGGL((oace_bwd_gemm_sum_kernel<DT, WN>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
                        (const f32x4_t*)b.part, b.parts, b.mt, b.nt, b.am, b.bn, b.out, b.ldo);
     return hipGetLastError();
   }
+  if (!g.a_mc && !g.b_mc) return bg_launch<DT, false, false, OUT_ELEM, WN>(b, st);
   if (g.a_mc && !g.b_mc) return bg_launch<DT, true, false, OUT_ELEM, WN>(b, st);
   if (g.a_mc && g.b_mc) return bg_launch<DT, true, true, OUT_ELEM, WN>(b, st);
   return hipErrorNotSupported;

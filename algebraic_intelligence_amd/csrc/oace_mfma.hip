@@ -21,8 +21,9 @@
 // through a 3-stage LDS ring filled by direct global -> LDS loads (64-byte rows, 16-byte chunks
 // swizzled by (row >> 2) & 3: 16 consecutive rows in 16 distinct bank groups), one barrier per
 // step.  Tiles of one vocabulary block are dispatched consecutively on one XCD (they share its W tile in L2).
-// W is used as W^T (vocab, d_model) with d_model contiguous: a tied embedding already is; the
-// (d_model, vocab) output head is transposed once per call into the workspace.
+// W is read where it lies, a tied (vocab, d_model) embedding along d_model and the (d_model, vocab)
+// output head along the vocabulary; a head whose rows are no whole 16-byte chunks (an odd vocabulary)
+// is copied once per call to aligned rows in the workspace.
 #include <algorithm>
 #include <type_traits>
 
@@ -45,8 +46,8 @@ constexpr int LOADS = A_LOADS + B_LOADS;
 constexpr int MODE_SQ = 0, MODE_OCTIC = 1, MODE_DZ = 2, MODE_SQZ = 3;
 
 struct GemmArgs {
-  const unsigned short* wt;  // (V, d), row stride ldwt
-  int64_t ldwt;
+  const unsigned short* w;  // (V, d) with row stride ldw, or, DV, (d, V) with 16-byte aligned rows
+  int64_t ldw;
   const unsigned short* h;  // (N, d), row stride ldh
   int64_t ldh;
   int N, V, d, nvt, nnt;
@@ -78,9 +79,32 @@ __host__ __device__ constexpr int vm_only(int n) { return (n & 0xF) | ((n >> 4) 
 // Byte offset of logical 16-byte chunk lc of row r in a tile of 64-byte rows.
 __device__ __forceinline__ int chunk_off(int r, int lc) { return r * 64 + ((lc ^ ((r >> 2) & 3)) << 4); }
 
+// A (d, V) weight's tile: 32 contraction rows of TV entries, 16-byte chunk c of row r at
+// c ^ ((r & 3) << 2), so that a transposed read's four rows use different bank groups.
+typedef __attribute__((ext_vector_type(4))) short m_s16x4_t;
+typedef __attribute__((address_space(3))) m_s16x4_t m_lds_s16x4_t;
+
+// MFMA operand from that tile: vocabulary rows 32 blk + l32, contraction rows 16 kk + 8 g .. + 7.
+__device__ __forceinline__ u32x4_t wdv_frag(const unsigned char* st, int blk, int kk, int lane) {
+  const int l16 = lane & 15, m16 = (lane >> 4) & 1, g = lane >> 5;
+  u32x4_t f;
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    const int row = 16 * kk + 8 * g + 4 * hh + (l16 >> 2), c = blk * 4 + m16 * 2 + ((l16 & 3) >> 1);
+    const unsigned char* p = st + row * (TV * 2) + ((c ^ ((row & 3) << 2)) << 4) + (l16 & 1) * 8;
+    const m_s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((m_lds_s16x4_t*)p);
+    const u32x2_t w = __builtin_bit_cast(u32x2_t, v);
+    f[2 * hh] = w[0];
+    f[2 * hh + 1] = w[1];
+  }
+  return f;
+}
+
 }  // namespace
 
-template <int DT, int MODE>
+// DV: W as the (d, V) output head, row-contiguous tiles (fragments by ds_read_tr16_b64): each step
+// reads 512 bytes of 32 rows, where a (V, d) weight's tiles take 64 bytes of 256.
+template <int DT, int MODE, bool DV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void oace_mfma_gemm_kernel(const GemmArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[NSTAGE * STAGE];
@@ -101,8 +125,15 @@ void oace_mfma_gemm_kernel(const GemmArgs a) {
   const unsigned short* bsrc[B_LOADS];
 #pragma unroll
   for (int i = 0; i < A_LOADS; ++i) {
-    const int s = 256 * i + tid, r = s >> 2, lc = (s & 3) ^ ((r >> 2) & 3);
-    asrc[i] = a.wt + (int64_t)min(v0 + r, a.V - 1) * a.ldwt + lc * 8;
+    const int s = 256 * i + tid;
+    if constexpr (DV) {
+      // contraction row s / 32, entries from v0 + 8 c (past the last chunk: the last one)
+      const int r = s >> 5, c = (s & 31) ^ ((r & 3) << 2);
+      asrc[i] = a.w + (int64_t)r * a.ldw + min(v0 + 8 * c, ((a.V + 7) >> 3) * 8 - 8);
+    } else {
+      const int r = s >> 2, lc = (s & 3) ^ ((r >> 2) & 3);
+      asrc[i] = a.w + (int64_t)min(v0 + r, a.V - 1) * a.ldw + lc * 8;
+    }
   }
 #pragma unroll
   for (int i = 0; i < B_LOADS; ++i) {
@@ -111,6 +142,16 @@ void oace_mfma_gemm_kernel(const GemmArgs a) {
   }
   auto issue = [&](int t) {
     unsigned char* st = lds + (t % NSTAGE) * STAGE;
+    if constexpr (DV) {
+      // lds_dma16: the compiler waits for every direct load it knows of before a transposed read
+#pragma unroll
+      for (int i = 0; i < A_LOADS; ++i)
+        lds_dma16((const void*)(asrc[i] + (int64_t)t * KS * a.ldw), st + (256 * i + wave * 64) * 16);
+#pragma unroll
+      for (int i = 0; i < B_LOADS; ++i)
+        lds_dma16((const void*)(bsrc[i] + t * KS), st + A_BYTES + (256 * i + wave * 64) * 16);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(asrc[i] + t * KS), (void*)(st + (256 * i + wave * 64) * 16), 16, 0, 0);
@@ -155,7 +196,9 @@ void oace_mfma_gemm_kernel(const GemmArgs a) {
     for (int kk = 0; kk < 2; ++kk) {
       u32x4_t af[2], bf[4];
 #pragma unroll
-      for (int vb = 0; vb < 2; ++vb) af[vb] = *(const u32x4_t*)(st + chunk_off(wave * 64 + vb * 32 + l32, 2 * kk + g));
+      for (int vb = 0; vb < 2; ++vb)
+        af[vb] = DV ? wdv_frag(st, wave * 2 + vb, kk, lane)
+                    : *(const u32x4_t*)(st + chunk_off(wave * 64 + vb * 32 + l32, 2 * kk + g));
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) bf[nb] = *(const u32x4_t*)(st + A_BYTES + chunk_off(nb * 32 + l32, 2 * kk + g));
 #pragma unroll
@@ -553,13 +596,25 @@ bool z_cached(const OaceArgs& a) {
   return !(a.flags & OACE_FLAG_RECOMPUTE_Z) && (size_t)a.N * ldz_of(a.V) * sizeof(float) <= ZC_MAX_BYTES;
 }
 
-// dh (N, d) = dz W^T as D[n][m] = sum_v W^T[v][m] dz[n][v]: A = W^T row-contiguous over the
-// model features, B = dz contraction-contiguous.  Its vocabulary contraction is split for this
-// many workgroups: a constant, so that the summation order, and the result, do not depend on
-// the device.
+// The (d, V) head is read where it lies when its rows are whole 16-byte chunks (V and ldw multiples of
+// 8; MAX_KC: oace_mfma_supported); otherwise through a copy with aligned rows at the start of the
+// workspace -- made here, or left there by a forward call on the same workspace and weights
+// (OACE_FLAG_WT_READY, the caller's guarantee).  A transposed (V, d) copy, which every (d, V) head took
+// before, cost 35 us of a forward of 512 x 768 x 50257 where the aligned copy takes 28: forward
+// 125 -> 119 us; at V = 50304, read in place, 125 -> 91 (backward 152 -> 158, dh's operand being
+// contraction-contiguous).
+constexpr int64_t MAX_KC = int64_t(1) << 23;
+bool dv_in_place(const OaceArgs& a) { return a.V % 8 == 0 && a.ldw % 8 == 0 && a.ldw <= MAX_KC && al16(a.w); }
+// Sized without the weight's address and stride, which a workspace query does not know.
+size_t copy_bytes(const OaceArgs& a) { return a.w_layout == OACE_W_DV ? al((size_t)a.d * ldz_of(a.V) * 2) : 0; }
+
+// dh (N, d) = dz W^T as D[n][m] = sum_v W(m, v) dz[n][v]: A = W row-contiguous over the model
+// features (a (V, d) embedding) or contraction-contiguous (a (d, V) head), B = dz
+// contraction-contiguous.  Its vocabulary contraction is split for this many workgroups: a constant,
+// so that the summation order, and the result, do not depend on the device.
 constexpr int SPLIT_WGS = 256;
-OaceGemm dh_gemm(const OaceArgs& a, const unsigned short* wt, int64_t ldwt, const unsigned short* dz) {
-  return OaceGemm{wt, ldwt, true, a.d, dz, ldz_of(a.V), false, a.N, a.V, a.dh, a.d};
+OaceGemm dh_gemm(const OaceArgs& a, const unsigned short* w, int64_t ldw, const unsigned short* dz) {
+  return OaceGemm{w, ldw, a.w_layout != OACE_W_DV, a.d, dz, ldz_of(a.V), false, a.N, a.V, a.dh, a.d};
 }
 
 // dW = h^T dz in W's layout, split over the rows when its tiles are fewer than the workgroup slots
@@ -576,7 +631,7 @@ struct Layout {
 };
 Layout layout_of(const OaceArgs& a) {
   Layout l;
-  l.wt = a.w_layout == OACE_W_DV ? al((size_t)a.V * a.d * 2) : 0;
+  l.wt = copy_bytes(a);
   l.zc = z_cached(a) ? al((size_t)a.N * ldz_of(a.V) * sizeof(float)) : 0;
   l.part = al((size_t)nvt_of(a.V) * a.N * 4 * sizeof(float));
   l.dz = al((size_t)a.N * ldz_of(a.V) * 2);
@@ -588,24 +643,19 @@ Layout layout_of(const OaceArgs& a) {
   return l;
 }
 
-// W^T (V, d) with d contiguous: the caller's tied embedding, or a transposed copy at the start of
-// the workspace -- made here, or left there by a forward call on the same workspace and weights
-// (OACE_FLAG_WT_READY, the caller's guarantee).
-const unsigned short* wt_of(const OaceArgs& a, void* ws, int64_t& ldwt, hipStream_t st, hipError_t& e) {
+const unsigned short* w_of(const OaceArgs& a, void* ws, int64_t& ldw, hipStream_t st, hipError_t& e) {
   e = hipSuccess;
-  if (a.w_layout == OACE_W_VD) {
-    ldwt = a.ldw;
-    return (const unsigned short*)a.w;
-  }
-  ldwt = a.d;
-  if (!(a.flags & OACE_FLAG_WT_READY)) e = oace_transpose16(a.w, a.d, a.V, a.ldw, ws, a.d, st);
+  ldw = a.ldw;
+  if (a.w_layout == OACE_W_VD || dv_in_place(a)) return (const unsigned short*)a.w;
+  ldw = ldz_of(a.V);
+  if (!(a.flags & OACE_FLAG_WT_READY)) e = oace_align_rows16(a.w, a.d, a.V, a.ldw, ws, ldw, st);
   return (const unsigned short*)ws;
 }
 
-GemmArgs gemm_args(const OaceArgs& a, const unsigned short* wt, int64_t ldwt) {
+GemmArgs gemm_args(const OaceArgs& a, const unsigned short* w, int64_t ldw) {
   GemmArgs g = {};
-  g.wt = wt;
-  g.ldwt = ldwt;
+  g.w = w;
+  g.ldw = ldw;
   g.h = (const unsigned short*)a.h;
   g.ldh = a.ldh;
   g.N = (int)a.N;
@@ -618,15 +668,16 @@ GemmArgs gemm_args(const OaceArgs& a, const unsigned short* wt, int64_t ldwt) {
 }
 
 template <int DT, int MODE>
-hipError_t launch_gemm(const GemmArgs& g, hipStream_t st) {
+hipError_t launch_gemm(const GemmArgs& g, bool dv, hipStream_t st) {
   const unsigned grid = (unsigned)(8 * g.nnt * ((g.nvt + 7) / 8));
-  hipLaunchKernelGGL((oace_mfma_gemm_kernel<DT, MODE>), dim3(grid), dim3(256), 0, st, g);
+  if (dv) hipLaunchKernelGGL((oace_mfma_gemm_kernel<DT, MODE, true>), dim3(grid), dim3(256), 0, st, g);
+  else hipLaunchKernelGGL((oace_mfma_gemm_kernel<DT, MODE, false>), dim3(grid), dim3(256), 0, st, g);
   return hipGetLastError();
 }
 
 template <int MODE>
-hipError_t launch_gemm_dt(int dtype, const GemmArgs& g, hipStream_t st) {
-  return dtype == AFA_BF16 ? launch_gemm<AFA_BF16, MODE>(g, st) : launch_gemm<AFA_F16, MODE>(g, st);
+hipError_t launch_gemm_dt(int dtype, const GemmArgs& g, bool dv, hipStream_t st) {
+  return dtype == AFA_BF16 ? launch_gemm<AFA_BF16, MODE>(g, dv, st) : launch_gemm<AFA_F16, MODE>(g, dv, st);
 }
 
 }  // namespace
@@ -635,8 +686,9 @@ bool oace_mfma_supported(int dtype, const OaceArgs& a) {
   if (dtype != AFA_BF16 && dtype != AFA_F16) return false;
   if (a.d % KS != 0 || a.ldh % 8 != 0 || !al16(a.h)) return false;
   if (a.w_layout == OACE_W_VD && (a.ldw % 8 != 0 || !al16(a.w))) return false;
-  if (a.N > (1 << 28) || a.V >= (1 << 24)) return false;
-  // 32-bit per-lane offsets of the backward GEMMs' direct loads
+  if (a.N > (1 << 28) || a.V > MAX_KC) return false;
+  // 32-bit per-lane byte offsets of the backward GEMMs' direct loads: 31 rows of a row-contiguous
+  // operand, 255 of a contraction-contiguous one (dz, the (d, V) head)
   if (a.ldh >= (1 << 26) || (a.w_layout == OACE_W_VD && a.ldw >= (1 << 26))) return false;
   return true;
 }
@@ -650,11 +702,12 @@ hipError_t oace_linear_fwd_mfma(int dtype, const OaceArgs& a, void* rows, void* 
   const Layout l = layout_of(a);
   char* base = (char*)ws;
   hipError_t e;
-  int64_t ldwt = 0;
-  const unsigned short* wt = wt_of(a, base, ldwt, st, e);
+  int64_t ldw = 0;
+  const bool dv = a.w_layout == OACE_W_DV;
+  const unsigned short* w = w_of(a, base, ldw, st, e);
   if (e != hipSuccess) return e;
   float* part = (float*)(base + l.wt + l.zc);
-  GemmArgs g = gemm_args(a, wt, ldwt);
+  GemmArgs g = gemm_args(a, w, ldw);
   g.rows = (const float*)rows;
   g.part = part;
   const float inv_v = (float)(1.0 / (double)a.V);
@@ -662,10 +715,10 @@ hipError_t oace_linear_fwd_mfma(int dtype, const OaceArgs& a, void* rows, void* 
   if (zc) {
     g.zc = (float*)(base + l.wt);
     g.ldz = ldz_of(a.V);
-    e = launch_gemm_dt<MODE_SQZ>(dtype, g, st);
+    e = launch_gemm_dt<MODE_SQZ>(dtype, g, dv, st);
   } else {
     g.zt = (float*)rows + (OACE_ROW - 1);
-    e = launch_gemm_dt<MODE_SQ>(dtype, g, st);
+    e = launch_gemm_dt<MODE_SQ>(dtype, g, dv, st);
   }
   if (e != hipSuccess) return e;
   if (zc && a.V <= ROWS_VEC_MAX_V) {
@@ -683,7 +736,7 @@ hipError_t oace_linear_fwd_mfma(int dtype, const OaceArgs& a, void* rows, void* 
   hipLaunchKernelGGL(oace_mfma_tau_kernel, dim3(rg), dim3(256), 0, st, (const float*)part, g.nvt, g.N, inv_v,
                      (float)a.eps, (float*)rows);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = launch_gemm_dt<MODE_OCTIC>(dtype, g, st)) != hipSuccess) return e;
+  if ((e = launch_gemm_dt<MODE_OCTIC>(dtype, g, dv, st)) != hipSuccess) return e;
   const unsigned wg = (unsigned)((a.N + 3) / 4);
   hipLaunchKernelGGL(oace_mfma_rows_kernel, dim3(wg), dim3(256), 0, st, (const float*)part, g.nvt, g.N, inv_v,
                      (float)a.gamma, g.V, a.targets, (float*)rows);
@@ -695,12 +748,13 @@ hipError_t oace_linear_bwd_mfma(int dtype, const OaceArgs& a, const void* rows, 
   const Layout l = layout_of(a);
   char* base = (char*)ws;
   hipError_t e;
-  int64_t ldwt = 0;
-  const unsigned short* wt = wt_of(a, base, ldwt, st, e);
+  int64_t ldw = 0;
+  const bool dv = a.w_layout == OACE_W_DV;
+  const unsigned short* w = w_of(a, base, ldw, st, e);
   if (e != hipSuccess) return e;
   char* sbase = base + l.wt + l.zc;  // the region after the cached logits
   unsigned short* dz = (unsigned short*)sbase;
-  GemmArgs g = gemm_args(a, wt, ldwt);
+  GemmArgs g = gemm_args(a, w, ldw);
   g.rows = (const float*)rows;
   g.dz = dz;
   g.ldz = ldz_of(a.V);
@@ -718,11 +772,11 @@ hipError_t oace_linear_bwd_mfma(int dtype, const OaceArgs& a, const void* rows, 
                          (const float*)rows, a.targets, g.c0, g.g_loss, dz);
     e = hipGetLastError();
   } else {
-    e = launch_gemm_dt<MODE_DZ>(dtype, g, st);
+    e = launch_gemm_dt<MODE_DZ>(dtype, g, dv, st);
   }
   if (e != hipSuccess) return e;
   float* parts = (float*)(sbase + l.dz);
-  const OaceGemm gh = dh_gemm(a, wt, ldwt, dz);
+  const OaceGemm gh = dh_gemm(a, w, ldw, dz);
   if ((e = oace_gemm(dtype, gh, oace_gemm_parts(gh, SPLIT_WGS), parts, st)) != hipSuccess) return e;
   const OaceGemm gw = dw_gemm(a, dz);
   return oace_gemm(dtype, gw, oace_gemm_parts(gw, SPLIT_WGS), parts, st);

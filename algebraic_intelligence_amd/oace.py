@@ -76,7 +76,7 @@ def fused_linear_oace_forward(h, w_vocab, targets, eps_vocab: float = 100.0, gam
     loss = torch.empty((), dtype=acc, device=dev)
     rows = torch.empty((N, ROW_FIELDS), dtype=acc, device=dev)
     code = _lib.dtype_code(h.dtype)
-    # the backward reuses this workspace (and the transposed weights the forward leaves in it)
+    # the backward reuses this workspace (and the copy or planes of the weights the forward leaves in it)
     with _lib.on_device(dev):
         wsb = _lib.workspace_size("oace_workspace_size", dev, code, N, d, V, layout, flags)
         ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
@@ -105,7 +105,7 @@ def fused_linear_oace_backward(cache, g):
     else:
         dw_store = torch.empty((V, ldw), dtype=w_vocab.dtype, device=dev)
         dw = dw_store[:, :d].t()
-    # the forward's transposed weights are still valid unless w_vocab was modified in place since,
+    # the forward's copy or planes of the weights are still valid unless w_vocab was modified in place since,
     # and its logits unless h or w_vocab was
     w_same = w_vocab._version == w_version
     bflags = flags | (FLAG_WT_READY if w_same else 0) | (FLAG_Z_READY if w_same and hf._version == h_version else 0)

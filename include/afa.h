@@ -226,8 +226,8 @@ int ago_rotate_qk(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int6
 #define OACE_W_VD 1
 #define OACE_ROW_FIELDS 8
 /* oace_linear_bwd: the workspace is the one an oace_linear_fwd call with the same arguments used,
-   and the weights have not changed since; the transposed copy of an OACE_W_DV weight (fp32: the
-   bf16 planes of the weight) that call left in it is reused. */
+   and the weights have not changed since; the aligned copy of an OACE_W_DV weight (fp32: the bf16
+   planes of the weight) that call left in it is reused. */
 #define OACE_FLAG_WT_READY 0x10u
 /* oace_linear_bwd: as OACE_FLAG_WT_READY, and h has not changed either; the fp32 logits that the
    forward keeps in the workspace (when rows x vocab x 4 bytes fit 256 MB) are reused, so dz is

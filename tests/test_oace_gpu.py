@@ -389,3 +389,22 @@ def test_forward_rows_at_the_kernel_change(N, V):
     assert abs(float(loss) - float(ref)) <= 2e-5 * abs(float(ref))
     for f in range(7):
         assert normwise(to_f64(cache[3][:, f]), to_f64(rcache[3][:, f])) <= (1e-4 if f == 5 else 2e-5), f
+
+
+@pytest.mark.parametrize("dtype", LOW)
+@pytest.mark.parametrize("shape", [(3, 32, 8), (130, 64, 248), (33, 96, 264), (520, 32, 1088), (257, 160, 2056)])
+def test_head_read_in_place_equals_its_aligned_copy(shape, dtype):
+    """A (d, V) head whose rows are whole 16-byte chunks is read where it lies; the same weights at an
+    odd offset or row stride go through the aligned copy.  Same products in the same order: equal."""
+    N, d, V = shape
+    h, w, t = _case(N, d, V, dtype, seed=N + V, scale=0.5)
+    loss, cache = _fwd(h, w, t)
+    dh, dw = _grads(cache, 1.0)
+    for off, ld in [(0, V + 8), (8, V + 16), (1, V + 8), (3, V + 7), (0, V + 1)]:
+        store = torch.full((d * ld + off + 16,), float("nan"), dtype=dtype, device=w.device)
+        view = store[off:off + d * ld].view(d, ld)[:, :V]
+        view.copy_(w)
+        loss2, cache2 = _fwd(h, view, t)
+        dh2, dw2 = _grads(cache2, 1.0)
+        assert float(loss2) == float(loss), (off, ld)
+        assert torch.equal(cache2[3], cache[3]) and torch.equal(dh2, dh) and torch.equal(dw2, dw), (off, ld)
