@@ -5,7 +5,8 @@
 // score of a key tile by Cauchy-Schwarz with it (|q . k| <= |q| |k|) and use the branch-free
 // rho^8 only where that bound keeps |s| <= kFastRhoMaxScore.  It reads the tensor once and writes
 // B H ceil(L/64) floats; with rotary tables the K rotation pass (afa_krot_kernel) produces the
-// same bounds from the rotated rows instead, for the forward's k and the backward's q and k.
+// same bounds from the rotated rows instead.  The backward's come from its own pre-pass up to head_dim
+// 128, from here at 256.
 #include <cmath>
 
 #include "afa_common.h"

@@ -600,7 +600,7 @@ bool z_cached(const OaceArgs& a) {
 // 8; MAX_KC: oace_mfma_supported); otherwise through a copy with aligned rows at the start of the
 // workspace -- made here, or left there by a forward call on the same workspace and weights
 // (OACE_FLAG_WT_READY, the caller's guarantee).  A transposed (V, d) copy, which every (d, V) head took
-// before, cost 35 us of a forward of 512 x 768 x 50257 where the aligned copy takes 28: forward
+// before, cost 35 us of a forward of 512 x 768 x 50257 where the aligned copy takes 26: forward
 // 125 -> 119 us; at V = 50304, read in place, 125 -> 91 (backward 152 -> 158, dh's operand being
 // contraction-contiguous).
 constexpr int64_t MAX_KC = int64_t(1) << 23;
