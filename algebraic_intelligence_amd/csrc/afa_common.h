@@ -89,6 +89,11 @@ struct Elem<AFA_F32> {
 // aligned address at or below the row's start and the start.  Whole chunks move as one 16-byte
 // access; the first and the last chunk of a row that starts or ends inside one move element by
 // element, so nothing outside the row is read or written (entries outside it load as zeros).
+// Kernels that sum over a row take its whole chunks (RowSpan) and, one to a lane, the elements before
+// and after them: a chunk's zeros would add rho(0) = 1 each to sums that can be far smaller.
+struct RowSpan {
+  int head, body, tail;  // elements before the first whole chunk, whole chunks, elements after the last
+};
 template <int DT>
 struct RowChunk {
   static constexpr int ESZ = DT == AFA_F32 ? 4 : 2;
@@ -96,6 +101,15 @@ struct RowChunk {
   static __device__ __forceinline__ int lead(const void* row) { return (int)((uintptr_t)row & 15u) / ESZ; }
   static __host__ __device__ __forceinline__ int count(int n, int lead) {
     return (int)(((int64_t)n + lead + EPC - 1) / EPC);
+  }
+  static __host__ __device__ __forceinline__ RowSpan span(const void* row, int n) {
+    const int to = (int)((16u - ((uintptr_t)row & 15u)) & 15u) / ESZ, head = to < n ? to : n;
+    const int body = (n - head) / EPC;
+    return RowSpan{head, body, n - head - body * EPC};
+  }
+  // the element outside the whole chunks that lane i of a row takes (2 * EPC lanes), or -1
+  static __device__ __forceinline__ int edge(RowSpan s, int n, int i) {
+    return i < s.head ? i : i >= EPC && i < EPC + s.tail ? n - s.tail + i - EPC : -1;
   }
   // chunks of the worst start
   static __host__ __device__ __forceinline__ int count_max(int n) { return count(n, EPC - 1); }

@@ -207,13 +207,12 @@ __device__ __forceinline__ float octic_hw(float z, float& r_out) {
 }
 
 // ---------------------------------------------------------------- register-resident row kernels
-// T threads per row (one wave, or 4 or 8 waves for longer rows), the whole row held in registers as the
-// aligned 16-byte chunks that cover it (RowChunk: any length and any start; thread l owns chunks
-// l, l + T, ...): one HBM read of x (and g), one write; rho^8 and r are evaluated once per element
-// with the hardware rsqrt / reciprocal (octic_hw) and the row is normalised with one division and
-// products; the multi-pass kernels above keep IEEE 1/sqrt and divisions throughout.  Entries of a
-// chunk outside the row are zeros: they add nothing to the sum of squares and 1 (rho(0)) each to the
-// octic sum, taken off again.
+// T threads per row (one wave, or 4 to 16 waves for longer rows), the whole row held in registers as its
+// aligned 16-byte chunks (RowChunk: any length and any start; thread l owns chunks l, l + T, ...) and,
+// where it starts or ends inside a chunk, one element each of the first lanes: one HBM read of x (and
+// g), one write; rho^8 and r are evaluated once per element with the hardware rsqrt / reciprocal
+// (octic_hw) and the row is normalised with one division and products; the multi-pass kernels above
+// keep IEEE 1/sqrt and divisions throughout.
 // Forward of (18372, 1531) fp32 109 -> 41 us (5.5 TB/s) and its VJP 267 -> 80 us (4.2 TB/s) against the
 // multi-pass kernels, which served every row whose length was no multiple of a chunk or over 64 x 8
 // (VJP: 64 x 4) chunks.
@@ -250,16 +249,18 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
   const int tid = threadIdx.x % T;
   const char* xr = (const char*)x + row * n * R::ESZ;
   char* yr = (char*)y + row * n * R::ESZ;
-  const int lead = R::lead(xr), nch = R::count(n, lead);
+  const RowSpan sp = R::span(xr, n);
+  const int edge = R::edge(sp, n, tid);
   u32x4_t raw[NCH];
   float v[NCH][R::EPC];
-  float ss[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int c = tid + T * j;
     raw[j] = u32x4_t{0u, 0u, 0u, 0u};
-    if (c < nch) raw[j] = R::load(xr, c * R::EPC - lead, n);
+    if (c < sp.body) raw[j] = *(const u32x4_t*)(xr + (int64_t)(sp.head + c * R::EPC) * R::ESZ);
   }
+  float ve = edge >= 0 ? Elem<DT>::load(xr, edge) : 0.f;
+  float ss[1] = {ve * ve};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     R::unpack(raw[j], v[j]);
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
   float ks[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if (tid + T * j < nch) {
+    if (tid + T * j < sp.body) {
 #pragma unroll
       for (int i = 0; i < R::EPC; ++i) {
         float r;
@@ -280,17 +281,23 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
       }
     }
   }
+  if (edge >= 0) {
+    float r;
+    ve = octic_hw(ve * tau, r);
+    ks[0] += ve;
+  }
   row_sum<T, 1>(ks, sh);
-  const float inv = 1.0f / (ks[0] - (float)(nch * R::EPC - n) + sink);
+  const float inv = 1.0f / (ks[0] + sink);
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int c = tid + T * j;
-    if (c < nch) {
+    if (c < sp.body) {
 #pragma unroll
       for (int i = 0; i < R::EPC; ++i) v[j][i] = v[j][i] * inv;
-      R::store(yr, c * R::EPC - lead, n, R::pack(v[j]));
+      *(u32x4_t*)(yr + (int64_t)(sp.head + c * R::EPC) * R::ESZ) = R::pack(v[j]);
     }
   }
+  if (edge >= 0) Elem<DT>::store(yr, edge, ve * inv);
 }
 
 template <int DT, int T, int NCH>
@@ -312,20 +319,23 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int
   const char* xr = (const char*)x + row * n * R::ESZ;
   const char* gr = (const char*)g + row * n * R::ESZ;
   char* dr = (char*)dx + row * n * R::ESZ;
-  const int lead = R::lead(xr), nch = R::count(n, lead);
+  const RowSpan sp = R::span(xr, n);
+  const int edge = R::edge(sp, n, tid);
   const float inv_n = 1.f / (float)n;
   u32x4_t xw[NCH], gw[NCH];
   float w[NCH][R::EPC];
-  float ss[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int c = tid + T * j;
     xw[j] = gw[j] = u32x4_t{0u, 0u, 0u, 0u};
-    if (c < nch) {
-      xw[j] = R::load(xr, c * R::EPC - lead, n);
-      gw[j] = R::load(gr, c * R::EPC - lead, n);
+    if (c < sp.body) {
+      const int64_t off = (int64_t)(sp.head + c * R::EPC) * R::ESZ;
+      xw[j] = *(const u32x4_t*)(xr + off);
+      gw[j] = *(const u32x4_t*)(gr + off);
     }
   }
+  const float xe = edge >= 0 ? Elem<DT>::load(xr, edge) : 0.f, ge = edge >= 0 ? Elem<DT>::load(gr, edge) : 0.f;
+  float ss[1] = {xe * xe}, we = 0.f;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     float z[R::EPC];
@@ -338,7 +348,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int
   float kp[2] = {0.f, 0.f};  // sum rho^8, sum rho^8 g
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if (tid + T * j < nch) {
+    if (tid + T * j < sp.body) {
       float z[R::EPC], gv[R::EPC];
       R::unpack(xw[j], z);
       R::unpack(gw[j], gv);
@@ -353,37 +363,47 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int
     }
     __builtin_amdgcn_sched_barrier(0);  // one chunk's unpacked values live at a time
   }
+  if (edge >= 0) {
+    float r;
+    const float p = octic_hw(xe * tau, r);
+    kp[0] += p;
+    kp[1] += p * ge;
+    we = 8.f * r * p;
+  }
   row_sum<T, 2>(kp, sh);
-  const float inv = 1.0f / (kp[0] - (float)(nch * R::EPC - n) + sink);
+  const float inv = 1.0f / (kp[0] + sink);
   const float dot = kp[1] * inv;
   float rad[1] = {0.f};
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if (tid + T * j < nch) {
+    if (tid + T * j < sp.body) {
       float z[R::EPC], gv[R::EPC];
       R::unpack(xw[j], z);
       R::unpack(gw[j], gv);
 #pragma unroll
       for (int i = 0; i < R::EPC; ++i) {
         w[j][i] = w[j][i] * inv * (gv[i] - dot);  // ng
-        rad[0] += w[j][i] * (z[i] * tau);  // z = 0 outside the row
+        rad[0] += w[j][i] * (z[i] * tau);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  we = we * inv * (ge - dot);  // 0 where the lane has no edge element
+  if (edge >= 0) rad[0] += we * (xe * tau);
   row_sum<T, 1>(rad, sh);
   rad[0] *= inv_n;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int c = tid + T * j;
-    if (c < nch) {
+    if (c < sp.body) {
       float z[R::EPC];
       R::unpack(xw[j], z);
 #pragma unroll
       for (int i = 0; i < R::EPC; ++i) w[j][i] = tau * (w[j][i] - rad[0] * (z[i] * tau));
-      R::store(dr, c * R::EPC - lead, n, R::pack(w[j]));
+      *(u32x4_t*)(dr + (int64_t)(sp.head + c * R::EPC) * R::ESZ) = R::pack(w[j]);
     }
   }
+  if (edge >= 0) Elem<DT>::store(dr, edge, tau * (we - rad[0] * (xe * tau)));
 }
 
 // The rows of all tensors start at the same offset from a 16-byte boundary (the chunks of one are the
@@ -421,13 +441,6 @@ static void oc_bwd(int64_t n, const void* x, const void* g, void* dx, hipStream_
   hipLaunchKernelGGL((octic_bwd_kernel<DT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, x, g, dx);
 }
 
-// Chunks that cover any row: rows of whole chunks all start where the first one does.
-template <int DT>
-static int row_chunks(int64_t n, const void* x) {
-  using R = RowChunk<DT>;
-  return n % R::EPC == 0 ? R::count((int)n, (int)((uintptr_t)x & 15u) / R::ESZ) : R::count_max((int)n);
-}
-
 // Threads per row and chunks per thread by the row's chunk count: the fewest threads that hold the row
 // in at most four chunks each (the VJP's x, g and 8 r rho^8 take 12 or 16 registers a chunk: six
 // chunks a lane leave one wave per SIMD, and (18372, 1531) fp32 took 173 us instead of 80).  false: no
@@ -439,7 +452,7 @@ static bool sm_reg_fits(int64_t rows, int nch) { return nch <= 4096 && (nch <= 2
 template <int DT>
 static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
   if (n > (1 << 20) || !same_lead(x, y, nullptr)) return false;
-  const int nch = row_chunks<DT>(n, x);
+  const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
 #define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_fwd_reg_kernel, T, NCH, x, y, (float)sink, (float)eps)
   if (nch <= 64) AFA_SM(64, 1);
@@ -459,7 +472,7 @@ template <int DT>
 static bool sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, void* dx, double sink, double eps,
                        hipStream_t st) {
   if (n > (1 << 20) || !same_lead(x, g, dx)) return false;
-  const int nch = row_chunks<DT>(n, x);
+  const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
 #define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_bwd_reg_kernel, T, NCH, x, g, dx, (float)sink, (float)eps)
   if (nch <= 64) AFA_SM(64, 1);

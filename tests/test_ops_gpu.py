@@ -656,3 +656,36 @@ def test_algebraic_softmax_row_kernels(dt, epc, tol, chunks):
             # at n = 1 the gradient is 0 but for eps: the size of its terms, p g, stands in
             scale = max(float(dd.abs().max()), 1e-3 * float((yd * g).abs().max()))
             assert float((dx.double() - dd).abs().max()) <= tol * scale, (n, off)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 9, 15, 17, 65, 129, 1031])
+@pytest.mark.parametrize("sink", [0.0, 0.5])
+def test_algebraic_softmax_small_row_sums(dt, n, sink):
+    """Rows of negative scores, whose octic sum (n terms near 9e-4) is far below the 1 that an entry
+    outside the row would add to it, at every start of a row against the fp64 kernel.  Bound: a
+    weight's relative error is 8 times that of rho, 6 roundings of 2^-24 (tau, the product, 1 + y^2, two
+    1-ulp units, one product), and 7 more of its squarings, 3.3e-6; a row's sum has no larger one, so p is
+    within 6.6e-6 plus the element type's rounding, and dx, the difference of two terms of up to 16 tau p g
+    that carry it, within four times that of 8 tau p g."""
+    from algebraic_intelligence_amd import _lib
+    # half a unit in the last place, relative to the smallest significand: 24, 8 and 11 bits
+    rows, eps = 16, {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    x = (-60.0 - torch.rand((rows, n), generator=gen, device=DEV)).to(dt)
+    g = torch.randn((rows, n), generator=gen, device=DEV).to(dt)
+    for start in range(0, 16 // x.element_size(), 3):
+        xs, gs = (torch.empty(rows * n + start, dtype=dt, device=DEV)[start:].view(rows, n).copy_(t) for t in (x, g))
+        y, dx = (torch.empty(rows * n + start, dtype=dt, device=DEV)[start:].view(rows, n) for _ in range(2))
+        code, stream = _lib.dtype_code(dt), _lib.stream_ptr(xs.device)
+        _lib.check(_lib.lib().asoftmax_fwd(code, rows, n, xs.data_ptr(), y.data_ptr(), sink, 1e-5, stream), "fwd")
+        _lib.check(_lib.lib().asoftmax_bwd(code, rows, n, xs.data_ptr(), gs.data_ptr(), dx.data_ptr(), sink, 1e-5, stream),
+                   "bwd")
+        xd = x.double().requires_grad_(True)
+        yd = A.algebraic_softmax(xd, sink_omega=sink)
+        (dd,) = torch.autograd.grad(yd, xd, g.double())
+        # fp16's smallest normal, 2^-14, bounds the rounding of the small p and dx of long rows
+        tiny = 2.0 ** -25 if dt == torch.float16 else 0.0
+        assert ((y.double() - yd).abs() <= (6.6e-6 + eps) * yd + tiny).all(), start
+        terms = 8.0 / 60.0 * (yd * g.double().abs().amax(-1, keepdim=True))
+        assert ((dx.double() - dd).abs() <= 2.7e-5 * terms + eps * dd.abs() + tiny).all(), start
