@@ -120,7 +120,8 @@ __global__ __launch_bounds__(256) void oace_mean_kernel(A* rows, int64_t N, int6
 }
 
 // The row records of 16- and 32-bit logits: T threads per row, the row read once into registers as
-// 16-byte chunks (NCH per thread; NCH = 0 streams a longer row twice).  Bound by the octic terms' VALU issue (about
+// its 16-byte chunks (NCH per thread; NCH = 0 streams a longer row twice) and, where it starts or ends
+// inside one, one element each of the first lanes.  Bound by the octic terms' VALU issue (about
 // 20 instructions and two quarter-rate ones per 16-bit entry) just above its one HBM read:
 // (2048, 50257) bf16, forward call with the mean 176 -> 76 us (2.7 TB/s; the two passes of 2-byte
 // loads by one 256-thread workgroup per row took 171 of the 176), fp32 97 us (4.3 TB/s).
@@ -136,10 +137,13 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
   if (row >= N) return;  // whole waves, and only where no barrier follows (one wave per row)
   const int tid = threadIdx.x % T, lane = threadIdx.x & 63, wave = tid >> 6;
   const char* zr = (const char*)z + row * ldz * R::ESZ;
-  const int lead = R::lead(zr), nch = R::count(V, lead);
+  const RowSpan sp = R::span(zr, V);
+  const int edge = R::edge(sp, V, tid);
+  const u32x4_t* body = (const u32x4_t*)(zr + (int64_t)sp.head * R::ESZ);
   constexpr int NR = NCH > 0 ? NCH : 1;
   u32x4_t raw[NR];
-  float ss = 0.f;
+  const float ve = edge >= 0 ? Elem<DT>::load(zr, edge) : 0.f;
+  float ss = ve * ve;
   auto sq = [&](u32x4_t w) {
     float v[R::EPC];
     R::unpack(w, v);
@@ -151,7 +155,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
     for (int j = 0; j < NCH; ++j) {
       const int c = tid + T * j;
       raw[j] = u32x4_t{0u, 0u, 0u, 0u};
-      if (c < nch) raw[j] = R::load(zr, c * R::EPC - lead, V);
+      if (c < sp.body) raw[j] = body[c];
     }
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
       __builtin_amdgcn_sched_barrier(0);
     }
   } else {
-    for (int c = tid; c < nch; c += T) sq(R::load(zr, c * R::EPC - lead, V));
+    for (int c = tid; c < sp.body; c += T) sq(body[c]);
   }
   ss = wave_sum(ss);
   if constexpr (NW > 1) {
@@ -171,33 +175,32 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
   }
   const float tau = o_rsq<float>(ss * inv_v + eps);
   float s[4] = {0.f, 0.f, 0.f, 0.f};
-  // entries of a covering chunk outside the row are zeros, whose terms are exact (rho = 1): they
-  // add 1 each to the first two sums, taken off again below
+  auto term = [&](float x) {
+    float rho, rho7, r;
+    octic7(x, rho, rho7, r);
+    s[0] = __builtin_fmaf(rho7, rho, s[0]);
+    s[1] += rho7;
+    const float m = (r * x) * rho7;
+    s[2] = __builtin_fmaf(m, rho, s[2]);
+    s[3] += m;
+  };
   auto eval = [&](u32x4_t w) {
     float v[R::EPC];
     R::unpack(w, v);
 #pragma unroll
-    for (int i = 0; i < R::EPC; ++i) {
-      const float x = v[i] * tau;
-      float rho, rho7, r;
-      octic7(x, rho, rho7, r);
-      s[0] = __builtin_fmaf(rho7, rho, s[0]);
-      s[1] += rho7;
-      const float m = (r * x) * rho7;
-      s[2] = __builtin_fmaf(m, rho, s[2]);
-      s[3] += m;
-    }
+    for (int i = 0; i < R::EPC; ++i) term(v[i] * tau);
   };
   if constexpr (NCH > 0) {
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
       asm("" : "+v"(raw[j]));  // unpack again here: the first pass's floats would take twice the registers
-      if (tid + T * j < nch) eval(raw[j]);
+      if (tid + T * j < sp.body) eval(raw[j]);
       __builtin_amdgcn_sched_barrier(0);  // one chunk's terms live at a time
     }
   } else {
-    for (int c = tid; c < nch; c += T) eval(R::load(zr, c * R::EPC - lead, V));
+    for (int c = tid; c < sp.body; c += T) eval(body[c]);
   }
+  if (edge >= 0) term(ve * tau);
 #pragma unroll
   for (int q = 0; q < 4; ++q) s[q] = wave_sum(s[q]);
   if constexpr (NW > 1) {
@@ -214,7 +217,6 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
     }
   }
   if (tid == 0) {
-    const float pad = (float)(nch * R::EPC - V);
     const int64_t t = targets[row];
     float rho_t = 0.f, rn_t = 0.f;  // a target outside [0, V) leaves rho_t = 0 (loss = inf), as the reference
     if (t >= 0 && t < V) {
@@ -223,8 +225,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
       rho_t = o.rho;
       rn_t = o.r * x;
     }
-    oace_finalize_row<float>(rows + row * OACE_ROW, tau, s[0] - pad, s[1] - pad, s[2], s[3], rho_t, rn_t, inv_v,
-                             gamma);
+    oace_finalize_row<float>(rows + row * OACE_ROW, tau, s[0], s[1], s[2], s[3], rho_t, rn_t, inv_v, gamma);
   }
 }
 
@@ -459,7 +460,7 @@ void w_strides(const OaceArgs& a, int64_t& sk, int64_t& sv) {
 // longer rows are streamed.
 template <int DT>
 void rows_fwd_vec(const OaceArgs& a, const void* z, int64_t ldz, void* rows, hipStream_t st) {
-  const int nch = RowChunk<DT>::count_max((int)a.V);
+  const int nch = (int)a.V / RowChunk<DT>::EPC;  // whole chunks of the best start
   const float inv_v = (float)(1.0 / (double)a.V);
 #define OACE_ROWS_VEC(T, NCH)                                                                                       \
   hipLaunchKernelGGL((oace_rows_fwd_vec_kernel<DT, T, NCH>), dim3((unsigned)((a.N * T + (T < 256 ? 255 : T - 1)) /  \

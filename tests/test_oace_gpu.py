@@ -408,3 +408,33 @@ def test_head_read_in_place_equals_its_aligned_copy(shape, dtype):
         dh2, dw2 = _grads(cache2, 1.0)
         assert float(loss2) == float(loss), (off, ld)
         assert torch.equal(cache2[3], cache[3]) and torch.equal(dh2, dh) and torch.equal(dw2, dw), (off, ld)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [1, 2, 3, 5, 9, 15, 17, 65, 129, 1031])
+def test_softmax_loss_small_row_sums(dtype, V):
+    """Row records of negative logits, whose octic sum (V terms near 9e-4) is far below the 1 that an
+    entry outside the row would add to it, from every start of a row against the fp64 kernel.  Bounds as
+    test_algebraic_softmax_small_row_sums: 3.3e-6 for a weight and for the sums; the target's is one of
+    them, so p_target^(-1/8), S^(1/8) and sum p^(7/8) are within 3.3e-6 (1 + 7/8) of theirs, and the loss
+    within that of its terms."""
+    N = 16
+    rng = np.random.default_rng(V)
+    z = _t(-60.0 - rng.random((N, V)), dtype)
+    t = torch.from_numpy(rng.integers(0, V, size=N)).to(DEV)
+    stream = _lib.stream_ptr(z.device)
+
+    def records(x):
+        acc = _lib.accum_dtype(x.dtype)
+        loss, rec = torch.empty((), dtype=acc, device=DEV), torch.empty((N, A.oace.ROW_FIELDS), dtype=acc, device=DEV)
+        _lib.check(_lib.lib().oace_softmax_loss_fwd(_lib.dtype_code(x.dtype), N, V, x.data_ptr(), t.data_ptr(), 100.0, 2.0,
+                                                    loss.data_ptr(), rec.data_ptr(), stream), "oace_softmax_loss_fwd")
+        return rec.double()
+
+    ref = records(z.double())
+    for start in range(0, 16 // z.element_size(), 3):
+        got = records(torch.empty(N * V + start, dtype=dtype, device=DEV)[start:].view(N, V).copy_(z))
+        for f in range(5):  # tau, 1/S, S^(1/8), sum p^(7/8), p_target^(-1/8)
+            assert ((got[:, f] - ref[:, f]).abs() <= 6.2e-6 * ref[:, f].abs()).all(), (start, f)
+        terms = 2.0 * (8.0 * ref[:, 4] + 8.0 / 7.0 * ref[:, 3])
+        assert ((got[:, 6] - ref[:, 6]).abs() <= 6.2e-6 * terms).all(), start
