@@ -438,3 +438,26 @@ def test_softmax_loss_small_row_sums(dtype, V):
             assert ((got[:, f] - ref[:, f]).abs() <= 6.2e-6 * ref[:, f].abs()).all(), (start, f)
         terms = 2.0 * (8.0 * ref[:, 4] + 8.0 / 7.0 * ref[:, 3])
         assert ((got[:, 6] - ref[:, 6]).abs() <= 6.2e-6 * terms).all(), start
+
+
+@pytest.mark.parametrize("N,V,dtype", [(700, 12289, torch.bfloat16), (700, 12289, torch.float16),
+                                       (1400, 3075, torch.float32)])
+def test_softmax_loss_many_chunks_per_lane(N, V, dtype):
+    """dz of enough rows that a lane takes four chunks of a row: several spans per row, ragged rows of
+    every start, and targets in each of the four chunk positions, on both sides of a span's edge and at
+    both ends of the row; against the fp64 kernel, tolerances as test_softmax_loss_row_kernels."""
+    rng = np.random.default_rng(V)
+    z = _t(rng.standard_normal((N, V)) * 10.0, dtype).requires_grad_(True)
+    t = rng.integers(0, V, size=N)
+    epc = 16 // z.element_size()
+    edges = [c * 64 * epc + o for c in range(V // (64 * epc) + 1) for o in (-epc, -1, 0, 1, epc)] + [0, 1, V - 2, V - 1]
+    edges = [e for e in edges if 0 <= e < V]
+    t[:len(edges)] = edges
+    t = torch.from_numpy(t).to(DEV)
+    g = 1024.0
+    (dz,) = torch.autograd.grad(A.fused_oace_softmax_loss(z, t) * g, z)
+    zd = z.detach().double().requires_grad_(True)
+    (ref,) = torch.autograd.grad(A.fused_oace_softmax_loss(zd, t) * g, zd)
+    tol = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
+    err = (dz.double() - ref).abs()
+    assert (err.amax(-1) <= tol * ref.abs().amax(-1)).all()  # every row by itself
