@@ -15,7 +15,8 @@
 //   * afa_bwd_f32_dkdv_kernel: one lane per key, the mirror image: k and v planes in registers,
 //     S = Q K^T and dP = g V^T from Q / g rows in LDS, then dV^T += g^T W and dK^T += Q^T dS.
 // Tiles of 32 rows are staged through registers, rotated and split there, into double-buffered LDS
-// (one barrier per tile); dq and dk are rotated back through R^T before they are stored.
+// (one barrier per tile); dq and dk are rotated back through R^T before they are stored.  Waves that met
+// an operand the planes do not hold take their rows again in plain fp32 (afa_f32_split.h).
 #include "afa_common.h"
 #include "afa_f32_split.h"
 #include "afa_launch.h"
@@ -278,6 +279,33 @@ void afa_bwd_f32_dq_kernel(const GenArgs a) {
     __syncthreads();
   }
 
+  if (f32_any_nan(dq)) {
+    const float* gp = (const float*)a.g + base;
+    const float* qp = (const float*)a.q + base;
+    F32Look look;
+    look.rows<D>(qp + (int64_t)q0_w * D, D, min(32, L - q0_w));
+    look.rows<D>(gp + (int64_t)q0_w * D, D, min(32, L - q0_w));
+    look.rows<D>(kp, D, kend_w);
+    look.rows<D>(vp, D, kend_w);
+    look.big |= __builtin_isinf(ei);
+    if (look.redo()) {
+      f32x4_t qo[D / 8], go[D / 8];
+      f32_half_row<D, ROT>(qp + (int64_t)min(qi, L - 1) * D, rc, rs, min(qi, L - 1), qo);
+      f32_half_row<D, false>(gp + (int64_t)min(qi, L - 1) * D, nullptr, nullptr, 0, go);
+      f32_clear(dq);
+#pragma unroll 1
+      for (int j = 0; j < kend_w; ++j) {
+        f32x4_t kr[D / 8], vr[D / 8];
+        f32_half_row<D, ROT>(kp + (int64_t)j * D, rc, rs, j, kr);
+        f32_half_row<D, false>(vp + (int64_t)j * D, nullptr, nullptr, 0, vr);
+        const float s = f32_half_dot(qo, kr) * scale, p = f32_half_dot(go, vr);
+        float rr;
+        const float w = frho8r(s, rr) * invd;
+        if (qi < L && (!a.causal || j <= qi)) f32_half_axpy(c8 * rr * w * (p - ei), kr, dq);
+      }
+    }
+  }
+
   if (qi < L) {
     float* op = (float*)a.out + base + (int64_t)qi * D;
 #pragma unroll
@@ -432,6 +460,39 @@ void afa_bwd_f32_dkdv_kernel(const GenArgs a) {
     }
     if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
+  }
+
+  if (f32_any_nan(dk) || f32_any_nan(dv)) {
+    const float* kp = (const float*)a.k + base;
+    const float* vp = (const float*)a.v + base;
+    const int i0 = a.causal ? k0_w : 0;  // a NaN: the wave is live, k0_w < L
+    F32Look look;
+    look.rows<D>(kp + (int64_t)k0_w * D, D, min(32, L - k0_w));
+    look.rows<D>(vp + (int64_t)k0_w * D, D, min(32, L - k0_w));
+    look.rows<D>(qp + (int64_t)i0 * D, D, L - i0);
+    look.rows<D>(gp + (int64_t)i0 * D, D, L - i0);
+#pragma unroll 1
+    for (int i = i0 + lane; i < L; i += 64) look.big |= __builtin_isinf(ep[i]);
+    if (look.redo()) {
+      f32x4_t ko[D / 8], vo[D / 8];
+      f32_half_row<D, ROT>(kp + (int64_t)min(kj, L - 1) * D, rc, rs, min(kj, L - 1), ko);
+      f32_half_row<D, false>(vp + (int64_t)min(kj, L - 1) * D, nullptr, nullptr, 0, vo);
+      f32_clear(dk);
+      f32_clear(dv);
+#pragma unroll 1
+      for (int i = i0; i < L; ++i) {
+        f32x4_t qr[D / 8], gr[D / 8];
+        f32_half_row<D, ROT>(qp + (int64_t)i * D, rc, rs, i, qr);
+        f32_half_row<D, false>(gp + (int64_t)i * D, nullptr, nullptr, 0, gr);
+        const float s = f32_half_dot(ko, qr) * scale, p = f32_half_dot(vo, gr);
+        float rr;
+        const float w = frho8r(s, rr) * ip[i];
+        if (kj < vlen && (!a.causal || kj <= i)) {
+          f32_half_axpy(c8 * rr * w * (p - ep[i]), qr, dk);
+          f32_half_axpy(w, gr, dv);
+        }
+      }
+    }
   }
 
   if (kj < L) {

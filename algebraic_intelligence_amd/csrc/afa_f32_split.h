@@ -4,7 +4,8 @@
 //   x y = hi hi' + (hi mid' + mid hi') + (mid mid' + hi lo' + lo hi') + terms below 2^-23 |x y|,
 // six products of the bf16 matrix cores, accumulated in fp32.  They run at 16 times the fp32 rate:
 // 2.7 times after six passes, and one fp32 rounding serves 16 of the contraction where the fp32
-// MFMA's serves two.
+// MFMA's serves two.  Below about 2^-110 the lower planes reach bf16's subnormals (steps of 2^-133) and
+// fewer bits of a value are held.
 #pragma once
 
 #include "afa_common.h"
@@ -21,8 +22,8 @@ __device__ __forceinline__ void split3_rne(float x0, float x1, unsigned& hi, uns
   lo = pack_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));
 }
 
-// Planes of four values whose infinities must come out of the product as infinities (v, and the
-// cotangent): hi is rounded towards zero, so it cannot overflow, and an infinity, which the planes
+// Planes of four values whose infinities must come out of the product as infinities (the forward's
+// v): hi is rounded towards zero, so it cannot overflow, and an infinity, which the planes
 // of the other operand (zeros and both signs) would turn into NaN, leaves zeros and returns true:
 // its terms are added by inf_terms.
 __device__ __forceinline__ bool split3_trunc(f32x4_t x, unsigned (&w)[3][2]) {
@@ -170,6 +171,90 @@ __device__ __forceinline__ f32x4_t f32_rotate4(f32x4_t x, const float* c, const 
     y[2 * p + 1] = s[p] * x[2 * p] + c[p] * x[2 * p + 1];
   }
   return y;
+}
+
+// ------------------------------------------------------------------ rows redone in fp32
+// An infinite operand, or one that rounds past the largest bf16, leaves NaN in its lower planes and so
+// in every product that meets it, where the fp32 product is an infinity or finite.  A wave whose sums hold a NaN
+// looks its operands over once its tiles are done and, unless NaN operands account for it, takes its
+// rows again in plain fp32: nothing is paid in the tiles, and the second pass reads one row of the other
+// side at a time (about ten times the work of the tiles it replaces).
+
+// Any NaN among a wave's sums (an infinite sum counts too: 0 times it is NaN).
+template <int N>
+__device__ __forceinline__ bool f32_any_nan(const f32x16_t (&acc)[N]) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) t = __builtin_fmaf(acc[i][e], 0.f, t);
+  return __ballot(t != t) != 0;
+}
+
+// What a wave has seen of its operands: a NaN; a value that planes do not hold.
+struct F32Look {
+  bool nan = false, big = false;
+  __device__ __forceinline__ void add(float x) {
+    nan |= x != x;
+    big |= __builtin_fabsf(x) > 3.38953138925153547590e38f;  // the largest bf16
+  }
+  // rows [0, n) of D features, row stride ld, dword aligned
+  template <int D>
+  __device__ __forceinline__ void rows(const float* p, int64_t ld, int n) {
+    typedef f32x4_t f32x4_dword_t __attribute__((aligned(4)));
+#pragma unroll 1
+    for (int i = threadIdx.x & 63; i < n * (D / 4); i += 64) {
+      const f32x4_t x = *(const f32x4_dword_t*)(p + (int64_t)(i / (D / 4)) * ld + 4 * (i % (D / 4)));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(x[u]);
+    }
+  }
+  __device__ __forceinline__ bool redo() const { return __ballot(big) != 0 || __ballot(nan) == 0; }
+};
+
+// The features of one row that a lane holds in the accumulators, 8 c + 4 g .. + 3 (rotated when ROT).
+template <int D, bool ROT>
+__device__ __forceinline__ void f32_half_row(const float* row, const float* rc, const float* rs, int pos,
+                                             f32x4_t (&x)[D / 8]) {
+  typedef f32x4_t f32x4_dword_t __attribute__((aligned(4)));
+  const int g = (threadIdx.x >> 5) & 1;
+#pragma unroll
+  for (int c = 0; c < D / 8; ++c) {
+    const int m = 8 * c + 4 * g;
+    x[c] = *(const f32x4_dword_t*)(row + m);
+    if constexpr (ROT) {
+      const int64_t t = (int64_t)pos * (D / 2) + m / 2;
+      x[c] = f32_rotate4(x[c], rc + t, rs + t);
+    }
+  }
+}
+
+// The dot product of two such rows, both lanes' halves.
+template <int N>
+__device__ __forceinline__ float f32_half_dot(const f32x4_t (&x)[N], const f32x4_t (&y)[N]) {
+  float s = 0.f;
+#pragma unroll
+  for (int c = 0; c < N; ++c)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s = __builtin_fmaf(x[c][u], y[c][u], s);
+  return s + __shfl_xor(s, 32);
+}
+
+// acc += w x for such a row x.
+template <int N, int NDB>
+__device__ __forceinline__ void f32_half_axpy(float w, const f32x4_t (&x)[N], f32x16_t (&acc)[NDB]) {
+#pragma unroll
+  for (int c = 0; c < N; ++c)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[c >> 2][4 * (c & 3) + u] = __builtin_fmaf(w, x[c][u], acc[c >> 2][4 * (c & 3) + u]);
+}
+
+template <int N>
+__device__ __forceinline__ void f32_clear(f32x16_t (&acc)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
 }
 
 }  // namespace afa

@@ -428,3 +428,56 @@ def test_f32_planes_strides_and_infinities(D, L, causal, valid, rot):
     gen, _ = _fwd(q, k, v, causal=False, valid=valid, rotary=rotary, flags=_lib.FLAG_GENERIC)
     bad = ~torch.isfinite(gen)
     assert bad[0, 1, :, 5].all() and torch.equal(bad, ~torch.isfinite(out)) and torch.equal(out[bad], gen[bad])
+
+
+def _bwd_f32(q, k, v, out, den, g, causal, rotary, flags):
+    B, H, L, D = q.shape
+    dq, dk, dv = (torch.empty_like(q) for _ in range(3))
+    lib = _lib.lib()
+    ws_bytes = lib.afa_bwd_workspace_size(_lib.dtype_code(q.dtype), B, H, L, D, int(rotary is not None))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    c, s, n = (None, None, 0) if rotary is None else (rotary.c, rotary.s, rotary.c.shape[0])
+    rc = lib.afa_bwd(_lib.dtype_code(q.dtype), B, H, L, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out),
+                     _lib.ptr(den), _lib.ptr(g), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(c), _lib.ptr(s), n,
+                     0.5, int(causal), 0, flags, _lib.ptr(ws), ws_bytes, _lib.stream_ptr(q.device))
+    _lib.check(rc, "afa_bwd")
+    return dq, dk, dv
+
+
+@pytest.mark.parametrize("D", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("L", [31, 33, 160, 300])
+@pytest.mark.parametrize("case", ["g", "g_past_bf16", "v", "k_past_bf16", "E", "nan"])
+def test_f32_backward_infinities(D, L, case):
+    """The fp32 backward where an operand has no bf16 planes (an infinity, a value that rounds past the
+    largest bf16, a row's E that overflows): infinite, NaN and finite results where the generic
+    fp32 kernels have them, within the rounding of both (2e-5 of a feature's largest entry, and 2^-126: an
+    operand near 1e-38 has subnormal planes, steps of 2^-133, and at most 300 terms); and NaN inputs NaN
+    as there."""
+    q, k, v = make_qkv((1, 2, L, D), torch.float32, seed=L + D)
+    g = make_qkv((1, 2, L, D), torch.float32, seed=L)[0]
+    rot = A.build_cayley_rotary_matrix(D, L) if D == 64 and case != "k_past_bf16" else None
+    j = L // 2
+    if case == "v":
+        v[0, 1, j, 5] = float("-inf")
+    if case == "k_past_bf16":
+        q[0, 1, :, 3], k[0, 1, j, 3] = 1e-38, 3.4e38
+    out, den = _fwd(q, k, v, rotary=rot, flags=_lib.FLAG_GENERIC)
+    if case == "g":
+        g[0, 1, j, 2] = float("inf")
+    if case == "g_past_bf16":
+        g[0, 1, j, 2], v[0, 1, :, 2], out[0, 1, j, 2] = 3.4e38, 1e-38, 1e-38
+    if case == "E":
+        g[0, 0, j, 4], out[0, 0, j, 4] = 1e38, 1e10
+    if case == "nan":
+        g[0, 1, j, 2] = float("nan")
+    got = _bwd_f32(q, k, v, out, den, g, False, rot, 0)
+    want = _bwd_f32(q, k, v, out, den, g, False, rot, _lib.FLAG_GENERIC)
+    for name, x, y in zip(("dq", "dk", "dv"), got, want):
+        bad = ~torch.isfinite(y)
+        assert torch.equal(bad, ~torch.isfinite(x)), name
+        assert torch.equal(x[bad].nan_to_num(9e9), y[bad].nan_to_num(9e9)), name
+        xf, yf = x.masked_fill(bad, 0.0).double(), y.masked_fill(bad, 0.0).double()
+        scale = yf.abs().amax(2, keepdim=True)
+        assert ((xf - yf).abs() <= 2e-5 * scale + 2.0 ** -126).all(), name
+    if case == "g":  # the feature's dv is infinite and nothing else of it is lost
+        assert torch.isinf(got[2][0, 1, :, 2]).all() and torch.isfinite(got[2][0, 0]).all()
