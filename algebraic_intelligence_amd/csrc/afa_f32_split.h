@@ -13,66 +13,13 @@
 namespace afa {
 
 // Planes of a pair, packed.  Rounded to nearest: the dropped terms are at most 2^-24 |x y|.  An
-// infinity, or a value that rounds past the largest bf16, gives a NaN in the lower planes: for
-// operands whose infinite products already end as NaN (scores: rho of an infinite score is NaN).
+// infinity, or a value that rounds past the largest bf16, gives a NaN in the lower planes (rows redone in
+// fp32, below).
 __device__ __forceinline__ void split3_rne(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
   hi = pack_bf16(x0, x1);
   const float r0 = x0 - bf16_lo(hi), r1 = x1 - bf16_hi(hi);
   mid = pack_bf16(r0, r1);
   lo = pack_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));
-}
-
-// Planes of four values whose infinities must come out of the product as infinities (the forward's
-// v): hi is rounded towards zero, so it cannot overflow, and an infinity, which the planes
-// of the other operand (zeros and both signs) would turn into NaN, leaves zeros and returns true:
-// its terms are added by inf_terms.
-__device__ __forceinline__ bool split3_trunc(f32x4_t x, unsigned (&w)[3][2]) {
-  const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])),
-                                  __builtin_fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])));
-  const bool inf = m == __builtin_inff();
-  if (inf) {
-    asm volatile("" ::: "memory");  // keeps the rare case a branch
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = __builtin_isinf(x[i]) ? 0.f : x[i];
-  }
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const float x0 = x[2 * p], x1 = x[2 * p + 1];
-    const unsigned u0 = __builtin_bit_cast(unsigned, x0), u1 = __builtin_bit_cast(unsigned, x1);
-    w[0][p] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-    const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xffff0000u);
-    const float r1 = x1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
-    w[1][p] = pack_bf16(r0, r1);
-    w[2][p] = pack_bf16(r0 - bf16_lo(w[1][p]), r1 - bf16_hi(w[1][p]));
-  }
-  return inf;
-}
-
-// The terms of infinite elements of one 32-row tile x (row stride ld, `rows` rows of it exist):
-// acc[db][e] += p[row] x[row][feature] over
-// the infinite x, p in accumulator order (element e of lane group g is row 8 (e >> 2) + 4 g +
-// (e & 3)) and acc as the transposed product leaves it.  Reached only by tiles that hold an infinity.
-template <int D, int NDB>
-__device__ __forceinline__ void inf_terms(const float* x, int64_t ld, int rows, const float (&p)[16],
-                                          f32x16_t (&acc)[NDB]) {
-  const int g = (threadIdx.x >> 5) & 1;
-#pragma unroll 1
-  for (int r = 0; r < min(32, rows); ++r) {
-    float mine = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) mine = e == 4 * (r >> 3) + (r & 3) ? p[e] : mine;
-    const float other = __shfl_xor(mine, 32);
-    const float pr = ((r >> 2) & 1) == g ? mine : other;
-    const float* row = x + (int64_t)r * ld;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int f = db * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
-        const float v = f < D ? row[f] : 0.f;
-        if (__builtin_isinf(v)) acc[db][e] += pr * v;
-      }
-  }
 }
 
 // acc += A B over 16 of the contraction, both operands as planes; smallest terms first.

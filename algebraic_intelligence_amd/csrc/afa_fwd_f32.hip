@@ -3,9 +3,9 @@
 // (q . k) scale in fp32, w = rho(s)^8 by the cancellation-safe two-branch form, out = sum_j w v_j /
 // (sum_j w + Omega), d = sum_j w + Omega; only the order of the fp32 additions differs.
 //
-// Every fp32 operand of the two products is split exactly into three bf16 planes (F32Planes in
-// afa_f32_split.h) and a product is the six plane products of at least 2^-16 relative weight,
-// accumulated in fp32: 2.7 times the rate of v_mfma_f32_32x32x2_f32 for both products.
+// Every fp32 operand of the two products is split exactly into three bf16 planes (afa_f32_split.h)
+// and a product is the six plane products of at least 2^-16 relative weight, accumulated in fp32: 2.7
+// times the rate of v_mfma_f32_32x32x2_f32 for both products.
 //
 // A wave owns 32 queries; a unit is 32 keys x 32 queries.
 //   S^T = K Q^T: 32x32x16 steps over head_dim, the query planes in registers, K planes read as
@@ -55,7 +55,6 @@ void afa_fwd_f32_kernel(const FwdArgs a) {
   constexpr bool RAGGED = KT * (D / 4) % 256 != 0;  // head_dim 48: the last job is half a workgroup's
   __shared__ __attribute__((aligned(16))) unsigned short ks[2][3 * X::PLANE];
   __shared__ __attribute__((aligned(16))) unsigned short vs[2][3 * X::PLANE];
-  __shared__ int vinf[2];  // the tile in each buffer if it holds an infinite v, else not
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -138,7 +137,8 @@ void afa_fwd_f32_kernel(const FwdArgs a) {
       split3_rne(y[0], y[1], w[0][0], w[1][0], w[2][0]);
       split3_rne(y[2], y[3], w[0][1], w[1][1], w[2][1]);
       X::put(ks[buf], X::at(r, c), w);
-      if (split3_trunc(vx[i], w)) vinf[buf] = t;
+      split3_rne(vx[i][0], vx[i][1], w[0][0], w[1][0], w[2][0]);
+      split3_rne(vx[i][2], vx[i][3], w[0][1], w[1][1], w[2][1]);
       X::put(vs[buf], X::at(r, c), w);
     }
   };
@@ -177,8 +177,6 @@ void afa_fwd_f32_kernel(const FwdArgs a) {
     for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
   float dsum = 0.f;
 
-  if (tid < 2) vinf[tid] = -1;
-  __syncthreads();
   if (t_beg < ntiles) store(t_beg);
   __syncthreads();
   for (int t = t_beg; t < ntiles; ++t) {
@@ -237,12 +235,38 @@ void afa_fwd_f32_kernel(const FwdArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[db][e] += ot[e];
       }
-      if (__builtin_amdgcn_readfirstlane(vinf[t & 1]) == t)
-        inf_terms<D, NDB>(vp + (int64_t)t * KT * a.v_l, a.v_l, L - t * KT, w, o);
     }
     // the buffer of tile t+1 was last read in tile t-1, before the previous barrier
     if (t + 1 < ntiles) store(t + 1);
     __syncthreads();
+  }
+
+  if (f32_any_nan(o)) {  // a NaN: the wave has queries, q0_w < L
+    const int key0 = t_beg * KT, key1 = min(kend_w, ntiles * KT);
+    F32Look look;
+    look.rows<D>(qp + (int64_t)q0_w * a.q_l, a.q_l, min(32, L - q0_w));
+    look.rows<D>(kp + (int64_t)key0 * a.k_l, a.k_l, key1 - key0);
+    look.rows<D>(vp + (int64_t)key0 * a.v_l, a.v_l, key1 - key0);
+    if (look.redo()) {
+      f32x4_t qo[D / 8];
+      f32_half_row<D, ROT>(qp + (int64_t)min(qi, L - 1) * a.q_l, a.rc, a.rs, min(qi, L - 1), qo);
+#pragma unroll
+      for (int c = 0; c < D / 8; ++c) qo[c] *= a.q_scale;
+      f32_clear(o);
+      dsum = 0.f;
+#pragma unroll 1
+      for (int j = key0; j < key1; ++j) {
+        f32x4_t kr[D / 8], vr[D / 8];
+        f32_half_row<D, ROT>(kp + (int64_t)j * a.k_l, a.rc, a.rs, j, kr);
+        f32_half_row<D, false>(vp + (int64_t)j * a.v_l, nullptr, nullptr, 0, vr);
+        const float s = f32_half_dot(qo, kr);
+        const float w = rho8_exact(D == 64 ? s : s * a.s_mult);
+        if (qi < L && (!a.causal || j <= qi)) {
+          f32_half_axpy(w, vr, o);
+          if (g == 0) dsum += w;
+        }
+      }
+    }
   }
 
   dsum += __shfl_xor(dsum, 32);

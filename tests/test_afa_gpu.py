@@ -481,3 +481,32 @@ def test_f32_backward_infinities(D, L, case):
         assert ((xf - yf).abs() <= 2e-5 * scale + 2.0 ** -126).all(), name
     if case == "g":  # the feature's dv is infinite and nothing else of it is lost
         assert torch.isinf(got[2][0, 1, :, 2]).all() and torch.isfinite(got[2][0, 0]).all()
+
+
+@pytest.mark.parametrize("D", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("B,L", [(1, 31), (1, 160), (1, 700), (40, 300)])
+@pytest.mark.parametrize("case", ["k", "v", "v_inf", "nan"])
+def test_f32_forward_values_without_planes(D, B, L, case):
+    """The fp32 forward, whole and with split key ranges, where an operand rounds past the largest bf16 or is
+    infinite: finite and infinite results where the generic fp32 kernel has them, within the rounding of
+    both (2e-5 of a row's largest entry); and NaN inputs NaN as there."""
+    q, k, v = make_qkv((B, 2, L, D), torch.float32, seed=L + D)
+    rot = A.build_cayley_rotary_matrix(D, L) if D == 64 and case in ("v_inf", "nan") else None
+    j = L // 2
+    if case == "k":
+        q[0, 1, :, 3], k[0, 1, j, 3] = 1e-38, -3.4e38
+    if case == "v":  # scores of key j below 0: weights below 1, so that no product overflows
+        q[0, 1], k[0, 1, j], v[0, 1, j, 2] = q[0, 1].abs(), -k[0, 1, j].abs(), 3.4e38
+    if case == "v_inf":
+        v[0, 1, j, 2] = float("inf")
+    if case == "nan":
+        k[0, 1, j, 2] = float("nan")
+    out, den = _fwd(q, k, v, rotary=rot)
+    want, wden = _fwd(q, k, v, rotary=rot, flags=_lib.FLAG_GENERIC)
+    bad = ~torch.isfinite(want)
+    assert bad.any() == (case in ("v_inf", "nan"))
+    assert torch.equal(bad, ~torch.isfinite(out)) and torch.equal(torch.isnan(den), torch.isnan(wden))
+    assert torch.equal(out[bad].nan_to_num(9e9), want[bad].nan_to_num(9e9))
+    x, y = out.masked_fill(bad, 0.0).double(), want.masked_fill(bad, 0.0).double()
+    assert ((x - y).abs() <= 2e-5 * y.abs().amax(2, keepdim=True)).all()
+    assert (den.double() - wden.double()).abs().nan_to_num(0.0).amax() <= 2e-5 * wden.nan_to_num(0.0).amax()
