@@ -365,7 +365,8 @@ namespace {
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 int64_t up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
-constexpr size_t Z_MAX_BYTES = (size_t)256 << 20;  // fp32 logits held at a time
+// Logits held at a time, 4 bytes each; their dz, 6 bytes each (three planes), come on top.
+constexpr size_t Z_MAX_BYTES = (size_t)256 << 20;
 constexpr size_t W_MAX_BYTES = (size_t)8 << 30;    // planes of the weights
 constexpr int DH_ITEMS = 256;  // workgroups of dh's split contraction: fixed, so the sum order is
 
@@ -383,12 +384,14 @@ int64_t tiles(int64_t m, int64_t n, int wm) {
 // The tile orientation that covers m x n with fewer tiles (equal areas), 256 x 128 on a tie.
 bool wide_m(int64_t m, int64_t n) { return tiles(m, n, 4) <= tiles(m, n, 2); }
 
+int64_t rows_that_fit(const OaceArgs& a) { return (int64_t)(Z_MAX_BYTES / ((size_t)up(a.V, 64) * 4)); }
+
 Plan plan_of(const OaceArgs& a) {
   Plan p;
   p.dp = up(a.d, 64);
   p.Vp = up(a.V, 64);
-  const int64_t fit = (int64_t)(Z_MAX_BYTES / ((size_t)p.Vp * 4)) / 256 * 256;
-  p.R = std::min<int64_t>(a.N, std::max<int64_t>(256, fit));
+  const int64_t fit = rows_that_fit(a);  // at least XK: oace_f32_supported
+  p.R = std::min<int64_t>(a.N, fit >= 256 ? fit / 256 * 256 : fit / XK * XK);
   p.Rp = up(p.R, XK);
   p.wr = a.w_layout == OACE_W_DV ? p.dp : p.Vp;
   p.wc = a.w_layout == OACE_W_DV ? p.Vp : p.dp;
@@ -455,8 +458,8 @@ hipError_t z_gemm(const OaceArgs& a, const Plan& p, const unsigned short* wp, co
 }  // namespace
 
 bool oace_f32_supported(const OaceArgs& a) {
-  // 32-bit lane offsets (256 rows of a plane) and 32-bit extents
-  if (a.N > (1 << 28) || a.V >= (1 << 22) || a.d >= (1 << 22)) return false;
+  // 32-bit lane offsets (256 rows of a plane) and 32-bit extents; a chunk is at least one step of rows
+  if (a.N > (1 << 28) || rows_that_fit(a) < XK || a.d >= (1 << 22)) return false;
   return (size_t)up(a.d, 64) * up(a.V, 64) * 6 <= W_MAX_BYTES;
 }
 
