@@ -365,7 +365,8 @@ namespace {
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 int64_t up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
-// Logits held at a time, 4 bytes each; their dz, 6 bytes each (three planes), come on top.
+// Logits held at a time, 4 bytes each; their dz, 6 bytes each (three planes), come on top, and within it
+// when the caller asks for none to be kept (OACE_FLAG_RECOMPUTE_Z).
 constexpr size_t Z_MAX_BYTES = (size_t)256 << 20;
 constexpr size_t W_MAX_BYTES = (size_t)8 << 30;    // planes of the weights
 constexpr int DH_ITEMS = 256;  // workgroups of dh's split contraction: fixed, so the sum order is
@@ -384,7 +385,8 @@ int64_t tiles(int64_t m, int64_t n, int wm) {
 // The tile orientation that covers m x n with fewer tiles (equal areas), 256 x 128 on a tie.
 bool wide_m(int64_t m, int64_t n) { return tiles(m, n, 4) <= tiles(m, n, 2); }
 
-int64_t rows_that_fit(const OaceArgs& a) { return (int64_t)(Z_MAX_BYTES / ((size_t)up(a.V, 64) * 4)); }
+bool keeps_z(const OaceArgs& a) { return (a.flags & OACE_FLAG_RECOMPUTE_Z) == 0; }
+int64_t rows_that_fit(const OaceArgs& a) { return (int64_t)(Z_MAX_BYTES / ((size_t)up(a.V, 64) * (keeps_z(a) ? 4 : 10))); }
 
 Plan plan_of(const OaceArgs& a) {
   Plan p;
@@ -499,7 +501,7 @@ hipError_t oace_linear_bwd_f32(const OaceArgs& a, const void* rows, void* ws, hi
   if (h_ready) hj.prows = 0;
   hipError_t e = split_launch(wj, hj, st);
   if (e != hipSuccess) return e;
-  const bool z_ready = h_ready && p.R == a.N;
+  const bool z_ready = h_ready && p.R == a.N && keeps_z(a);
   const float c0 = (float)(8.0 * a.gamma / (double)a.N);
   const int64_t h_plane = up(a.N, XK) * p.dp;
   for (int64_t r0 = 0; r0 < a.N; r0 += p.R) {

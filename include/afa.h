@@ -234,8 +234,9 @@ int ago_rotate_qk(int dtype, int64_t outer, int64_t seq_len, int64_t inner, int6
    formed elementwise instead of by a second GEMM.  No counterpart in the reference. */
 #define OACE_FLAG_Z_READY 0x20u
 /* oace_workspace_size / oace_linear_fwd / oace_linear_bwd (the same on all three): never keep
-   the logits; the backward recomputes them (a workspace of O(rows x d_model + vocab x d_model)).
-   No counterpart in the reference. */
+   the logits; the backward recomputes them.  Beside the copy or planes of h and w the workspace then
+   holds at most 256 MB of logits (fp32: and of their gradient), and partial sums; bf16/fp16: the
+   gradient of every logit, 2 bytes each.  No counterpart in the reference. */
 #define OACE_FLAG_RECOMPUTE_Z 0x40u
 size_t oace_workspace_size(int dtype, int64_t rows, int64_t d_model, int64_t vocab, int w_layout,
                            unsigned flags);

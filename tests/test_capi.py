@@ -234,13 +234,17 @@ def test_oace_rejects_invalid_arguments(lib):
 @pytest.mark.parametrize("layout", [0, 1])
 def test_oace_f32_workspace_bounds(rows, d, vocab, layout):
     """The fp32 head's workspace beside its planes (6 bytes per padded element of h and w) and row records:
-    at most 256 MB of logits, and 384 MB of their gradient's planes; partial sums of at most 256 tiles of
-    256 x 128 floats."""
+    at most 256 MB of logits, and 384 MB of their gradient's planes; 256 MB for both where no logits
+    are to be kept (OACE_FLAG_RECOMPUTE_Z); partial sums of at most 256 tiles of 256 x 128 floats."""
     up = lambda n, m: (n + m - 1) // m * m
     mb = 1 << 20
     size = lambda flags: _lib.lib().oace_workspace_size(_lib.AFA_F32, rows, d, vocab, layout, flags)
     planes = 6 * up(d, 64) * (up(vocab, 64) + up(rows, 32)) + up(rows * 32, 256)
-    assert size(0) <= planes + (256 + 384 + 32) * mb + 4096
+    kept, recomputed = size(0), size(0x40)
+    assert kept <= planes + (256 + 384 + 32) * mb + 4096
+    assert recomputed <= planes + (256 + 32) * mb + 4096
+    if rows * vocab * 10 > 256 * mb and vocab <= 1 << 21:
+        assert recomputed < kept
 
 
 def test_python_constants_match_the_header():

@@ -461,3 +461,23 @@ def test_softmax_loss_many_chunks_per_lane(N, V, dtype):
     tol = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
     err = (dz.double() - ref).abs()
     assert (err.amax(-1) <= tol * ref.abs().amax(-1)).all()  # every row by itself
+
+
+@pytest.mark.parametrize("shape", [(130, 96, 1000), (1100, 288, 50257), (70, 32, 800000), (300, 40, 270000)])
+@pytest.mark.parametrize("tied", [False, True])
+def test_fp32_kept_logits_match_recomputed(shape, tied):
+    """The fp32 head with and without kept logits (OACE_FLAG_RECOMPUTE_Z: other row chunks, down to 32 rows
+    at 800000 entries): the same fp32 logits, so the same row records, and dh and dW but for the order
+    of their sums (1e-5 as test_linear_fp32_split_planes); bitwise equal where no logits were kept but the
+    chunks are the same."""
+    N, d, V = shape
+    h, w, t = _case(N, d, V, torch.float32, seed=N + V)
+    wv = _tied(w) if tied else w
+    loss, cache = _fwd(h, wv, t)
+    rloss, rcache = _fwd(h, wv, t, flags=A.oace.FLAG_RECOMPUTE_Z)
+    assert float(loss) == float(rloss) and torch.equal(cache[3], rcache[3])
+    dh, dw = _grads(cache, 1.3)
+    rh, rw = _grads(rcache, 1.3)
+    assert normwise(to_f64(rh), to_f64(dh)) <= 1e-5 and normwise(to_f64(rw), to_f64(dw)) <= 1e-5
+    if N * V * 10 <= 1 << 28:
+        assert torch.equal(rh, dh) and torch.equal(rw, dw)
