@@ -231,7 +231,9 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
 
 // dz of 16- and 32-bit logits: one wave per U * 64 chunks of a row, U 16-byte loads in flight per
 // lane.  The terms of every entry are formed without the target (the tau, c and sum factors folded
-// into three row scalars); the one chunk that holds it is formed again with it.  HBM
+// into three row scalars); the one chunk that holds it is formed again with it.  A factor tau c that an
+// infinite loss cotangent makes infinite is not folded, where it would meet itself as NaN, but multiplied
+// on at the end, in code of its own: one more multiplication per entry cost 4 us at the size below.  HBM
 // bound: (2048, 50257) bf16 157 -> 84 us for the call (4.9 TB/s read and written; the device copies
 // at the same rate), against 2-byte loads and stores before.
 template <int DT, int U>
@@ -258,43 +260,53 @@ __global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, i
   }
   const float* rec = rows + row * OACE_ROW;
   const float tau = rec[OACE_TAU], inv_S = rec[OACE_INV_S], pc = rec[OACE_PC_INV8];
-  const float tc = tau * (c0 * (g_loss ? *g_loss : 1.f));
+  const float tau_c = tau * (c0 * (g_loss ? *g_loss : 1.f));
+  const bool inf = __ballot(__builtin_isinf(tau_c)) != 0;  // the same in the whole wave: one row
+  const float tc = inf ? 1.f : tau_c;
   const float scale = rec[OACE_S8] * inv_S;
   const float cs = tc * scale, cd = tc * (inv_S * (rec[OACE_SUM_P78] - pc)), cr = tc * rec[OACE_RADIAL];
   const int64_t t = targets[row];
+  auto form = [&](auto times_tau_c) {
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int c = cb + 64 * u;
-    if (c < nch) {
-      const int e0 = c * R::EPC - lead;
-      float v[R::EPC], o[R::EPC];
-      R::unpack(raw[u], v);
-      // the entry of this chunk that is the target (outside [0, EPC): none)
-      const int64_t et = t >= 0 && t < V ? t - e0 : -1;
-      const bool hit = et >= 0 && et < R::EPC;
-#pragma unroll
-      for (int i = 0; i < R::EPC; ++i) {
-        const float x = v[i] * tau;
-        float rho, rho7, r;
-        octic7(x, rho, rho7, r);
-        const float b = rho7 * __builtin_fmaf(-cd, rho, cs);
-        o[i] = __builtin_fmaf(r, b, -cr * x);
-      }
-      if (hit) {
+    for (int u = 0; u < U; ++u) {
+      const int c = cb + 64 * u;
+      if (c < nch) {
+        const int e0 = c * R::EPC - lead;
+        float v[R::EPC], o[R::EPC];
+        R::unpack(raw[u], v);
+        // the entry of this chunk that is the target (outside [0, EPC): none)
+        const int64_t et = t >= 0 && t < V ? t - e0 : -1;
+        const bool hit = et >= 0 && et < R::EPC;
 #pragma unroll
         for (int i = 0; i < R::EPC; ++i) {
-          if (i == (int)et) {
-            const float x = v[i] * tau;
-            float rho, rho7, r;
-            octic7(x, rho, rho7, r);
-            const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - tc * pc;
-            o[i] = __builtin_fmaf(r, b, -cr * x);
+          const float x = v[i] * tau;
+          float rho, rho7, r;
+          octic7(x, rho, rho7, r);
+          const float b = rho7 * __builtin_fmaf(-cd, rho, cs);
+          o[i] = __builtin_fmaf(r, b, -cr * x);
+        }
+        if (hit) {
+#pragma unroll
+          for (int i = 0; i < R::EPC; ++i) {
+            if (i == (int)et) {
+              const float x = v[i] * tau;
+              float rho, rho7, r;
+              octic7(x, rho, rho7, r);
+              const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - tc * pc;
+              o[i] = __builtin_fmaf(r, b, -cr * x);
+            }
           }
         }
+        if constexpr (times_tau_c.value) {
+#pragma unroll
+          for (int i = 0; i < R::EPC; ++i) o[i] *= tau_c;
+        }
+        R::store(dr, e0, V, R::pack(o));
       }
-      R::store(dr, e0, V, R::pack(o));
     }
-  }
+  };
+  if (inf) form(std::true_type());
+  else form(std::false_type());
 }
 
 // dz = tau c (r bracket - radial x) for every element of rows (grid.y = row), c = c0 * g.

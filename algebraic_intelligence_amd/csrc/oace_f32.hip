@@ -184,7 +184,10 @@ __global__ __launch_bounds__(256) void oace_f32_dz_kernel(const float* z, int64_
     const f32x4_t za = *(const f32x4_t*)zr, zb = *(const f32x4_t*)(zr + 4);
     const float* rec = rows + row * OACE_ROW;
     const float tau = rec[OACE_TAU], inv_S = rec[OACE_INV_S], pc = rec[OACE_PC_INV8];
-    const float tc = tau * (c0 * (g_loss ? *g_loss : 1.f));
+    // an infinite factor is multiplied on at the end, as in oace_rows_bwd_vec_kernel
+    const float tau_c = tau * (c0 * (g_loss ? *g_loss : 1.f));
+    const bool inf = __ballot(__builtin_isinf(tau_c)) != 0;
+    const float tc = inf ? 1.f : tau_c;
     const float cs = tc * (rec[OACE_S8] * inv_S), cd = tc * (inv_S * (rec[OACE_SUM_P78] - pc));
     const float cr = tc * rec[OACE_RADIAL];
     const int64_t t = targets[row] - c;
@@ -195,6 +198,11 @@ __global__ __launch_bounds__(256) void oace_f32_dz_kernel(const float* z, int64_
       octic7(x, rho, rho7, r);
       const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - (t == u && c + u < V ? tc * pc : 0.f);
       o[u] = c + u < V ? __builtin_fmaf(r, b, -cr * x) : 0.f;
+    }
+    if (inf) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (c + u < V) o[u] *= tau_c;
     }
   }
   u32x4_t p[3];

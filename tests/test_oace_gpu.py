@@ -6,6 +6,7 @@ and fused_linear_oace (src/kernels/pallas_oace.py:59-293), forward and backward,
 Tolerances (normwise max error, the reference's metric): fp64 1e-10 against 40-digit values;
 fp32 and the bf16/fp16 loss (inputs exact, fp32 arithmetic) 2e-5; bf16/fp16 gradients 2e-2
 (dz and the outputs are rounded to the element type; the reference gates bf16 at 2e-2)."""
+import math
 import os
 
 import numpy as np
@@ -481,3 +482,19 @@ def test_fp32_kept_logits_match_recomputed(shape, tied):
     assert normwise(to_f64(rh), to_f64(dh)) <= 1e-5 and normwise(to_f64(rw), to_f64(dw)) <= 1e-5
     if N * V * 10 <= 1 << 28:
         assert torch.equal(rh, dh) and torch.equal(rw, dw)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,V", [(3, 1031), (4099, 9), (700, 6145)])
+def test_softmax_loss_infinite_cotangent(dtype, N, V):
+    """An infinite loss cotangent gives infinite dlogits, of the sign and with the NaN (an entry whose
+    bracket is 0) that a finite one predicts."""
+    rng = np.random.default_rng(V)
+    z = _t(rng.standard_normal((N, V)) * 10.0, dtype).requires_grad_(True)
+    t = torch.from_numpy(rng.integers(0, V, size=N)).to(DEV)
+    zd = z.detach().double().requires_grad_(True)
+    (ref,) = torch.autograd.grad(A.fused_oace_softmax_loss(zd, t), zd)
+    (dz,) = torch.autograd.grad(A.fused_oace_softmax_loss(z, t) * math.inf, z)
+    # entries not within rounding of 0 (2e-5 of a row's largest, as test_softmax_loss_vs_oracle)
+    clear = ref.abs() > 2e-5 * ref.abs().amax(-1, keepdim=True)
+    assert torch.equal(dz[clear].double(), ref[clear].sign() * math.inf) and not torch.isfinite(dz).any()
