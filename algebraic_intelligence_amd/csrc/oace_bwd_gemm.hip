@@ -71,6 +71,7 @@ struct BgArgs {
   int64_t ldb;
   int bn;
   int K, kpart, parts, mt, nt;
+  bool by_n;            // n tiles outermost in the workgroups' order
   unsigned short* out;  // OUT_ELEM: D[n][m] at out[n * ldo + m]
   int64_t ldo;
   int own;      // columns per tile that the tile stores (256; 248 for rows that are not dword aligned)
@@ -194,12 +195,10 @@ void oace_bwd_gemm_kernel(const BgArgs a) {
   // Workgroups that share an operand slice run consecutively on one XCD (block b runs on XCD
   // b mod 8), each XCD taking an equal contiguous run of work items.  With parts: items in
   // (part, n tile, m tile) order, so that the tiles of one contraction part share both
-  // operands' slices.  Without, at 8 m tiles or more: the n tiles of one m tile (its A slice), m tiles
-  // in order, so that neighbouring tiles -- which share the 128-byte lines at the ends of their
-  // output row segments when rows are not 128-byte aligned -- write them through the same L2.  With
-  // fewer m tiles than XCDs (dW of a (V, d) embedding: 3 at d = 768, which ran on 3 XCDs) the m
-  // tiles of one n tile (its B slice) run side by side, n tiles in order
-  // (512 x 768 x 50257: the backward 221 -> 155 us; 8192 rows: 3181 -> 2321 us).
+  // operands' slices.  Without: the n tiles of one m tile (its A slice), whole m tiles to an XCD, in
+  // order, so that neighbouring tiles -- which share the 128-byte lines at the ends of their output
+  // row segments when rows are not 128-byte aligned -- write them through the same L2; or, by_n
+  // (n_major), the m tiles of one n tile (its B slice) side by side, n tiles in order.
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   int part, mi, ni;
   if (a.parts > 1) {
@@ -209,7 +208,7 @@ void oace_bwd_gemm_kernel(const BgArgs a) {
     part = item / tiles;
     mi = (item % tiles) % a.mt;
     ni = (item % tiles) / a.mt;
-  } else if (a.mt < 8) {
+  } else if (a.by_n) {
     const int ipx = (a.mt * a.nt + 7) / 8, item = xcd * ipx + j;
     if (j >= ipx || item >= a.mt * a.nt) return;
     part = 0;
@@ -494,9 +493,17 @@ int64_t kpart_of(int64_t K, int parts) {
   return std::max<int64_t>(GK, (kp + GK - 1) / GK * GK);
 }
 
+// Order of the tiles without parts.  Whole m tiles to an XCD leave XCDs idle when mt is no multiple of 8:
+// single tiles in n order serve the (V, d) embedding's dW, whose m tiles (d / 256) are few and whose n
+// tiles are many.  Backward at 512 x d x 50257: d = 768 (3 m tiles) 221 -> 155 us, 2304 (9) 418 -> 336, 2560
+// 438 -> 372, 3072 454 -> 417, 3584 482 -> 464, 4352 (17) 606 -> 552, 4864 648 -> 614; equal at 8 and 16.
+// With more m than n tiles (the (d, V) head's dW) the shared lines and A slices count for more: in n order
+// 512 x 768 x 32001 takes 114 us instead of 105, 2048 x 2048 x 20801 467 instead of 430.
+bool n_major(int mt, int nt) { return mt < 8 || (mt < nt && mt % 8 != 0); }
+
 template <int DT, bool A_MC, bool B_MC, int OUT, int WN>
 hipError_t bg_launch(const BgArgs& g, hipStream_t st) {
-  const unsigned grid = (unsigned)(g.parts > 1 || g.mt < 8 ? 8 * ((g.parts * g.mt * g.nt + 7) / 8)
+  const unsigned grid = (unsigned)(g.parts > 1 || g.by_n ? 8 * ((g.parts * g.mt * g.nt + 7) / 8)
                                                            : 8 * g.nt * ((g.mt + 7) / 8));
   hipLaunchKernelGGL((oace_bwd_gemm_kernel<DT, A_MC, B_MC, OUT, WN>), dim3(grid), dim3(256 * WN), 0, st, g);
   return hipGetLastError();
@@ -582,6 +589,7 @@ hipError_t oace_gemm(int dtype, const OaceGemm& g, int parts, float* part, hipSt
   b.own = parts <= 1 && (((g.ldo & 1) != 0) || (((uintptr_t)g.out & 2u) != 0)) ? GM - 8 : GM;
   b.mt = tiles_m(g.m, b.own);
   b.nt = tiles_n(g.n, wn);
+  b.by_n = n_major(b.mt, b.nt);
   b.parts = parts > 1 ? parts : 1;
   b.kpart = b.parts > 1 ? (int)kpart_of(g.k, b.parts) : (int)g.k;
   if (b.parts > 1 && (int64_t)(b.parts - 1) * b.kpart >= g.k) return hipErrorInvalidValue;

@@ -498,3 +498,19 @@ def test_softmax_loss_infinite_cotangent(dtype, N, V):
     # entries not within rounding of 0 (2e-5 of a row's largest, as test_softmax_loss_vs_oracle)
     clear = ref.abs() > 2e-5 * ref.abs().amax(-1, keepdim=True)
     assert torch.equal(dz[clear].double(), ref[clear].sign() * math.inf) and not torch.isfinite(dz).any()
+
+
+@pytest.mark.parametrize("d", [1792, 2048, 2080, 2304])
+@pytest.mark.parametrize("V", [1100, 1531])
+def test_tied_dw_tile_orders(d, V):
+    """dW of a (V, d) embedding on both sides of the 8 m tiles (256 features each) at which their order over the
+    workgroups changes, with more n tiles (128 entries) than m tiles and ragged ones: every tile once.
+    Against the fp32 path on the same operands: the element type's rounding of dz and of dW, 2e-2."""
+    h, w, t = _case(160, d, V, torch.bfloat16, seed=d + V, scale=0.2)
+    _, cache = _fwd(h, _tied(w), t)
+    dh, dw = _grads(cache)
+    _, rcache = _fwd(h.float(), _tied(w).float(), t)
+    rh, rw = _grads(rcache)
+    assert normwise(to_f64(dh), to_f64(rh)) <= 2e-2 and normwise(to_f64(dw), to_f64(rw)) <= 2e-2
+    blocks = (dw.double() - rw.double()).abs()[: d // 32 * 32].reshape(d // 32, 32, V).amax(1)
+    assert (blocks <= 2e-2 * rw.double().abs().max()).all()
