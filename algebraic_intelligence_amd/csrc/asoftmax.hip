@@ -191,15 +191,14 @@ __global__ __launch_bounds__(256) void octic_bwd_kernel(int64_t n, const void* x
 }
 
 
-// rho(z)^8 and r = rsqrt(1 + z^2) with the hardware reciprocal square root and reciprocal
-// (1 ulp each), the reference's own operations (src/attention.py:18-26 uses lax.rsqrt; its
-// division r / (1 - u) becomes r * rcp(1 - u)).  Used by the register-resident kernels.
+// rho(z)^8 and r = rsqrt(1 + z^2) with the hardware reciprocal square root and reciprocal (1 ulp
+// each): rho(|z|) = |z| + (1 + z^2) r, which has no cancellation, and rho(-z) = 1 / rho(z).  Used by the
+// register-resident kernels.
 __device__ __forceinline__ float octic_hw(float z, float& r_out) {
   const float t = __builtin_fmaf(z, z, 1.0f);
   const float r = __builtin_amdgcn_rsqf(t);
-  const float neg = r * __builtin_amdgcn_rcpf(1.0f - z * r);
-  const float pos = __builtin_fmaf(t, r, z);
-  const float rho = z < 0.0f ? neg : pos;
+  const float pos = __builtin_fmaf(t, r, __builtin_fabsf(z));
+  const float rho = z < 0.0f ? __builtin_amdgcn_rcpf(pos) : pos;
   const float k2 = rho * rho;
   const float k4 = k2 * k2;
   r_out = r;
