@@ -229,13 +229,14 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
   }
 }
 
-// dz of 16- and 32-bit logits: one wave per U * 64 chunks of a row, U 16-byte loads in flight per
-// lane.  The terms of every entry are formed without the target (the tau, c and sum factors folded
+// dz of 16- and 32-bit logits: one wave per U * 64 whole chunks of a row, U 16-byte loads in flight per
+// lane, and a row's first wave takes the elements before and after them, one to a lane.  The terms of every entry are formed without the target (the tau, c and sum factors folded
 // into three row scalars); the one chunk that holds it is formed again with it.  A factor tau c that an
 // infinite loss cotangent makes infinite is not folded, where it would meet itself as NaN, but multiplied
 // on at the end, in code of its own: one more multiplication per entry cost 4 us at the size below.  HBM
 // bound: (2048, 50257) bf16 157 -> 84 us for the call (4.9 TB/s read and written; the device copies
-// at the same rate), against 2-byte loads and stores before.
+// at the same rate), against 2-byte loads and stores before.  8 million bf16 entries in rows of 10: 246 us,
+// of 33: 103, of 65: 57 (350, 112 and 61 with a workgroup per row and 2-byte accesses).
 template <int DT, int U>
 __global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, int64_t ldz, int64_t N, int V,
                                                                 const int64_t* targets, const float* rows,
@@ -243,21 +244,26 @@ __global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, i
                                                                 int64_t lddz) {
   using R = RowChunk<DT>;
   const int lane = threadIdx.x & 63;
-  const int spans = (R::count_max(V) + 64 * U - 1) / (64 * U);
-  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t row = w / spans;
+  const int spans = max(1, (V / R::EPC + 64 * U - 1) / (64 * U));
+  const unsigned w = blockIdx.x * 4 + (threadIdx.x >> 6);  // below 2^26
+  const int64_t row = w / (unsigned)spans;
   if (row >= N) return;
+  const int span = (int)(w % (unsigned)spans);
   const char* zr = (const char*)z + row * ldz * R::ESZ;
   char* dr = (char*)dz + row * lddz * R::ESZ;
-  const int lead = R::lead(zr), nch = R::count(V, lead);
-  const int cb = (int)(w % spans) * (64 * U) + lane;
+  const RowSpan sp = R::span(zr, V);
+  const int edge = span == 0 ? R::edge(sp, V, lane) : -1;  // a row's first wave takes its ends
+  const u32x4_t* zb = (const u32x4_t*)(zr + (int64_t)sp.head * R::ESZ);
+  u32x4_t* db = (u32x4_t*)(dr + (int64_t)sp.head * R::ESZ);
+  const int cb = span * (64 * U) + lane;
   u32x4_t raw[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int c = cb + 64 * u;
     raw[u] = u32x4_t{0u, 0u, 0u, 0u};
-    if (c < nch) raw[u] = R::load(zr, c * R::EPC - lead, V);
+    if (c < sp.body) raw[u] = zb[c];
   }
+  const float ze = edge >= 0 ? Elem<DT>::load(zr, edge) : 0.f;
   const float* rec = rows + row * OACE_ROW;
   const float tau = rec[OACE_TAU], inv_S = rec[OACE_INV_S], pc = rec[OACE_PC_INV8];
   const float tau_c = tau * (c0 * (g_loss ? *g_loss : 1.f));
@@ -267,43 +273,33 @@ __global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, i
   const float cs = tc * scale, cd = tc * (inv_S * (rec[OACE_SUM_P78] - pc)), cr = tc * rec[OACE_RADIAL];
   const int64_t t = targets[row];
   auto form = [&](auto times_tau_c) {
+    auto term = [&](float v, float target) {
+      const float x = v * tau;
+      float rho, rho7, r;
+      octic7(x, rho, rho7, r);
+      const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - target;
+      const float o = __builtin_fmaf(r, b, -cr * x);
+      return times_tau_c.value ? o * tau_c : o;
+    };
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = cb + 64 * u;
-      if (c < nch) {
-        const int e0 = c * R::EPC - lead;
+      if (c < sp.body) {
+        const int e0 = sp.head + c * R::EPC;
         float v[R::EPC], o[R::EPC];
         R::unpack(raw[u], v);
-        // the entry of this chunk that is the target (outside [0, EPC): none)
-        const int64_t et = t >= 0 && t < V ? t - e0 : -1;
-        const bool hit = et >= 0 && et < R::EPC;
 #pragma unroll
-        for (int i = 0; i < R::EPC; ++i) {
-          const float x = v[i] * tau;
-          float rho, rho7, r;
-          octic7(x, rho, rho7, r);
-          const float b = rho7 * __builtin_fmaf(-cd, rho, cs);
-          o[i] = __builtin_fmaf(r, b, -cr * x);
-        }
-        if (hit) {
+        for (int i = 0; i < R::EPC; ++i) o[i] = term(v[i], 0.f);
+        // the entry of this chunk that is the target (a target outside [0, V) is none)
+        if (t >= e0 && t < e0 + R::EPC) {
 #pragma unroll
-          for (int i = 0; i < R::EPC; ++i) {
-            if (i == (int)et) {
-              const float x = v[i] * tau;
-              float rho, rho7, r;
-              octic7(x, rho, rho7, r);
-              const float b = rho7 * __builtin_fmaf(-cd, rho, cs) - tc * pc;
-              o[i] = __builtin_fmaf(r, b, -cr * x);
-            }
-          }
+          for (int i = 0; i < R::EPC; ++i)
+            if (i == (int)(t - e0)) o[i] = term(v[i], tc * pc);
         }
-        if constexpr (times_tau_c.value) {
-#pragma unroll
-          for (int i = 0; i < R::EPC; ++i) o[i] *= tau_c;
-        }
-        R::store(dr, e0, V, R::pack(o));
+        db[c] = R::pack(o);
       }
     }
+    if (edge >= 0) Elem<DT>::store(dr, edge, term(ze, t == edge ? tc * pc : 0.f));
   };
   if (inf) form(std::true_type());
   else form(std::false_type());
@@ -498,7 +494,7 @@ template <int DT>
 bool rows_bwd_vec(const OaceArgs& a, const void* rows, void* dz, float c0, hipStream_t st) {
   using R = RowChunk<DT>;
   if ((((uintptr_t)a.h ^ (uintptr_t)dz) & 15u) != 0) return false;
-  const int nch = R::count_max((int)a.V);
+  const int nch = std::max(1, (int)a.V / R::EPC);  // whole chunks of the best start
   // four chunks per lane when that still leaves four waves per SIMD, else one
   const bool wide = a.N * ((nch + 255) / 256) >= 4096;
   const int64_t waves = a.N * (int64_t)((nch + (wide ? 255 : 63)) / (wide ? 256 : 64));
