@@ -211,7 +211,7 @@ __device__ __forceinline__ float octic_hw(float z, float& r_out) {
 // where it starts or ends inside a chunk, one element each of the first lanes: one HBM read of x (and
 // g), one write; rho^8 and r are evaluated once per element with the hardware rsqrt / reciprocal
 // (octic_hw) and the row is normalised with one division and products; the multi-pass kernels above
-// keep IEEE 1/sqrt and divisions throughout.
+// keep IEEE 1/sqrt and divisions throughout.  whole: every row is whole chunks, none has an edge.
 // Forward of (18372, 1531) fp32 109 -> 41 us (5.5 TB/s) and its VJP 267 -> 80 us (4.2 TB/s) against the
 // multi-pass kernels, which served every row whose length was no multiple of a chunk or over 64 x 8
 // (VJP: 64 x 4) chunks.
@@ -237,8 +237,9 @@ __device__ __forceinline__ void row_sum(float (&x)[K], float* sh) {
 }
 
 template <int DT, int T, int NCH>
-__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int64_t rows, int n, const void* x,
-                                                                            void* y, float sink, float eps) {
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int64_t rows, int n, bool whole,
+                                                                            const void* x, void* y, float sink,
+                                                                            float eps) {
 #pragma clang fp contract(off)
   using R = RowChunk<DT>;
   constexpr int RPB = T < 256 ? 256 / T : 1;  // rows per workgroup
@@ -248,8 +249,8 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
   const int tid = threadIdx.x % T;
   const char* xr = (const char*)x + row * n * R::ESZ;
   char* yr = (char*)y + row * n * R::ESZ;
-  const RowSpan sp = R::span(xr, n);
-  const int edge = R::edge(sp, n, tid);
+  const RowSpan sp = whole ? RowSpan{0, n / R::EPC, 0} : R::span(xr, n);
+  const int edge = whole ? -1 : R::edge(sp, n, tid);
   u32x4_t raw[NCH];
   float v[NCH][R::EPC];
 #pragma unroll
@@ -300,9 +301,9 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
 }
 
 template <int DT, int T, int NCH>
-__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int64_t rows, int n, const void* x,
-                                                                            const void* g, void* dx, float sink,
-                                                                            float eps) {
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int64_t rows, int n, bool whole,
+                                                                            const void* x, const void* g, void* dx,
+                                                                            float sink, float eps) {
 #pragma clang fp contract(off)
   // The row's x and g stay in registers as their raw 16-byte chunks and are unpacked where used;
   // one float per element, w = 8 r rho^8, carries the octic between passes.  sum(p g) is taken
@@ -318,8 +319,8 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int
   const char* xr = (const char*)x + row * n * R::ESZ;
   const char* gr = (const char*)g + row * n * R::ESZ;
   char* dr = (char*)dx + row * n * R::ESZ;
-  const RowSpan sp = R::span(xr, n);
-  const int edge = R::edge(sp, n, tid);
+  const RowSpan sp = whole ? RowSpan{0, n / R::EPC, 0} : R::span(xr, n);
+  const int edge = whole ? -1 : R::edge(sp, n, tid);
   const float inv_n = 1.f / (float)n;
   u32x4_t xw[NCH], gw[NCH];
   float w[NCH][R::EPC];
@@ -447,12 +448,13 @@ static void oc_bwd(int64_t n, const void* x, const void* g, void* dx, hipStream_
 static bool sm_reg_fits(int64_t rows, int nch) { return nch <= 4096 && (nch <= 256 || rows < (1 << 22)); }
 #define AFA_SM_GO(KERNEL, T, NCH, ...)                                                                       \
   hipLaunchKernelGGL((KERNEL<DT, T, NCH>), dim3((unsigned)((rows * T + (T < 256 ? 255 : T - 1)) /            \
-                     (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, rows, (int)n, __VA_ARGS__)
+                     (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, rows, (int)n, whole, __VA_ARGS__)
 template <int DT>
 static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
   if (n > (1 << 20) || !same_lead(x, y, nullptr)) return false;
   const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
+  const bool whole = n % RowChunk<DT>::EPC == 0 && ((uintptr_t)x & 15u) == 0;
 #define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_fwd_reg_kernel, T, NCH, x, y, (float)sink, (float)eps)
   if (nch <= 64) AFA_SM(64, 1);
   else if (nch <= 128) AFA_SM(64, 2);
@@ -473,6 +475,7 @@ static bool sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, vo
   if (n > (1 << 20) || !same_lead(x, g, dx)) return false;
   const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
+  const bool whole = n % RowChunk<DT>::EPC == 0 && ((uintptr_t)x & 15u) == 0;
 #define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_bwd_reg_kernel, T, NCH, x, g, dx, (float)sink, (float)eps)
   if (nch <= 64) AFA_SM(64, 1);
   else if (nch <= 128) AFA_SM(64, 2);
