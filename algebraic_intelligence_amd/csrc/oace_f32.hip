@@ -60,6 +60,8 @@ struct XArgs {
   float* out;                   // D[n][m] at out[part * part_stride + n * ldo + m]
   int64_t ldo, part_stride;
   int accumulate;  // D is added to what out holds
+  const float* g_loss;  // the backward's products: the loss cotangent (nullable) and its factor
+  float c0;
 };
 
 // Byte offset in a plane's stage of (tile row, logical 16-byte chunk): contraction-contiguous (KC)
@@ -249,17 +251,22 @@ void oace_f32_gemm_kernel(const XArgs a) {
   const char* bbase = (const char*)(a.b + (B_MC ? (int64_t)k_lo * a.ldb + n0 : (int64_t)n0 * a.ldb + k_lo));
   const int64_t astep = A_MC ? (int64_t)XK * a.lda * 2 : XK * 2;
   const int64_t bstep = B_MC ? (int64_t)XK * a.ldb * 2 : XK * 2;
+  // An infinite cotangent leaves no finite dz.  Its zero lower planes, and the signs of the other operand's,
+  // would make NaN of every infinite product: all planes are then taken from hi, whose six equal
+  // products are infinite, or NaN, as the fp32 product is.
+  const bool inf = a.g_loss != nullptr && __builtin_isinf(a.c0 * *a.g_loss);
+  const int64_t ap = inf ? 0 : a.ap, bp = inf ? 0 : a.bp;
   auto issue = [&](int t) {
     unsigned char* st = lds + (t & 1) * C::STAGE;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const char* ab = abase + t * astep + p * a.ap * 2;
+      const char* ab = abase + t * astep + p * ap * 2;
 #pragma unroll
       for (int i = 0; i < C::A_LOADS; ++i) lds_dma16(ab, aoff[i], st + p * C::A_PLANE + (512 * i + wave * 64) * 16);
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const char* bb = bbase + t * bstep + p * a.bp * 2;
+      const char* bb = bbase + t * bstep + p * bp * 2;
 #pragma unroll
       for (int i = 0; i < C::B_LOADS; ++i)
         lds_dma16(bb, boff[i], st + 3 * C::A_PLANE + p * C::B_PLANE + (512 * i + wave * 64) * 16);
@@ -537,6 +544,8 @@ hipError_t oace_linear_bwd_f32(const OaceArgs& a, const void* rows, void* ws, hi
     g.out = g.parts > 1 ? part : dh;
     g.ldo = g.parts > 1 ? p.dp : a.d;
     g.part_stride = rn * p.dp;
+    g.g_loss = (const float*)a.g_loss;
+    g.c0 = c0;
     e = a.w_layout == OACE_W_DV ? x_gemm<false, false>(g, p.dh_wide, st) : x_gemm<true, false>(g, p.dh_wide, st);
     if (e != hipSuccess) return e;
     if (g.parts > 1) {
@@ -558,6 +567,8 @@ hipError_t oace_linear_bwd_f32(const OaceArgs& a, const void* rows, void* ws, hi
     w.bn = (int)(dv ? a.d : a.V);
     w.K = w.kpart = (int)rp;
     w.parts = 1;
+    w.g_loss = g.g_loss;
+    w.c0 = c0;
     w.out = (float*)a.dw;
     w.ldo = a.ldw;
     w.accumulate = r0 > 0;

@@ -514,3 +514,26 @@ def test_tied_dw_tile_orders(d, V):
     assert normwise(to_f64(dh), to_f64(rh)) <= 2e-2 and normwise(to_f64(dw), to_f64(rw)) <= 2e-2
     blocks = (dw.double() - rw.double()).abs()[: d // 32 * 32].reshape(d // 32, 32, V).amax(1)
     assert (blocks <= 2e-2 * rw.double().abs().max()).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 40, 300), (1, 130, 1031), (1, 33, 50257)])
+@pytest.mark.parametrize("tied", [False, True])
+def test_linear_fp32_infinite_cotangent(shape, tied):
+    """dh and dW of the fp32 head where the loss cotangent is infinite: infinite, of the sign that a finite
+    one predicts, and NaN where infinite terms of both signs or a zero factor meet, as the generic fp32
+    kernels have them.  Feature 0 is 0 in h, so its weights are free to take the signs of dz."""
+    N, d, V = shape
+    h, w, t = _case(N, d, V, torch.float32, seed=V)
+    h[:, 0] = 0.0
+    wv = _tied(w) if tied else w
+    dz = (_grads(_fwd(h, wv, t)[1])[1][1] / h[0, 1]).double()
+    # an entry within rounding of 0 (2e-5 of the largest, as test_softmax_loss_vs_oracle) has no sign to predict
+    clear = dz.abs() > 2e-5 * dz.abs().max()
+    wv[0] = (dz.sign() * (0.5 + torch.rand(V, device=DEV, dtype=torch.float64))).float()
+    dh, dw = _grads(_fwd(h, wv, t)[1], math.inf)
+    gh, gw = _grads(_fwd(h, wv, t, flags=_lib.FLAG_GENERIC)[1], math.inf)
+    assert torch.isinf(dw[1:, clear]).all() and torch.isnan(dw[0]).all()
+    for got, want in ((dw[:, clear], gw[:, clear]), (dh[:, 1:], gh[:, 1:])):
+        assert torch.equal(got.nan_to_num(9e9), want.nan_to_num(9e9))
+    if clear.all():
+        assert float(dh[0, 0]) == float(gh[0, 0]) == math.inf
