@@ -211,10 +211,11 @@ __device__ __forceinline__ float octic_hw(float z, float& r_out) {
 // where it starts or ends inside a chunk, one element each of the first lanes: one HBM read of x (and
 // g), one write; rho^8 and r are evaluated once per element with the hardware rsqrt / reciprocal
 // (octic_hw) and the row is normalised with one division and products; the multi-pass kernels above
-// keep IEEE 1/sqrt and divisions throughout.  whole: every row is whole chunks, none has an edge.
-// Forward of (18372, 1531) fp32 109 -> 41 us (5.5 TB/s) and its VJP 267 -> 80 us (4.2 TB/s) against the
-// multi-pass kernels, which served every row whose length was no multiple of a chunk or over 64 x 8
-// (VJP: 64 x 4) chunks.
+// keep IEEE 1/sqrt and divisions throughout.  WHOLE, all_whole: every row is whole chunks, none has an edge;
+// known when compiled for rows of one chunk a lane (2^20 rows of 8 fp32 218 -> 205 us, VJP 296 -> 279).
+// Kernels alone, forward of (18372, 1531) fp32 99 -> 35 us (6.4 TB/s) and its VJP 254 -> 60 us (5.6 TB/s)
+// against the multi-pass kernels, which served every row whose length was no multiple of a chunk or
+// over 64 x 8 (VJP: 64 x 4) chunks.
 template <int T, int K>
 __device__ __forceinline__ void row_sum(float (&x)[K], float* sh) {
 #pragma unroll
@@ -236,8 +237,8 @@ __device__ __forceinline__ void row_sum(float (&x)[K], float* sh) {
   }
 }
 
-template <int DT, int T, int NCH>
-__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int64_t rows, int n, bool whole,
+template <int DT, int T, int NCH, bool WHOLE>
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int64_t rows, int n, bool all_whole,
                                                                             const void* x, void* y, float sink,
                                                                             float eps) {
 #pragma clang fp contract(off)
@@ -249,6 +250,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
   const int tid = threadIdx.x % T;
   const char* xr = (const char*)x + row * n * R::ESZ;
   char* yr = (char*)y + row * n * R::ESZ;
+  const bool whole = WHOLE || all_whole;
   const RowSpan sp = whole ? RowSpan{0, n / R::EPC, 0} : R::span(xr, n);
   const int edge = whole ? -1 : R::edge(sp, n, tid);
   u32x4_t raw[NCH];
@@ -300,8 +302,8 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_fwd_reg_kernel(int
   if (edge >= 0) Elem<DT>::store(yr, edge, ve * inv);
 }
 
-template <int DT, int T, int NCH>
-__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int64_t rows, int n, bool whole,
+template <int DT, int T, int NCH, bool WHOLE>
+__global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int64_t rows, int n, bool all_whole,
                                                                             const void* x, const void* g, void* dx,
                                                                             float sink, float eps) {
 #pragma clang fp contract(off)
@@ -319,6 +321,7 @@ __global__ __launch_bounds__(T < 256 ? 256 : T) void asoftmax_bwd_reg_kernel(int
   const char* xr = (const char*)x + row * n * R::ESZ;
   const char* gr = (const char*)g + row * n * R::ESZ;
   char* dr = (char*)dx + row * n * R::ESZ;
+  const bool whole = WHOLE || all_whole;
   const RowSpan sp = whole ? RowSpan{0, n / R::EPC, 0} : R::span(xr, n);
   const int edge = whole ? -1 : R::edge(sp, n, tid);
   const float inv_n = 1.f / (float)n;
@@ -446,8 +449,8 @@ static void oc_bwd(int64_t n, const void* x, const void* g, void* dx, hipStream_
 // chunks a lane leave one wave per SIMD, and (18372, 1531) fp32 took 173 us instead of 80).  false: no
 // variant holds the row, or a launch would pass 2^32 threads (the multi-pass kernels take 64 per row).
 static bool sm_reg_fits(int64_t rows, int nch) { return nch <= 4096 && (nch <= 256 || rows < (1 << 22)); }
-#define AFA_SM_GO(KERNEL, T, NCH, ...)                                                                       \
-  hipLaunchKernelGGL((KERNEL<DT, T, NCH>), dim3((unsigned)((rows * T + (T < 256 ? 255 : T - 1)) /            \
+#define AFA_SM_GO(KERNEL, T, NCH, WHOLE, ...)                                                                \
+  hipLaunchKernelGGL((KERNEL<DT, T, NCH, WHOLE>), dim3((unsigned)((rows * T + (T < 256 ? 255 : T - 1)) /     \
                      (T < 256 ? 256 : T))), dim3(T < 256 ? 256 : T), 0, st, rows, (int)n, whole, __VA_ARGS__)
 template <int DT>
 static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double sink, double eps, hipStream_t st) {
@@ -455,8 +458,16 @@ static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double s
   const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
   const bool whole = n % RowChunk<DT>::EPC == 0 && ((uintptr_t)x & 15u) == 0;
-#define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_fwd_reg_kernel, T, NCH, x, y, (float)sink, (float)eps)
-  if (nch <= 64) AFA_SM(64, 1);
+  // Ragged rows of 2-byte scores that one wave holds with one score to a lane: the multi-pass kernel forms their
+  // octics side by side, where a lane here forms a chunk's eight and then its edge element (2^18 rows of
+  // 17, 33, 63 bf16 73, 77, 78 against 85 us, fp16 73, 77, 78 against 91).  Below 15 not every row holds a
+  // whole chunk (9: 72 against 62), above 64 it takes two turns (2^17 rows of 65: 70 against 44).  fp32
+  // chunks hold four (33: 76 against 66), and the VJP's multi-pass kernel reads more (33: 140 against 122).
+  if (RowChunk<DT>::EPC == 8 && !whole && n >= 15 && n <= 64) return false;
+#define AFA_SM_W(T, NCH, WHOLE) AFA_SM_GO(asoftmax_fwd_reg_kernel, T, NCH, WHOLE, x, y, (float)sink, (float)eps)
+#define AFA_SM(T, NCH) AFA_SM_W(T, NCH, false)
+  if (nch <= 64 && whole) AFA_SM_W(64, 1, true);  // no edge code where the rows are short
+  else if (nch <= 64) AFA_SM(64, 1);
   else if (nch <= 128) AFA_SM(64, 2);
   else if (nch <= 192) AFA_SM(64, 3);
   else if (nch <= 256) AFA_SM(64, 4);
@@ -467,6 +478,7 @@ static bool sm_fwd_reg(int64_t rows, int64_t n, const void* x, void* y, double s
   else if (nch <= 2048) AFA_SM(512, 4);
   else AFA_SM(1024, 4);
 #undef AFA_SM
+#undef AFA_SM_W
   return true;
 }
 template <int DT>
@@ -476,8 +488,10 @@ static bool sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, vo
   const int nch = (int)n / RowChunk<DT>::EPC;  // whole chunks of the best start
   if (!sm_reg_fits(rows, nch)) return false;
   const bool whole = n % RowChunk<DT>::EPC == 0 && ((uintptr_t)x & 15u) == 0;
-#define AFA_SM(T, NCH) AFA_SM_GO(asoftmax_bwd_reg_kernel, T, NCH, x, g, dx, (float)sink, (float)eps)
-  if (nch <= 64) AFA_SM(64, 1);
+#define AFA_SM_W(T, NCH, WHOLE) AFA_SM_GO(asoftmax_bwd_reg_kernel, T, NCH, WHOLE, x, g, dx, (float)sink, (float)eps)
+#define AFA_SM(T, NCH) AFA_SM_W(T, NCH, false)
+  if (nch <= 64 && whole) AFA_SM_W(64, 1, true);
+  else if (nch <= 64) AFA_SM(64, 1);
   else if (nch <= 128) AFA_SM(64, 2);
   else if (nch <= 192) AFA_SM(64, 3);
   else if (nch <= 256) AFA_SM(64, 4);
@@ -488,6 +502,7 @@ static bool sm_bwd_reg(int64_t rows, int64_t n, const void* x, const void* g, vo
   else if (nch <= 2048) AFA_SM(512, 4);
   else AFA_SM(1024, 4);
 #undef AFA_SM
+#undef AFA_SM_W
   return true;
 }
 #undef AFA_SM_GO

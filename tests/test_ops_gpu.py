@@ -659,7 +659,7 @@ def test_algebraic_softmax_row_kernels(dt, epc, tol, chunks):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 9, 15, 17, 65, 129, 1031])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 8, 9, 14, 15, 17, 64, 65, 129, 256, 1031])
 @pytest.mark.parametrize("sink", [0.0, 0.5])
 def test_algebraic_softmax_small_row_sums(dt, n, sink):
     """Rows of negative scores, whose octic sum (n terms near 9e-4) is far below the 1 that an entry
