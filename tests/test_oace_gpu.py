@@ -115,7 +115,7 @@ def test_softmax_loss_row_kernels(dtype, epc, chunks):
     one an element past it (its dz, allocated aligned, then takes the element-wise kernel); and the
     mean over more rows than one workgroup sums.  Tolerances as test_softmax_loss_vs_oracle; fp16
     dz (2^-11 rounding, entries of 1e-4 and up at 2^10 times the loss) 2e-3."""
-    for V in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1}):
+    for V in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1, chunks * epc + epc}):
         N = 4099 if V <= 9 else 3
         rng = np.random.default_rng(V)
         for off in (0, 1):
@@ -129,7 +129,7 @@ def test_softmax_loss_row_kernels(dtype, epc, chunks):
             ref, cache = O.oace_softmax_loss(to_f64(z), t.cpu().numpy())
             # at V = 1 the loss is 0, the difference of terms of 2 * 64/7 = 18.3 whose S^(1/8) and
             # reciprocals are within about 8 roundings of 2^-24: 8.7e-6
-            assert abs(float(loss) - ref) <= 2e-5 * abs(ref) + 8.7e-6, (V, off)
+            assert abs(float(loss) - ref) <= 2e-5 * abs(ref) + (8.7e-6 if V == 1 else 0.0), (V, off)
             tol = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
             if V > 1:
                 assert normwise(to_f64(dz), O.oace_softmax_loss_vjp(cache, g)) <= tol, (V, off)
@@ -161,7 +161,7 @@ def test_linear_generic_vs_oracle(shape, dtype, tied):
 @pytest.mark.parametrize("pad", [0, 3])
 def test_linear_fp32_split_planes(shape, tied, pad):
     """fp32 through the three-plane bf16 products at the edges of tiles, steps and splits, with odd
-    row strides (pad), and in row chunks (270000 entries: 256 rows at a time), against the fp64
+    row strides (pad), and in row chunks (270000 entries: 224 rows at a time), against the fp64
     path.  Tolerance: sums of up to 270000 terms, 16 to a rounding of 2^-24, add up to about
     sqrt(270000 / 16) 2^-24 = 8e-6 of the largest result."""
     N, d, V = shape
@@ -176,7 +176,8 @@ def test_linear_fp32_split_planes(shape, tied, pad):
     dh, dw = _grads(cache, 1.3)
     ref, rcache = _fwd(h.double(), w.double(), t)
     rh, rw = _grads(rcache, 1.3)
-    assert abs(float(loss) - float(ref)) <= 2e-5 * abs(float(ref)) + 8.7e-6  # as test_softmax_loss_row_kernels
+    # at V = 1 the loss is 0: as test_softmax_loss_row_kernels
+    assert abs(float(loss) - float(ref)) <= 2e-5 * abs(float(ref)) + (8.7e-6 if V == 1 else 0.0)
     if V > 1:
         # in place of a new forward: weights changed since, or hidden rows changed since
         assert normwise(to_f64(dh), to_f64(rh)) <= 1e-5 and normwise(to_f64(dw), to_f64(rw)) <= 1e-5

@@ -639,7 +639,7 @@ def test_algebraic_softmax_row_kernels(dt, epc, tol, chunks):
     another offset from a 16-byte boundary, from an aligned base and from one an element past it (its
     output, allocated aligned, then takes the multi-pass kernel), against the fp64 kernel;
     tolerances as the tests of the same kernels above."""
-    for n in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1}):
+    for n in sorted({max(1, chunks * epc - epc), max(1, chunks * epc - 1), chunks * epc + 1, chunks * epc + epc}):
         gen = torch.Generator(device=DEV).manual_seed(n)
         for off in (0, 1):
             rows = 5
