@@ -1,7 +1,7 @@
 // fp32 products on the bf16 matrix cores: exact three-plane splits and the LDS tiles of planes.
 //
 // x = hi + mid + lo with three bf16 values holds an fp32 value exactly (3 x 8 significant bits), and
-//   x y = hi hi' + (hi mid' + mid hi') + (mid mid' + hi lo' + lo hi') + terms below 2^-23 |x y|,
+//   x y = hi hi' + (hi mid' + mid hi') + (mid mid' + hi lo' + lo hi') + terms together below 2^-23 |x y|,
 // six products of the bf16 matrix cores, accumulated in fp32.  They run at 16 times the fp32 rate:
 // 2.7 times after six passes, and one fp32 rounding serves 16 of the contraction where the fp32
 // MFMA's serves two.  Below about 2^-110 the lower planes reach bf16's subnormals (steps of 2^-133) and
@@ -12,7 +12,7 @@
 
 namespace afa {
 
-// Planes of a pair, packed.  Rounded to nearest: the dropped terms are at most 2^-24 |x y|.  An
+// Planes of a pair, packed.  Rounded to nearest: |mid| < 2^-8 |x| and |lo| < 2^-16 |x|.  An
 // infinity, or a value that rounds past the largest bf16, gives a NaN in the lower planes (rows redone in
 // fp32, below).
 __device__ __forceinline__ void split3_rne(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {

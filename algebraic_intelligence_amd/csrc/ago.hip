@@ -121,9 +121,8 @@ __global__ __launch_bounds__(256) void ago_rotate_kernel(int64_t npairs_total, i
 // The same in 16-byte chunks: a thread owns one chunk of a (seq, inner, dim) slice, holds its table
 // entries and turns that chunk of ROT_OUTER consecutive slices, their loads in flight together, so
 // the table and the index arithmetic (two divisions) are paid once per ROT_OUTER chunks.  HBM
-// bound: q and k of (2, 16, 8192, 128) bf16 in one launch 44 us (6.1 TB/s), of (8, 12, 2048, 64)
-// two launches of 19 us element by element -> one, the training pass 178 -> 69 us (now the host's
-// time per call).
+// bound: q and k of (2, 16, 8192, 128) bf16 in one launch 44 us (6.1 TB/s), of (8, 12, 2048, 64) two
+// launches of 19 us element by element -> one of 16, the training pass 170 -> 112 us (now the host's time).
 constexpr int ROT_OUTER = 4;
 template <int DT, int TD>
 __global__ __launch_bounds__(256) void ago_rotate_vec_kernel(uint32_t slice, int64_t outer, uint32_t seq_chunks,

@@ -123,8 +123,8 @@ __global__ __launch_bounds__(256) void oace_mean_kernel(A* rows, int64_t N, int6
 // its 16-byte chunks (NCH per thread; NCH = 0 streams a longer row twice) and, where it starts or ends
 // inside one, one element each of the first lanes.  Bound by the octic terms' VALU issue (about
 // 20 instructions and two quarter-rate ones per 16-bit entry) just above its one HBM read:
-// (2048, 50257) bf16, forward call with the mean 176 -> 76 us (2.7 TB/s; the two passes of 2-byte
-// loads by one 256-thread workgroup per row took 171 of the 176), fp32 97 us (4.3 TB/s).
+// (2048, 50257) bf16, forward call with the mean 176 -> 64 us (3.2 TB/s; the two passes of 2-byte
+// loads by one 256-thread workgroup per row took 171 of the 176), (1024, 48001) fp32 41 us (4.8 TB/s).
 template <int DT, int T, int NCH>
 __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel(const void* z, int64_t ldz, int64_t N,
                                                                              int V, const int64_t* targets, float eps,
@@ -230,13 +230,14 @@ __global__ __launch_bounds__(T < 256 ? 256 : T, 4) void oace_rows_fwd_vec_kernel
 }
 
 // dz of 16- and 32-bit logits: one wave per U * 64 whole chunks of a row, U 16-byte loads in flight per
-// lane, and a row's first wave takes the elements before and after them, one to a lane.  The terms of every entry are formed without the target (the tau, c and sum factors folded
-// into three row scalars); the one chunk that holds it is formed again with it.  A factor tau c that an
-// infinite loss cotangent makes infinite is not folded, where it would meet itself as NaN, but multiplied
-// on at the end, in code of its own: one more multiplication per entry cost 4 us at the size below.  HBM
-// bound: (2048, 50257) bf16 157 -> 84 us for the call (4.9 TB/s read and written; the device copies
-// at the same rate), against 2-byte loads and stores before.  8 million bf16 entries in rows of 10: 246 us,
-// of 33: 103, of 65: 57 (350, 112 and 61 with a workgroup per row and 2-byte accesses).
+// lane, and a row's first wave takes the elements before and after them, one to a lane.  The terms of
+// every entry are formed without the target (the tau, c and sum factors folded into three row scalars);
+// the one chunk that holds it is formed again with it.  A factor tau c that an infinite loss cotangent
+// makes infinite is not folded, where it would meet itself as NaN, but multiplied on at the end, in code
+// of its own: one more multiplication per entry cost 4 us at the size below.  HBM bound: (2048, 50257)
+// bf16 157 -> 76 us (5.4 TB/s read and written), against 2-byte loads and stores before.  8 million bf16
+// entries in rows of 10: 246 us, of 33: 103, of 65: 57 (350, 112 and 61 with a workgroup per row and
+// 2-byte accesses).
 template <int DT, int U>
 __global__ __launch_bounds__(256) void oace_rows_bwd_vec_kernel(const void* z, int64_t ldz, int64_t N, int V,
                                                                 const int64_t* targets, const float* rows,
@@ -463,9 +464,11 @@ void w_strides(const OaceArgs& a, int64_t& sk, int64_t& sv) {
 }
 
 // Threads per row and 16-byte chunks per thread by the row's length: the fewest threads that hold
-// the row in at most 4 chunks each, then 512 threads with up to 26 (104 registers of a 128-register
-// wave, so two workgroups still share a compute unit and one loads while the other evaluates);
-// longer rows are streamed.
+// the row in at most 4 chunks each, then 512 threads with up to 25 (100 registers of a 128-register
+// wave, so two workgroups still share a compute unit and one loads while the other evaluates), or half as
+// many where 256 or 512 threads hold the row so: a chunk a thread does not have costs its turns all the
+// same (calls of 4096 rows of 2100 chunks bf16 69 us in 25s, 50 in 13s; 2048 of 6282 66 and 64, fp32 43 and
+// 38).  Longer rows are streamed.
 template <int DT>
 void rows_fwd_vec(const OaceArgs& a, const void* z, int64_t ldz, void* rows, hipStream_t st) {
   const int nch = (int)a.V / RowChunk<DT>::EPC;  // whole chunks of the best start

@@ -6,11 +6,11 @@
 //   lo_x hi_y + hi_x lo_y + mid_x mid_y + mid_x hi_y + hi_x mid_y + hi_x hi_y,
 // accumulated in fp32 by v_mfma_f32_32x32x16_bf16: the scheme of a six-pass bf16 product at full
 // fp32 precision, which the reference asks of its fp32 dots (Precision.HIGHEST).  The dropped terms
-// are below 2^-24 of the product, one rounding serves 16 of them where an fp32 fma chain rounds
+// are together below 2^-23 of the product, one rounding serves 16 of them where an fp32 fma chain rounds
 // each, and the bf16 pipes have 16 times the rate of the fp32 ones: 2.7 times after six passes.
 // Error against 64 bits (2-norm; SIMT fp32 GEMM it replaces in brackets), 512 x 288 x 50257: dh
 // 4.1e-7 (4.0e-6), dW 2.6e-7 (4.1e-7); lower at every size tried from 4 x 32 x 100 to
-// 1024 x 1024 x 50257.  Forward + backward there: 12.0 -> 0.50 ms; 1024 x 1024 x 50257 20.4 ->
+// 1024 x 1024 x 50257.  Forward + backward of the 512 rows, tied: 12.1 -> 0.434 ms; 1024 x 1024 x 50257 20.4 ->
 // 1.84 ms (the two backward GEMMs at 1.3 PFLOP/s of bf16 products, the rate a library bf16 GEMM
 // reaches on the device); 4 x 32 x 100 54 -> 51 us, so small problems take this path too.
 //
