@@ -84,13 +84,9 @@ struct Elem<AFA_F32> {
 };
 
 // ------------------------------------------------------------------ rows in 16-byte chunks
-// A row of n elements at any element-aligned address, seen as the 16-byte aligned chunks that
-// cover it: chunk c holds elements c * EPC - lead .. + EPC - 1, lead the elements between the
-// aligned address at or below the row's start and the start.  Whole chunks move as one 16-byte
-// access; the first and the last chunk of a row that starts or ends inside one move element by
-// element, so nothing outside the row is read or written (entries outside it load as zeros).
-// Kernels that sum over a row take its whole chunks (RowSpan) and, one to a lane, the elements before
-// and after them: a chunk's zeros would add rho(0) = 1 each to sums that can be far smaller.
+// A row of n elements at any element-aligned address: its whole 16-byte aligned chunks, each moved as
+// one access, and the elements before the first and after the last of them, fewer than a chunk each, which
+// the first lanes take one by one.  Nothing outside the row is read, written or summed.
 struct RowSpan {
   int head, body, tail;  // elements before the first whole chunk, whole chunks, elements after the last
 };
@@ -98,10 +94,6 @@ template <int DT>
 struct RowChunk {
   static constexpr int ESZ = DT == AFA_F32 ? 4 : 2;
   static constexpr int EPC = 16 / ESZ;
-  static __device__ __forceinline__ int lead(const void* row) { return (int)((uintptr_t)row & 15u) / ESZ; }
-  static __host__ __device__ __forceinline__ int count(int n, int lead) {
-    return (int)(((int64_t)n + lead + EPC - 1) / EPC);
-  }
   static __host__ __device__ __forceinline__ RowSpan span(const void* row, int n) {
     const int to = (int)((16u - ((uintptr_t)row & 15u)) & 15u) / ESZ, head = to < n ? to : n;
     const int body = (n - head) / EPC;
@@ -110,24 +102,6 @@ struct RowChunk {
   // the element outside the whole chunks that lane i of a row takes (2 * EPC lanes), or -1
   static __device__ __forceinline__ int edge(RowSpan s, int n, int i) {
     return i < s.head ? i : i >= EPC && i < EPC + s.tail ? n - s.tail + i - EPC : -1;
-  }
-  // chunks of the worst start
-  static __host__ __device__ __forceinline__ int count_max(int n) { return count(n, EPC - 1); }
-  static __device__ __forceinline__ u32x4_t load(const void* row, int e0, int n) {
-    if (e0 >= 0 && n - e0 >= EPC) return *(const u32x4_t*)((const char*)row + (int64_t)e0 * ESZ);
-    u32x4_t w = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < EPC; ++i) {
-      if (e0 + i >= 0 && (int64_t)e0 + i < n) {
-        if constexpr (DT == AFA_F32) {
-          w[i] = ((const unsigned*)row)[e0 + i];
-        } else {
-          const unsigned u = ((const unsigned short*)row)[e0 + i];
-          w[i >> 1] |= u << (16 * (i & 1));
-        }
-      }
-    }
-    return w;
   }
   static __device__ __forceinline__ void unpack(u32x4_t w, float (&v)[EPC]) {
 #pragma unroll
@@ -153,19 +127,6 @@ struct RowChunk {
       }
     }
     return w;
-  }
-  static __device__ __forceinline__ void store(void* row, int e0, int n, u32x4_t w) {
-    if (e0 >= 0 && n - e0 >= EPC) {
-      *(u32x4_t*)((char*)row + (int64_t)e0 * ESZ) = w;
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < EPC; ++i) {
-      if (e0 + i >= 0 && (int64_t)e0 + i < n) {
-        if constexpr (DT == AFA_F32) ((unsigned*)row)[e0 + i] = w[i];
-        else ((unsigned short*)row)[e0 + i] = (unsigned short)(w[i >> 1] >> (16 * (i & 1)));
-      }
-    }
   }
 };
 
