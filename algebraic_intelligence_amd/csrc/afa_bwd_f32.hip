@@ -301,7 +301,8 @@ void afa_bwd_f32_dq_kernel(const GenArgs a) {
         const float s = f32_half_dot(qo, kr) * scale, p = f32_half_dot(go, vr);
         float rr;
         const float w = frho8r(s, rr) * invd;
-        if (qi < L && (!a.causal || j <= qi)) f32_half_axpy(c8 * rr * w * (p - ei), kr, dq);
+        // a masked key's ds is 0, and its infinite entries are NaN, as in the tiles
+        f32_half_axpy(!a.causal || j <= qi ? c8 * rr * w * (p - ei) : 0.f, kr, dq);
       }
     }
   }
@@ -487,10 +488,9 @@ void afa_bwd_f32_dkdv_kernel(const GenArgs a) {
         const float s = f32_half_dot(ko, qr) * scale, p = f32_half_dot(vo, gr);
         float rr;
         const float w = frho8r(s, rr) * ip[i];
-        if (kj < vlen && (!a.causal || kj <= i)) {
-          f32_half_axpy(c8 * rr * w * (p - ep[i]), qr, dk);
-          f32_half_axpy(w, gr, dv);
-        }
+        const bool keep = kj < vlen && (!a.causal || kj <= i);
+        f32_half_axpy(keep ? c8 * rr * w * (p - ep[i]) : 0.f, qr, dk);
+        f32_half_axpy(keep ? w : 0.f, gr, dv);
       }
     }
   }

@@ -260,11 +260,10 @@ void afa_fwd_f32_kernel(const FwdArgs a) {
         f32_half_row<D, ROT>(kp + (int64_t)j * a.k_l, a.rc, a.rs, j, kr);
         f32_half_row<D, false>(vp + (int64_t)j * a.v_l, nullptr, nullptr, 0, vr);
         const float s = f32_half_dot(qo, kr);
-        const float w = rho8_exact(D == 64 ? s : s * a.s_mult);
-        if (qi < L && (!a.causal || j <= qi)) {
-          f32_half_axpy(w, vr, o);
-          if (g == 0) dsum += w;
-        }
+        // a masked key weighs 0, and its infinite values are NaN, as in the tiles
+        const float w = !a.causal || j <= qi ? rho8_exact(D == 64 ? s : s * a.s_mult) : 0.f;
+        f32_half_axpy(w, vr, o);
+        if (g == 0) dsum += w;
       }
     }
   }

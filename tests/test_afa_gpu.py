@@ -447,12 +447,13 @@ def _bwd_f32(q, k, v, out, den, g, causal, rotary, flags):
 @pytest.mark.parametrize("D", [32, 48, 64, 96, 128])
 @pytest.mark.parametrize("L", [31, 33, 160, 300])
 @pytest.mark.parametrize("case", ["g", "g_past_bf16", "v", "k_past_bf16", "E", "nan"])
-def test_f32_backward_infinities(D, L, case):
+@pytest.mark.parametrize("causal", [False, True])
+def test_f32_backward_infinities(D, L, case, causal):
     """The fp32 backward where an operand has no bf16 planes (an infinity, a value that rounds past the
     largest bf16, a row's E that overflows): infinite, NaN and finite results where the generic
     fp32 kernels have them, within the rounding of both (2e-5 of a feature's largest entry, and 2^-126: an
     operand near 1e-38 has subnormal planes, steps of 2^-133, and at most 300 terms); and NaN inputs NaN
-    as there."""
+    as there.  A causal mask's zero weights make NaN of the infinities they meet, as there."""
     q, k, v = make_qkv((1, 2, L, D), torch.float32, seed=L + D)
     g = make_qkv((1, 2, L, D), torch.float32, seed=L)[0]
     rot = A.build_cayley_rotary_matrix(D, L) if D == 64 and case != "k_past_bf16" else None
@@ -461,7 +462,7 @@ def test_f32_backward_infinities(D, L, case):
         v[0, 1, j, 5] = float("-inf")
     if case == "k_past_bf16":
         q[0, 1, :, 3], k[0, 1, j, 3] = 1e-38, 3.4e38
-    out, den = _fwd(q, k, v, rotary=rot, flags=_lib.FLAG_GENERIC)
+    out, den = _fwd(q, k, v, causal=causal, rotary=rot, flags=_lib.FLAG_GENERIC)
     if case == "g":
         g[0, 1, j, 2] = float("inf")
     if case == "g_past_bf16":
@@ -470,23 +471,27 @@ def test_f32_backward_infinities(D, L, case):
         g[0, 0, j, 4], out[0, 0, j, 4] = 1e38, 1e10
     if case == "nan":
         g[0, 1, j, 2] = float("nan")
-    got = _bwd_f32(q, k, v, out, den, g, False, rot, 0)
-    want = _bwd_f32(q, k, v, out, den, g, False, rot, _lib.FLAG_GENERIC)
+    got = _bwd_f32(q, k, v, out, den, g, causal, rot, 0)
+    want = _bwd_f32(q, k, v, out, den, g, causal, rot, _lib.FLAG_GENERIC)
     for name, x, y in zip(("dq", "dk", "dv"), got, want):
         bad = ~torch.isfinite(y)
         assert torch.equal(bad, ~torch.isfinite(x)), name
         assert torch.equal(x[bad].nan_to_num(9e9), y[bad].nan_to_num(9e9)), name
         xf, yf = x.masked_fill(bad, 0.0).double(), y.masked_fill(bad, 0.0).double()
-        scale = yf.abs().amax(2, keepdim=True)
+        # ds = 8 r w (p - E) carries the rounding of p and of E, whatever is left of their difference: with the
+        # one key of 3.4e38, whose entries alone make feature 3 of dq, those that overflow are its largest
+        top = y.double().nan_to_num(0.0, 3.4e38, -3.4e38) if case == "k_past_bf16" and name == "dq" else yf
+        scale = top.abs().amax(2, keepdim=True)
         assert ((xf - yf).abs() <= 2e-5 * scale + 2.0 ** -126).all(), name
     if case == "g":  # the feature's dv is infinite and nothing else of it is lost
-        assert torch.isinf(got[2][0, 1, :, 2]).all() and torch.isfinite(got[2][0, 0]).all()
+        assert torch.isinf(got[2][0, 1, :j + 1 if causal else L, 2]).all() and torch.isfinite(got[2][0, 0]).all()
 
 
 @pytest.mark.parametrize("D", [32, 48, 64, 96, 128])
 @pytest.mark.parametrize("B,L", [(1, 31), (1, 160), (1, 700), (40, 300)])
 @pytest.mark.parametrize("case", ["k", "v", "v_inf", "nan"])
-def test_f32_forward_values_without_planes(D, B, L, case):
+@pytest.mark.parametrize("causal", [False, True])
+def test_f32_forward_values_without_planes(D, B, L, case, causal):
     """The fp32 forward, whole and with split key ranges, where an operand rounds past the largest bf16 or is
     infinite: finite and infinite results where the generic fp32 kernel has them, within the rounding of
     both (2e-5 of a row's largest entry); and NaN inputs NaN as there."""
@@ -501,8 +506,8 @@ def test_f32_forward_values_without_planes(D, B, L, case):
         v[0, 1, j, 2] = float("inf")
     if case == "nan":
         k[0, 1, j, 2] = float("nan")
-    out, den = _fwd(q, k, v, rotary=rot)
-    want, wden = _fwd(q, k, v, rotary=rot, flags=_lib.FLAG_GENERIC)
+    out, den = _fwd(q, k, v, causal=causal, rotary=rot)
+    want, wden = _fwd(q, k, v, causal=causal, rotary=rot, flags=_lib.FLAG_GENERIC)
     bad = ~torch.isfinite(want)
     assert bad.any() == (case in ("v_inf", "nan"))
     assert torch.equal(bad, ~torch.isfinite(out)) and torch.equal(torch.isnan(den), torch.isnan(wden))
